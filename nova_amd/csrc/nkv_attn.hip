@@ -36,6 +36,7 @@
 #include "nkv_common.h"
 
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace nkv {
@@ -86,6 +87,8 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef int v2i_t __attribute__((vector_size(8)));
 typedef __attribute__((address_space(3))) v2i_t lds_v2i_t;
+typedef short v4s_t __attribute__((vector_size(8)));
+typedef __attribute__((address_space(3))) v4s_t lds_v4s_t;
 
 enum TailMode : int { TAIL_NONE = 0, TAIL_MASK = 1, TAIL_SCALARS = 2, TAIL_FUSED = 3 };
 // TAIL_FUSED with `tok`: the new token itself is the tail (its codes written by the prefix kernel).
@@ -3273,16 +3276,23 @@ __global__ void ring_mask_kernel(const int64_t* written, const int64_t* qlen, co
 // qoff + i (qoff = Mk - M) and attends fp16 tokens j <= qoff + i. With qoff = 0 the fp16
 // tokens are the chunk's own; with qoff > 0 they are an fp16 history plus the chunk (the
 // staged prefill, whose history is not quantized yet). Query rows of KV head
-// h: row r = (token r / gq, q head h gq + r % gq), M gq rows per head. Workgroup (h, tile,
-// split) takes rows 256 tile .. + 255 (8 waves x 2 MFMA row blocks of 16) and the split's
-// share of the 64-token groups: cache groups [split G / S, (split + 1) G / S) and chunk
-// groups j = split (mod S) up to its last query token. Per group, the 8 waves dequantize
-// the int8 codes once into fp16 LDS tiles (K row-major, V transposed, both padded against
-// bank conflicts), then every wave runs QK^T and PV on v_mfma_f32_16x16x32_f16 for its 32
-// rows. The cache groups take one workgroup barrier each: the tiles are double-buffered and
-// the next group is dequantized beside the current group's last product. P is a single fp16
-// operand (scaled by 2^15), as a fused fp16 attention kernel computes it. Each workgroup
-// writes one partial per row; a combine kernel merges the splits.
+// h: row r = (token r / gq, q head h gq + r % gq), M gq rows per head, in tiles of 256 rows
+// (8 waves x 2 MFMA row blocks of 16). A tile's steps are the 64-token groups it attends: the
+// G = U / 64 cache groups, then the fp16 groups up to its last query token, so later tiles have
+// more steps. The steps of a head's tiles, in order, are cut into W shares (PrefillArgs::cut) and
+// workgroup (h, w) takes share w: the end of one tile, whole tiles, the start of another. A tile
+// whose steps one workgroup took is normalized and written by it; the parts of a cut tile are
+// partials (one per row) that a combine kernel merges.
+// Per group, the 8 waves turn the staged codes (or fp16 rows) once into fp16 LDS tiles: K
+// row-major, V transposed, both padded against bank conflicts; then every wave runs QK^T and PV
+// on v_mfma_f32_16x16x32_f16 for its 32 rows. A group takes one workgroup barrier: the tiles are
+// double-buffered and the next group is converted beside the current group's last product. P is a
+// single fp16 operand (scaled by 2^15), as a fused fp16 attention kernel computes it.
+// Bound by issue: 68 MFMA and about 200 VALU instructions per wave and step, two waves per SIMD, a
+// step in 2.0 us. Against one workgroup per tile and split, with the fp16 groups loaded and scattered
+// between two barriers (3.9 us each) and a combine launch after every call (8 KV heads, 32 q heads):
+// 2048 tokens over 0 / 8192: 131 -> 60 us, 391 -> 326 us; 4096 over 0: 354 -> 149 us; 12001 over 0:
+// 2270 -> 1250 us; 8 over 16384: 46 -> 25 us; 512 over 16384 (no imbalance): 158 -> 156 us.
 constexpr int PF_WAVES = 8;
 constexpr int PF_THREADS = 64 * PF_WAVES;
 constexpr int PF_RB = 2;                             // MFMA row blocks per wave
@@ -3292,21 +3302,26 @@ constexpr int PF_KROW = D + 8;                       // fp16 K tile row stride (
 constexpr int PF_VROW = GT + 16;                     // fp16 V^T tile row stride (halves, 16-byte rows)
 constexpr float PF_TAU = 8.0f;                       // lazy softmax rescaling threshold (log2)
 constexpr int PF_PART = D + 4;                       // floats per row partial: acc[128], m, l, pad
+constexpr int PF_MAX_SHARES = 256;                   // shares of a head's steps (one workgroup per CU)
+constexpr int PF_STAGE = 2 * GT * D * 2;             // bytes of a stage: an fp16 group, or an int8 one with its rulers
+static_assert(PF_STAGE >= 2 * CODE_BYTES + RULER_BYTES, "an int8 group fits a stage");
+static_assert(2 * PF_STAGE >= PF_ROWS * D * 2, "a tile's fp16 output fits the stages");
 #ifndef PF_SCHED
 #define PF_SCHED 1
 #endif
 #ifndef PF_SCHED_V
-#define PF_SCHED_V 3  // VALU instructions scheduled after each interleaved MFMA
+#define PF_SCHED_V 2  // VALU instructions scheduled after each interleaved MFMA (1: +0.5%, 3: +2%, 4: +1% time)
 #endif
 // instruction classes of __builtin_amdgcn_sched_group_barrier
 constexpr int PF_SG_VALU = 0x2, PF_SG_MFMA = 0x8, PF_SG_DSR = 0x100;
 
-// token slot of the V^T tile: P's k-slot order (slot 8g + r of a 32-token block <-> token
-// 16 (r >> 2) + 4g + (r & 3))
-__device__ __forceinline__ int pf_vslot(int t) {
-  const int u = t & 31;
-  return (t & 32) + 8 * ((u >> 2) & 3) + 4 * (u >> 4) + (u & 3);
-}
+// The V^T tile keeps tokens in P's k-slot order: slot 8g + r of a 32-token block is token
+// 16 (r >> 2) + 4g + (r & 3).
+
+// Where a share of a head's steps starts: step `step` of the tile at position `tile` of its order.
+struct PrefillCut {
+  int tile, step;
+};
 
 struct PrefillArgs {
   const uint16_t* q;   // [hq][M][D]
@@ -3319,12 +3334,49 @@ struct PrefillArgs {
   const uint16_t* vmn;
   const uint16_t* vst;
   int64_t capacity, ngroups_cap, U;
-  int M, hq, hkv, gq, splits, tiles;
+  int M, hq, hkv, gq, tiles, shares;
   int Mk, qoff;    // fp16 tokens, and the fp16 index of query token 0
   int64_t kc_hs;   // head stride of kc / vc (elements)
   float sl2;
-  float* ws;       // [splits][hkv * M * gq][PF_PART]
+  float* ws;       // partials [hkv][slots][slot_rows][PF_PART]
+  int slots, slot_rows;
+  int zigzag;      // tiles are taken in the order 0, tiles - 1, 1, tiles - 2, ..., else 0, 1, 2, ...
+  int two_slots;   // share w's partials: slot 2 w (the end of a tile) and 2 w + 1 (the start of one); else slot w
   uint16_t* out;   // [hq][M][D]
+  PrefillCut cut[PF_MAX_SHARES + 1];
+};
+
+// The partial slot of share w's part of a tile, `start`: the part begins at the tile's step 0. (A
+// share has at most one cut tile that it ends and one that it starts.)
+__host__ __device__ __forceinline__ int pf_slot(const PrefillArgs& a, int w, bool start) {
+  return a.two_slots ? 2 * w + (start ? 1 : 0) : w;
+}
+
+// fp16 groups that rows up to `last_row` attend.
+__host__ __device__ __forceinline__ int pf_fp16_to(const PrefillArgs& a, int64_t last_row) {
+  const int64_t rows_h = (int64_t)a.M * a.gq;
+  const int n = ((int)(last_row < rows_h ? last_row : rows_h - 1) / a.gq + a.qoff) / GT + 1, cap = (a.Mk + GT - 1) / GT;
+  return n < cap ? n : cap;
+}
+// fp16 groups of tile `tile`: up to its last query token's.
+__host__ __device__ __forceinline__ int pf_fp16_groups(const PrefillArgs& a, int tile) {
+  return pf_fp16_to(a, ((int64_t)tile + 1) * PF_ROWS - 1);
+}
+// The tile at position `p` of a head's order.
+__host__ __device__ __forceinline__ int pf_tile_at(const PrefillArgs& a, int p) {
+  return !a.zigzag ? p : (p & 1) ? a.tiles - 1 - p / 2 : p / 2;
+}
+
+// The cut tiles the combine kernel merges: tile `tile`'s parts are those of shares first .. last.
+struct PrefillMerge {
+  int tile;
+  uint16_t first, last;
+};
+struct PrefillMergeArgs {
+  const float* ws;
+  uint16_t* out;
+  int M, gq, hkv, slots, slot_rows, two_slots, n;
+  PrefillMerge t[PF_MAX_SHARES];
 };
 
 // Online softmax of one 16-row block over 64 tokens, from the raw scores S[b][i] (token
@@ -3362,19 +3414,75 @@ __device__ __forceinline__ void pf_softmax(WaveState& st, const float (&S)[4][4]
 }
 
 __global__ __launch_bounds__(PF_THREADS, PF_WG_PER_CU) void prefill_chunk_kernel(PrefillArgs a) {
-  __shared__ __attribute__((aligned(16))) uint8_t stage[2][2 * CODE_BYTES + RULER_BYTES];
+  __shared__ __attribute__((aligned(16))) uint8_t stage[2][PF_STAGE];
   __shared__ __attribute__((aligned(16))) uint16_t ktile_buf[2][GT * PF_KROW];
   __shared__ __attribute__((aligned(16))) uint16_t vtile_buf[2][D * PF_VROW];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int h = blockIdx.x % a.hkv, tile = (blockIdx.x / a.hkv) % a.tiles, split = blockIdx.x / (a.hkv * a.tiles);
+  const int h = blockIdx.x % a.hkv, share = blockIdx.x / a.hkv;
   const int rows_h = a.M * a.gq;
+  const int G = (int)(a.U / GT);
+  const _Float16 one = (_Float16)1.0f;
+  const half8_t ones = half8_t{one, one, one, one, one, one, one, one};
+
+  int at = a.cut[share].tile, step0 = a.cut[share].step;
+  const int end_at = a.cut[share + 1].tile, end_step = a.cut[share + 1].step;
+  for (bool first_part = true; at < end_at || (at == end_at && step0 < end_step); first_part = false) {
+  const int tile = pf_tile_at(a, at);
+  const int nsteps = G + pf_fp16_groups(a, tile);
+  const int step1 = at < end_at ? nsteps : end_step;
+  if (!first_part) __syncthreads();  // every wave is done with the stages of the part before
   const int row0 = tile * PF_ROWS + wave * PF_RB * 16;  // first row of this wave
 
+  // cache group loads: wave w issues K and V code rows 8w .. 8w + 7 and half w & 1 of ruler
+  // w >> 1 (kst, kmn, vst, vmn)
+  auto issue = [&](int64_t grp, int sb) {
+    const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr(stage[sb]));
+    const void* kb = uniform_ptr(a.kq + ((int64_t)h * a.capacity + grp * GT) * D);
+    const void* vb = uniform_ptr(a.vq + ((int64_t)h * a.capacity + grp * GT) * D);
+    const int row = 8 * wave + (lane >> 3);
+    const uint32_t off = (uint32_t)(row * D + (((lane & 7) ^ swz(row)) << 4));
+    dma16(kb, off, base + 1024 * wave);
+    dma16(vb, off, base + CODE_BYTES + 1024 * wave);
+    const int64_t ro = ((int64_t)h * a.ngroups_cap + grp) * D + 64 * (wave & 1);
+    const int rw = wave >> 1;
+    const uint16_t* rsrc = rw == 0 ? a.kst : rw == 1 ? a.kmn : rw == 2 ? a.vst : a.vmn;
+    if (lane < 8) dma16(uniform_ptr(rsrc + ro), (uint32_t)(16 * lane), base + 2 * CODE_BYTES + 256 * rw + 128 * (wave & 1));
+  };
+  // fp16 group loads: wave w issues K and V rows 8w .. 8w + 7 (2 + 2 loads); a row keeps its 16-byte
+  // chunk x at position x ^ 2 (row & 7), so that the transposed V reads of 16 rows fall on distinct
+  // banks. Rows past the last token repeat it (they are masked).
+  auto issue16 = [&](int j, int sb) {
+    const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr(stage[sb]));
+    const void* kb = uniform_ptr(a.kc + (int64_t)h * a.kc_hs + (int64_t)j * GT * D);
+    const void* vb = uniform_ptr(a.vc + (int64_t)h * a.kc_hs + (int64_t)j * GT * D);
+    uint32_t off[2];
+    const int lane = tail_tid() & 63;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = 8 * wave + 4 * i + (lane >> 4);
+      off[i] = (uint32_t)(min(row, a.Mk - 1 - GT * j) * (2 * D) + (((lane & 15) ^ ((row & 7) << 1)) << 4));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      dma16(kb, off[i], base + 2048 * wave + 1024 * i);
+      dma16(vb, off[i], base + GT * D * 2 + 2048 * wave + 1024 * i);
+    }
+  };
+  auto issue_step = [&](int t) {  // step t's group into its stage
+    const int sb = (t - step0) & 1;
+    if (t < G) issue(t, sb);
+    else issue16(t - G, sb);
+  };
+  issue_step(step0);
+  if (step0 + 1 < step1) issue_step(step0 + 1);
+
   // ---- Q operands (B of S^T = K Q^T): lane (c, g) holds row 16 rb + c, dims of k-step k
+  // (here and after the steps: an opaque lane, so that these addresses do not stay live through them)
   half8_t qb[PF_RB][4];
 #pragma unroll
   for (int rb = 0; rb < PF_RB; ++rb) {
+    const int ol = tail_tid() & 63, c = ol & 15, g = ol >> 4;
     const int r = row0 + 16 * rb + c;
     const bool ok = r < rows_h;
     const int tk = ok ? r / a.gq : 0, hd = h * a.gq + (ok ? r % a.gq : 0);
@@ -3395,33 +3503,10 @@ __global__ __launch_bounds__(PF_THREADS, PF_WG_PER_CU) void prefill_chunk_kernel
     state_init(st[rb]);
     lsum[rb] = float4_t{0.f, 0.f, 0.f, 0.f};
   }
-  const _Float16 one = (_Float16)1.0f;
-  const half8_t ones = half8_t{one, one, one, one, one, one, one, one};
 
-  const int64_t G = a.U / GT;
-  const int64_t cs = (int64_t)split * G / a.splits, ce = (int64_t)(split + 1) * G / a.splits;
-  const int last_tok = min(rows_h - 1, (tile + 1) * PF_ROWS - 1) / a.gq;  // last query token of the tile
-  const int nchunk = min((a.Mk + GT - 1) / GT, (last_tok + a.qoff) / GT + 1);
 
-  // cache group loads: wave w issues K and V code rows 8w .. 8w + 7 and half w & 1 of ruler
-  // w >> 1 (kst, kmn, vst, vmn)
-  auto issue = [&](int64_t grp, int sb) {
-    const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr(stage[sb]));
-    const void* kb = uniform_ptr(a.kq + ((int64_t)h * a.capacity + grp * GT) * D);
-    const void* vb = uniform_ptr(a.vq + ((int64_t)h * a.capacity + grp * GT) * D);
-    const int row = 8 * wave + (lane >> 3);
-    const uint32_t off = (uint32_t)(row * D + (((lane & 7) ^ swz(row)) << 4));
-    dma16(kb, off, base + 1024 * wave);
-    dma16(vb, off, base + CODE_BYTES + 1024 * wave);
-    const int64_t ro = ((int64_t)h * a.ngroups_cap + grp) * D + 64 * (wave & 1);
-    const int rw = wave >> 1;
-    const uint16_t* rsrc = rw == 0 ? a.kst : rw == 1 ? a.kmn : rw == 2 ? a.vst : a.vmn;
-    if (lane < 8) dma16(uniform_ptr(rsrc + ro), (uint32_t)(16 * lane), base + 2 * CODE_BYTES + 256 * rw + 128 * (wave & 1));
-  };
-  constexpr int DMA_PF = 3;  // loads per wave and group
-
-  // ---- MFMA phase over the tiles in LDS; `mask_base` >= 0: chunk tokens from that index (causal)
-  auto attend_tiles = [&](int mask_base, int tb, auto&& tail_work) {
+  // ---- MFMA phase over the tiles in LDS; `masked`: fp16 tokens from mask_base on, causal
+  auto attend_tiles = [&](auto masked, int mask_base, int tb, auto&& convert) {
     const uint16_t* ktile = ktile_buf[tb];
     const uint16_t* vtile = vtile_buf[tb];
     float4_t S[PF_RB][4];
@@ -3456,16 +3541,20 @@ __global__ __launch_bounds__(PF_THREADS, PF_WG_PER_CU) void prefill_chunk_kernel
     };
     auto softmax = [&](int rb) {
       float sc[4][4];
-      const int tq = (row0 + 16 * rb + c) / a.gq;  // query token of row c (score column)
 #pragma unroll
       for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int kt = mask_base + 16 * b + 4 * g + i;
-          sc[b][i] = (mask_base < 0 || kt <= tq + a.qoff) ? S[rb][b][i] : NEG_INF;
-        }
-      // rows of the S^T layout are q rows c; the causal test above needs the row of column
-      // c, which is lane-independent of g: scores of lane (c, g) all belong to row c
+        for (int i = 0; i < 4; ++i) sc[b][i] = S[rb][b][i];
+      if constexpr (decltype(masked)::value) {
+        // scores of lane (c, g) all belong to query row c: the causal test needs that row's token
+        const int ol = tail_tid() & 63, mc = ol & 15, mg = ol >> 4;
+        const int tq = (row0 + 16 * rb + mc) / a.gq + a.qoff;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (mask_base + 16 * b + 4 * mg + i > tq) sc[b][i] = NEG_INF;
+      }
       pf_softmax(st[rb], sc, a.sl2, ph[rb], alpha[rb], moved[rb]);
 #if PF_SCHED
       // P is computed here, beside the other row block's products, not sunk past the rescale
@@ -3526,17 +3615,16 @@ __global__ __launch_bounds__(PF_THREADS, PF_WG_PER_CU) void prefill_chunk_kernel
     }
 #endif
     rescale(1);
-    // PV(1) and the caller's work (the next group's dequantization) in one basic block: the
-    // compiler interleaves the two by itself
-    tail_work();
+    // PV(1) and the next group's conversion in one basic block: the compiler interleaves the two
+    // by itself
+    convert();
     pv(1);
   };
 
-  // ---- cache groups: two LDS stages of int8 codes and two fp16 tile buffers. Group t's codes
-  // are dequantized into tile buffer t & 1 during group t - 1's last product (PV of the second
-  // row block), so a group takes one workgroup barrier: after it, tile buffer t & 1 is complete,
-  // the codes of group t + 1 have landed, and every wave is done with tile buffer (t + 1) & 1 and
-  // with the stage of group t
+  // ---- the steps: two LDS stages and two fp16 tile buffers. Step t + 1's group is converted into
+  // tile buffer (t + 1) & 1 during step t's last product (PV of the second row block), so a group
+  // takes one workgroup barrier: after it, tile buffer t & 1 is complete, the loads of group t + 1
+  // have landed, and every wave is done with tile buffer (t + 1) & 1 and with the stage of group t
   auto dequant = [&](const uint8_t* sg, uint16_t* ktile, uint16_t* vtile) {
     const uint16_t* rks = reinterpret_cast<const uint16_t*>(sg + 2 * CODE_BYTES);
     // K: thread t dequantizes row t >> 3, dims 16 (t & 7) .. + 15
@@ -3564,98 +3652,191 @@ __global__ __launch_bounds__(PF_THREADS, PF_WG_PER_CU) void prefill_chunk_kernel
             dq8_splat(vw.x, vw.y, half2_t{vs, vs}, half2_t{vm, vm});
       }
   };
-  if (cs < ce) {
-    issue(cs, 0);
-    if (cs + 1 < ce) {
-      issue(cs + 1, 1);
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DMA_PF) : "memory");
-    } else {
-      wait_groups_all();
-    }
-    __syncthreads();  // stage 0 is complete
-    dequant(stage[0], ktile_buf[0], vtile_buf[0]);
-  }
-  for (int64_t grp = cs; grp < ce; ++grp) {
-    const int tb = (int)((grp - cs) & 1);  // tile buffer and stage of group grp
-    wait_groups_all();                     // the codes of group grp + 1 (the only loads in flight)
-    __syncthreads();
-    if (grp + 2 < ce) issue(grp + 2, tb);  // into the stage of group grp, dequantized before the barrier
-    // (after the last group the dequantization reads a stale stage into a tile buffer nothing
-    // reads again: unconditional, so that it stays in one basic block with the product)
-    attend_tiles(-1, tb, [&]() { dequant(stage[tb ^ 1], ktile_buf[tb ^ 1], vtile_buf[tb ^ 1]); });
-  }
-
-  // ---- fp16 groups (causal): j = split, split + S, ...
-  for (int j = split; j < nchunk; j += a.splits) {
-    __syncthreads();  // every wave is done with the tiles
-    {
-      uint16_t* ktile = ktile_buf[0];
-      uint16_t* vtile = vtile_buf[0];
-      const int row = tid >> 3, cp = tid & 7, t = GT * j + row;
-      const bool ok = t < a.Mk;
-      const uint16_t* kr = a.kc + (int64_t)h * a.kc_hs + (int64_t)(ok ? t : 0) * D + 16 * cp;
-      const uint16_t* vr = a.vc + (int64_t)h * a.kc_hs + (int64_t)(ok ? t : 0) * D + 16 * cp;
-      const int vs = pf_vslot(row);
+  // fp16 groups: the staged rows are moved into the tiles (V through the 16-bit transpose read)
+  auto place16 = [&](const uint8_t* sg, uint16_t* ktile, uint16_t* vtile) {
+    // (an opaque thread index: these offsets are computed here, not kept live through the int8 steps,
+    // which leave no registers for them)
+    const int ot = tail_tid(), row = ot >> 3, ch = ot & 7, c = ot & 15, g = (ot & 63) >> 4;
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      *reinterpret_cast<uint4*>(ktile + row * PF_KROW + 16 * ch + 8 * e) =
+          *reinterpret_cast<const uint4*>(sg + row * (2 * D) + (((2 * ch + e) ^ ((row & 7) << 1)) << 4));
+    // wave w covers dims 16 w .. + 15: lane (c, g) supplies a quarter (c & 3) of row c >> 2 of four
+    // rows and receives dim 16 w + c of those four tokens
+#pragma unroll
+    for (int B = 0; B < 2; ++B) {
+      u32x2 v[2];
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
-        const uint4 kw = ok ? *reinterpret_cast<const uint4*>(kr + 8 * e) : uint4{0, 0, 0, 0};
-        const uint4 vw = ok ? *reinterpret_cast<const uint4*>(vr + 8 * e) : uint4{0, 0, 0, 0};
-        *reinterpret_cast<uint4*>(ktile + row * PF_KROW + 16 * cp + 8 * e) = kw;
-        const uint32_t wv[4] = {vw.x, vw.y, vw.z, vw.w};
+        const int vrow = 32 * B + 16 * e + 4 * g + (c >> 2);
+        v[e] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_v4s_t*)(const lds_void_t*)(sg + GT * D * 2 + vrow * (2 * D) +
+                                            (((2 * wave + ((c >> 1) & 1)) ^ ((vrow & 7) << 1)) << 4) + 8 * (c & 1))));
+      }
+      *reinterpret_cast<uint4*>(vtile + (16 * wave + c) * PF_VROW + 32 * B + 8 * g) =
+          uint4{v[0].x, v[0].y, v[1].x, v[1].y};
+    }
+  };
+  const int ce = min(step1, G);  // cache groups: steps step0 .. ce - 1
+  wait_groups_all();
+  __syncthreads();  // the first two groups have landed
+  auto convert = [&](int t) {  // step t's group from its stage into its tile buffer
+    const int tb = (t - step0) & 1;
+    if (t < G) dequant(stage[tb], ktile_buf[tb], vtile_buf[tb]);
+    else place16(stage[tb], ktile_buf[tb], vtile_buf[tb]);
+  };
+  convert(step0);
+  // this wave's rows attend the steps up to `end` (of a tile with many tokens, the last waves' rows have
+  // more; none for rows past the last); it joins the conversions and barriers of the others
+  const int end = row0 < rows_h ? min(step1, G + pf_fp16_to(a, row0 + PF_RB * 16 - 1)) : step0;
+  int t = step0;
+  if (t < min(ce, end)) {
+    for (; t < ce; ++t) {
+      const int tb = (t - step0) & 1;  // tile buffer and stage of step t
+      wait_groups_all();               // the loads of step t + 1 (the only ones in flight)
+      __syncthreads();
+      if (t + 2 < step1) issue_step(t + 2);  // into the stage of step t, converted before the barrier
+      // (after the last group the dequantization reads a stage of something else into a tile buffer
+      // nothing reads: unconditional, so that it stays in one basic block with the product)
+      attend_tiles(std::false_type{}, 0, tb, [&]() { dequant(stage[tb ^ 1], ktile_buf[tb ^ 1], vtile_buf[tb ^ 1]); });
+    }
+    if (t < step1) {  // the first fp16 group, loaded by now
+      wait_groups_all();
+      __syncthreads();
+      convert(t);
+    }
+  }
+  // the fp16 groups: first those that all of the wave's rows see whole, then the ones with a causal mask
+  if (G <= t && t < end) {
+    auto step16 = [&](auto masked) {
+      const int tb = (t - step0) & 1;
+      wait_groups_all();
+      __syncthreads();
+      if (t + 2 < step1) issue16(t + 2 - G, tb);
+      attend_tiles(masked, GT * (t - G), tb, [&]() { place16(stage[tb ^ 1], ktile_buf[tb ^ 1], vtile_buf[tb ^ 1]); });
+    };
+    const int whole = min(end, G + (row0 / a.gq + a.qoff + 1) / GT);
+    for (; t < whole; ++t) step16(std::false_type{});
+    for (; t < end; ++t) step16(std::true_type{});
+  }
+  for (; t < step1; ++t) {  // the conversions and barriers alone
+    wait_groups_all();
+    __syncthreads();
+    if (t + 2 < step1) issue_step(t + 2);
+    if (t + 1 >= step1) continue;
+    if (t + 1 == ce) {  // (the barrier that the attending waves take there)
+      wait_groups_all();
+      __syncthreads();
+    }
+    convert(t + 1);
+  }
+
+  const int ol = tail_tid() & 63, c = ol & 15, g = ol >> 4;
+  if (step0 == 0 && step1 == nsteps) {
+    // ---- the whole tile: out = acc / l (both x 2^15), through the wave's rows of the stages so that
+    // 16 lanes store a row's 256 bytes (the 2-byte values at chunk ^ 2 ((row >> 2) & 3))
+    __syncthreads();  // every wave is past its last read of the stages
+    uint8_t* ow = &stage[0][0] + wave * (PF_RB * 16 * D * 2);
 #pragma unroll
-        for (int q2 = 0; q2 < 8; ++q2)
-          vtile[(16 * cp + 8 * e + q2) * PF_VROW + vs] = (uint16_t)(wv[q2 >> 1] >> (16 * (q2 & 1)));
+    for (int rb = 0; rb < PF_RB; ++rb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float l = lsum[rb][i], inv = l > 0.0f ? 1.0f / l : 0.0f;
+        const int r = 16 * rb + 4 * g + i;
+#pragma unroll
+        for (int cb = 0; cb < 8; ++cb)
+          *reinterpret_cast<uint16_t*>(ow + r * (2 * D) + (((2 * cb + (c >> 3)) ^ (((r >> 2) & 3) << 1)) << 4) + 2 * (c & 7)) =
+              f2h(st[rb].acc[cb][i] * inv);
+      }
+#pragma unroll
+    for (int k = 0; k < PF_RB * 4; ++k) {
+      const int r = 4 * k + g;
+      const uint4 v = *reinterpret_cast<const uint4*>(ow + r * (2 * D) + ((c ^ (((r >> 2) & 3) << 1)) << 4));
+      const int row = row0 + r;
+      if (row < rows_h) {
+        const int tk = row / a.gq, hd = h * a.gq + row % a.gq;
+        *reinterpret_cast<uint4*>(a.out + ((int64_t)hd * a.M + tk) * D + 8 * c) = v;
       }
     }
-    __syncthreads();
-    attend_tiles(GT * j, 0, []() {});
-  }
-
-  // ---- one partial per row: acc[128] and l (both x 2^15), m (log2 domain)
-  const int64_t total_rows = (int64_t)a.hkv * rows_h;
+  } else {
+    // ---- one partial per row: acc[128] and l (both x 2^15), m (log2 domain)
+    float* dst = a.ws + ((int64_t)h * a.slots + pf_slot(a, share, step0 == 0)) * a.slot_rows * PF_PART;
 #pragma unroll
-  for (int rb = 0; rb < PF_RB; ++rb) {
-    const int rbase = row0 + 16 * rb;
-    float* dst = a.ws + ((int64_t)split * total_rows + (int64_t)h * rows_h) * PF_PART;
-    if (g == 0 && rbase + c < rows_h) dst[(int64_t)(rbase + c) * PF_PART + D] = st[rb].m;
+    for (int rb = 0; rb < PF_RB; ++rb) {
+      const int r0 = wave * PF_RB * 16 + 16 * rb, n = rows_h - tile * PF_ROWS;  // rows of the tile: [0, n)
+      if (g == 0 && r0 + c < n) dst[(int64_t)(r0 + c) * PF_PART + D] = st[rb].m;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (c == 0 && rbase + 4 * g + i < rows_h) dst[(int64_t)(rbase + 4 * g + i) * PF_PART + D + 1] = lsum[rb][i];
+      for (int i = 0; i < 4; ++i)
+        if (c == 0 && r0 + 4 * g + i < n) dst[(int64_t)(r0 + 4 * g + i) * PF_PART + D + 1] = lsum[rb][i];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = rbase + 4 * g + i;
-      if (r < rows_h)
+      for (int i = 0; i < 4; ++i) {
+        const int r = r0 + 4 * g + i;
+        if (r < n)
 #pragma unroll
-        for (int cb = 0; cb < 8; ++cb) dst[(int64_t)r * PF_PART + 16 * cb + c] = st[rb].acc[cb][i];
+          for (int cb = 0; cb < 8; ++cb) dst[(int64_t)r * PF_PART + 16 * cb + c] = st[rb].acc[cb][i];
+      }
     }
   }
+  ++at;
+  step0 = 0;
+  }  // parts
 }
 
-// Merge of the splits' partials: one thread per (row, 4 dims).
-__global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
-  const int rows_h = a.M * a.gq;
-  const int64_t total_rows = (int64_t)a.hkv * rows_h;
-  const int64_t item = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (item >= total_rows * (D / 4)) return;
-  const int64_t row = item / (D / 4);
-  const int d4 = (int)(item % (D / 4)) * 4;
-  float m = NEG_INF;
-  for (int s = 0; s < a.splits; ++s) m = fmaxf(m, a.ws[((int64_t)s * total_rows + row) * PF_PART + D]);
+// Merge of a cut tile's partials: 32 lanes per row, 4 dims each, 8 rows per workgroup. Latency-bound
+// for few rows and many parts, so the lanes read 32 parts' m and l at once (their weights pass
+// between lanes), and the columns of 8 parts are in flight together.
+__global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillMergeArgs a) {
+  const int rows_h = a.M * a.gq, blocks = (a.slot_rows + 7) / 8;
+  const int h = blockIdx.x % a.hkv, rest = blockIdx.x / a.hkv;
+  const PrefillMerge t = a.t[rest / blocks];
+  const int lr = rest % blocks * 8 + ((int)threadIdx.x >> 5), l32 = (int)threadIdx.x & 31;
+  const int r = t.tile * PF_ROWS + lr;
+  if (lr >= a.slot_rows || r >= rows_h) return;  // (whole rows: 32 lanes agree)
+  auto part = [&](int w) {
+    const int slot = a.two_slots ? 2 * w + (w == t.first ? 1 : 0) : w;
+    return a.ws + (((int64_t)h * a.slots + slot) * a.slot_rows + lr) * PF_PART;
+  };
+  // the row's maximum and each lane's first part
+  float m = NEG_INF, m0 = NEG_INF, l0 = 0.0f;
+  for (int w = t.first + l32; w <= t.last; w += 32) {
+    const float2 ml = *reinterpret_cast<const float2*>(part(w) + D);
+    if (w == t.first + l32) {
+      m0 = ml.x;
+      l0 = ml.y;
+    }
+    m = fmaxf(m, ml.x);
+  }
+#pragma unroll
+  for (int o = 16; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 32));
   const float mu = m == NEG_INF ? 0.0f : m;
   float4 acc = {0.f, 0.f, 0.f, 0.f};
   float l = 0.0f;
-  for (int s = 0; s < a.splits; ++s) {
-    const float* p = a.ws + ((int64_t)s * total_rows + row) * PF_PART;
-    const float ms = p[D];
-    const float w = ms == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(ms - mu);
-    const float4 v = *reinterpret_cast<const float4*>(p + d4);
-    acc.x += v.x * w; acc.y += v.y * w; acc.z += v.z * w; acc.w += v.w * w;
-    l += p[D + 1] * w;
+  for (int w0 = t.first; w0 <= t.last; w0 += 32) {
+    if (w0 != t.first) {
+      const bool on = w0 + l32 <= t.last;
+      m0 = on ? part(w0 + l32)[D] : NEG_INF;
+      l0 = on ? part(w0 + l32)[D + 1] : 0.0f;
+    }
+    const float wt = m0 == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(m0 - mu);
+    const int n = min(32, t.last + 1 - w0);
+    for (int k = 0; k < n; k += 8) {
+      float4 v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        v[e] = *reinterpret_cast<const float4*>(part(w0 + min(k + e, n - 1)) + 4 * l32);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float we = __shfl(wt, min(k + e, 31), 32), le = __shfl(l0, min(k + e, 31), 32);
+        if (k + e < n) {
+          acc.x += v[e].x * we; acc.y += v[e].y * we; acc.z += v[e].z * we; acc.w += v[e].w * we;
+          l += le * we;
+        }
+      }
+    }
   }
-  const int h = (int)(row / rows_h), r = (int)(row % rows_h);
   const int tk = r / a.gq, hd = h * a.gq + r % a.gq;
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;  // acc and l carry the same 2^15 scale
-  uint16_t* o = a.out + ((int64_t)hd * a.M + tk) * D + d4;
+  uint16_t* o = a.out + ((int64_t)hd * a.M + tk) * D + 4 * l32;
   *reinterpret_cast<uint2*>(o) = uint2{(uint32_t)f2h(acc.x * inv) | ((uint32_t)f2h(acc.y * inv) << 16),
                                        (uint32_t)f2h(acc.z * inv) | ((uint32_t)f2h(acc.w * inv) << 16)};
 }
@@ -4419,6 +4600,132 @@ extern "C" int64_t nkv_prefill_workspace_bytes(int64_t hkv, int64_t hq, int64_t 
   return splits * hq * m * PF_PART * (int64_t)sizeof(float);
 }
 
+// ---- how a head's steps are cut into shares. A step (64 tokens against 256 rows) takes a CU about
+// 2 us. Three cuttings; the one whose longest share is the shortest, its other costs counted in steps:
+//  - at tile boundaries (nothing to merge): many tiles per share;
+//  - every tile into the same number of parts: few tiles of about equal length (512 tokens over 16384:
+//    8 tiles x 4 parts). The partials' writes and the combine kernel cost about 6 steps;
+//  - even shares of the head's steps, wherever they end (a cut within 4 steps of a tile boundary moves
+//    there): tiles of unequal length, or a number of them that does not fit the CUs.
+// The first and the last take the tiles in zigzag order, so that each two neighbours have the same
+// sum: with a tile per share, only every second one is cut (2048 tokens: 32 tiles, the last with 31
+// more steps than the first). The last two take what slots the workspace has;
+// nkv_prefill_workspace_bytes always holds the second's.
+constexpr double PF_TILE_COST = 1.0, PF_PARTS_COST = 6.0, PF_EVEN_COST = 8.0;
+constexpr int64_t PF_MIN_SHARE = 4;  // steps of an even share, at least
+constexpr int64_t PF_SNAP = 4;
+
+struct PrefillPlan {
+  int shares = 0, slots = 0, two_slots = 0, merges = 0, zigzag = 0;
+  PrefillCut cut[PF_MAX_SHARES + 1];
+  PrefillMerge merge[PF_MAX_SHARES];
+};
+
+static int64_t prefill_slot_bytes(const PrefillArgs& a) {
+  return (int64_t)a.hkv * a.slot_rows * PF_PART * (int64_t)sizeof(float);
+}
+
+// `W` shares of about T / W steps into p, each cut moved to a tile boundary it is within `snap` steps
+// of; returns the longest share in steps, each of its tiles counted PF_TILE_COST more. T: the head's
+// steps.
+static double prefill_cut(const PrefillArgs& a, int64_t T, int64_t W, int64_t snap, PrefillPlan& p) {
+  const int64_t G = a.U / GT;
+  p.shares = (int)W;
+  int64_t before = 0, last = 0;  // steps before position t, and before the cut before
+  double longest = 0.0;
+  int t = 0;
+  for (int64_t w = 0; w <= W; ++w) {
+    const int64_t at = w * T / W;
+    int64_t n = 0;
+    while (t < a.tiles && before + (n = G + pf_fp16_groups(a, pf_tile_at(a, t))) <= at) {
+      before += n;
+      ++t;
+    }
+    PrefillCut c{t, (int)(at - before)};
+    int64_t pos = at;
+    if (c.step && c.step <= snap && at - before <= before + n - at) {
+      c = PrefillCut{t, 0};
+      pos = before;
+    } else if (c.step && before + n - at <= snap) {
+      c = PrefillCut{t + 1, 0};
+      pos = before + n;
+    }
+    p.cut[w] = c;
+    if (w > 0) longest = std::max(longest, (double)(pos - last) + PF_TILE_COST * (c.tile - p.cut[w - 1].tile + (c.step > 0)));
+    last = pos;
+  }
+  return longest;
+}
+
+// `splits` > 0 bounds the shares to splits per tile; `parts` is the parts per tile of the second
+// cutting. Leaves the chosen order in `a` and in p.
+static void prefill_plan(PrefillArgs& a, int64_t splits, int64_t parts, int64_t avail_slots, PrefillPlan& p) {
+  const int64_t G = a.U / GT;
+  const int64_t cap = std::max<int64_t>(1, PF_MAX_SHARES / a.hkv);  // one workgroup per CU
+  const int64_t W = std::min<int64_t>(cap, a.tiles);
+  int64_t T = 0, longest = 0;
+  for (int t = 0; t < a.tiles; ++t) {
+    const int64_t n = G + pf_fp16_groups(a, t);
+    T += n;
+    longest = std::max(longest, n);
+  }
+  // parts per tile (no part without a step: tile 0 is the shortest), and the even shares
+  const int64_t per_tile = std::max<int64_t>(1, std::min({parts, (int64_t)(PF_MAX_SHARES / a.tiles), G + pf_fp16_groups(a, 0)}));
+  int64_t We = std::max<int64_t>(a.tiles, T / PF_MIN_SHARE);
+  if (splits > 0) We = std::min<int64_t>(We, a.tiles * splits);
+  We = std::min(We, std::min(cap, T));
+  const double none = __builtin_huge_val();
+  a.zigzag = 1;
+  const double c_even = 2 * We <= avail_slots ? prefill_cut(a, T, We, PF_SNAP, p) + PF_EVEN_COST : none;
+  const double c_tiles = prefill_cut(a, T, W, INT64_MAX, p);
+  const double c_parts = per_tile > 1 && a.tiles * per_tile <= avail_slots
+                             ? (double)(cdiv(longest, per_tile) * cdiv(a.tiles * per_tile, cap)) + PF_PARTS_COST : none;
+  const double best = std::min({c_tiles, c_parts, c_even});
+  p.zigzag = a.zigzag = best != c_parts;
+  if (best == c_tiles) return;  // (cut already)
+  if (best == c_parts) {
+    p.shares = (int)(a.tiles * per_tile);
+    p.slots = p.shares;
+    for (int w = 0; w < p.shares; ++w) {
+      const int t = (int)(w / per_tile);
+      p.cut[w] = PrefillCut{t, (int)((G + pf_fp16_groups(a, t)) * (w % per_tile) / per_tile)};
+    }
+    p.cut[p.shares] = PrefillCut{a.tiles, 0};
+  } else {
+    prefill_cut(a, T, We, PF_SNAP, p);
+    p.two_slots = 1;
+    p.slots = (int)(2 * We);
+  }
+  for (int w = 1; w < p.shares; ++w) {
+    if (p.cut[w].step == 0) continue;
+    const int tile = pf_tile_at(a, p.cut[w].tile);
+    if (p.merges && p.merge[p.merges - 1].tile == tile) p.merge[p.merges - 1].last = (uint16_t)w;
+    else p.merge[p.merges++] = PrefillMerge{tile, (uint16_t)(w - 1), (uint16_t)w};
+  }
+}
+
+static void prefill_shape(PrefillArgs& a, int64_t hkv, int64_t hq, int64_t m, int64_t m_kv, int64_t used) {
+  a.M = (int)m; a.hq = (int)hq; a.hkv = (int)hkv; a.gq = (int)(hq / hkv);
+  a.tiles = (int)cdiv(m * a.gq, PF_ROWS);
+  a.Mk = (int)m_kv; a.qoff = (int)(m_kv - m);
+  a.U = used;
+  a.slot_rows = (int)std::min<int64_t>(PF_ROWS, m * a.gq);
+}
+
+extern "C" int64_t nkv_prefill_preferred_bytes(int64_t hkv, int64_t hq, int64_t m, int64_t m_kv, int64_t used,
+                                               int64_t splits) {
+  if (hkv <= 0 || hq <= 0 || hq % hkv || hq / hkv > 16 || m <= 0 || m > (1 << 20) || m_kv < m || m_kv > (1 << 24) ||
+      used < 0 || used % GT)
+    return 0;
+  PrefillArgs a{};
+  prefill_shape(a, hkv, hq, m, m_kv, used);
+  PrefillPlan p;
+  const int64_t parts = splits > 0 ? splits : nkv_prefill_default_splits(hkv, hq, m, used);
+  prefill_plan(a, splits, parts, INT64_MAX, p);
+  const int64_t least = nkv_prefill_workspace_bytes(hkv, hq, m, parts);
+  return std::max<int64_t>(least, p.slots * prefill_slot_bytes(a));
+}
+
 static int prefill_attn(const char* what, const uint16_t* q, int64_t m, const uint16_t* k16, const uint16_t* v16,
                         int64_t m_kv, int64_t kv_head_stride, const uint8_t* kq, const uint16_t* kmn,
                         const uint16_t* kst, const uint8_t* vq, const uint16_t* vmn, const uint16_t* vst,
@@ -4440,24 +4747,29 @@ static int prefill_attn(const char* what, const uint16_t* q, int64_t m, const ui
   if (!al16(q) || !al16(k16) || !al16(v16) || !al16(out) || !al16(workspace) ||
       (used > 0 && (!al16(kq) || !al16(vq) || !al16(kmn) || !al16(kst) || !al16(vmn) || !al16(vst))))
     return fail(NKV_ERR_UNSUPPORTED, "%s: buffers must be 16-byte aligned", what);
-  const int64_t gq = hq / hkv, rows_h = m * gq, tiles = cdiv(rows_h, PF_ROWS);
-  if (splits <= 0) splits = nkv_prefill_default_splits(hkv, hq, m, used);
-  if (workspace_bytes < nkv_prefill_workspace_bytes(hkv, hq, m, splits))
+  const int64_t parts = splits > 0 ? splits : nkv_prefill_default_splits(hkv, hq, m, used);
+  if (workspace_bytes < nkv_prefill_workspace_bytes(hkv, hq, m, parts))
     return fail(NKV_ERR_INVALID, "%s: workspace of %lld bytes, need %lld", what, (long long)workspace_bytes,
-                (long long)nkv_prefill_workspace_bytes(hkv, hq, m, splits));
+                (long long)nkv_prefill_workspace_bytes(hkv, hq, m, parts));
   PrefillArgs a{};
   a.q = q; a.kc = k16; a.vc = v16;
   a.kq = kq; a.kmn = kmn; a.kst = kst; a.vq = vq; a.vmn = vmn; a.vst = vst;
-  a.capacity = capacity; a.ngroups_cap = cdiv(capacity, GT); a.U = used;
-  a.M = (int)m; a.hq = (int)hq; a.hkv = (int)hkv; a.gq = (int)gq; a.splits = (int)splits; a.tiles = (int)tiles;
-  a.Mk = (int)m_kv; a.qoff = (int)(m_kv - m); a.kc_hs = kv_head_stride;
+  a.capacity = capacity; a.ngroups_cap = cdiv(capacity, GT);
+  prefill_shape(a, hkv, hq, m, m_kv, used);
+  a.kc_hs = kv_head_stride;
   a.sl2 = LOG2E / sqrtf((float)head_dim);
   a.ws = static_cast<float*>(workspace); a.out = out;
+  PrefillPlan p;
+  prefill_plan(a, splits, parts, workspace_bytes / prefill_slot_bytes(a), p);
+  a.shares = p.shares; a.slots = p.slots; a.two_slots = p.two_slots;
+  for (int w = 0; w <= p.shares; ++w) a.cut[w] = p.cut[w];
   hipStream_t s = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(prefill_chunk_kernel, dim3((unsigned)(hkv * tiles * splits)), dim3(PF_THREADS), 0, s, a);
+  hipLaunchKernelGGL(prefill_chunk_kernel, dim3((unsigned)(hkv * p.shares)), dim3(PF_THREADS), 0, s, a);
   if (int rc = check_launch(what)) return rc;
-  const int64_t items = hq * m * (D / 4);
-  hipLaunchKernelGGL(prefill_combine_kernel, dim3((unsigned)cdiv(items, 256)), dim3(256), 0, s, a);
+  if (!p.merges) return NKV_OK;
+  PrefillMergeArgs c{a.ws, out, a.M, a.gq, a.hkv, a.slots, a.slot_rows, a.two_slots, p.merges, {}};
+  for (int i = 0; i < p.merges; ++i) c.t[i] = p.merge[i];
+  hipLaunchKernelGGL(prefill_combine_kernel, dim3((unsigned)(hkv * p.merges * cdiv(a.slot_rows, 8))), dim3(256), 0, s, c);
   return check_launch(what);
 }
 

@@ -295,17 +295,16 @@ def int8_prefill_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Ten
     if out is None:
         out = torch.empty_like(query)
     lib = _lib.load()
-    if splits <= 0:
-        splits = int(lib.nkv_prefill_default_splits(hkv, hq, n, used + (m - n) // GROUP_T * GROUP_T))
-    need = int(lib.nkv_prefill_workspace_bytes(hkv, hq, n, splits))
+    least = splits if splits > 0 else int(lib.nkv_prefill_default_splits(hkv, hq, n, used + (m - n) // GROUP_T * GROUP_T))
+    need = int(lib.nkv_prefill_workspace_bytes(hkv, hq, n, least))
     if scratch is None or scratch.numel() * scratch.element_size() < need:
         if _capturing():
             raise ValueError("under graph capture int8_prefill_attend needs a large enough scratch")
-        scratch = _lib.workspace(query.device, need)
+        scratch = _lib.workspace(query.device, max(need, int(lib.nkv_prefill_preferred_bytes(hkv, hq, n, m, used, splits))))
     _lib.call("nkv_prefill_attn_hist_t64", query.data_ptr(), n, key.data_ptr(), value.data_ptr(), m,
               key.stride(1), kq.data_ptr(), kmn.data_ptr(), kst.data_ptr(), vq.data_ptr(), vmn.data_ptr(),
               vst.data_ptr(), cap, used, hq, hkv, d, out.data_ptr(), scratch.data_ptr(),
-              scratch.numel() * scratch.element_size(), splits, _lib.stream_ptr(query.device))
+              scratch.numel() * scratch.element_size(), max(0, splits), _lib.stream_ptr(query.device))
     return out
 
 

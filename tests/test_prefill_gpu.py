@@ -161,3 +161,34 @@ def test_staged_prefill_in_three_chunks_against_oracle():
                                                                  f"mean {err.mean():.2e}")
         off += n
     cache.finish_prefill(total)
+
+
+@pytest.mark.parametrize("hq,hkv,used,m,hist,least", [
+    (4, 1, 192, 1999, 0, False),    # even shares in zigzag order: parts of one step up to whole tiles
+    (4, 1, 192, 1999, 0, True),     # the least workspace: tile boundaries alone
+    (16, 1, 0, 700, 130, False),    # 16 tokens per tile, an fp16 history that ends inside a group
+    (2, 2, 64, 1025, 0, False),     # 256 tokens per tile: waves of a tile end at different groups
+    (6, 2, 1088, 171, 0, False),    # 3 heads per KV head: tiles that start inside a token
+    (8, 8, 320, 64, 0, True),       # parts per tile, in the least workspace
+])
+def test_prefill_cuttings(hq, hkv, used, m, hist, least):
+    """Each way the work of a head is cut over the workgroups, against the oracle."""
+    from nova_amd import _lib
+    from nova_amd.kvattn import int8_prefill_attend
+
+    print(f"case hq={hq} hkv={hkv} used={used} m={m} hist={hist} least={least}", flush=True)
+    q, k16, v16, packed = _case(hq, hkv, used, m + hist, seed=95 + m)
+    q = q[:, :, hist:].contiguous()
+    lib, scratch = _lib.load(), None
+    if least:
+        splits = int(lib.nkv_prefill_default_splits(hkv, hq, m, used))
+        scratch = torch.empty(int(lib.nkv_prefill_workspace_bytes(hkv, hq, m, splits)), dtype=torch.uint8, device="cuda")
+    got = int8_prefill_attend(q, k16, v16, *packed, used=used, scratch=scratch)
+    # the oracle takes a chunk of all fp16 tokens; its last m queries are this call's
+    kq, kmn, kst, vq, vmn, vst = (npy(t)[0] for t in packed)
+    qa = torch.zeros(1, hq, m + hist, D, dtype=q.dtype)
+    qa[:, :, hist:] = q.cpu()
+    want = oattn.chunk_prefill_attend(npy(qa)[0], kq, kmn, kst, vq, vmn, vst, used, npy(k16)[0], npy(v16)[0])[:, hist:]
+    err = np.abs(npy(got)[0].astype(np.float64) - want)
+    assert err.max() <= 2e-3, f"max abs {err.max():.2e}"
+    assert err.mean() <= 1.5e-4, f"mean abs {err.mean():.2e}"
