@@ -200,15 +200,6 @@ __device__ __forceinline__ int swz(int row) { return ((row >> 1) & 7) ^ (((row >
 // so the 16 rows a K operand read touches land on 16 distinct banks.
 __device__ __forceinline__ int ring_chunk_pos(int row, int chunk) { return chunk ^ (row & 15); }
 
-// Reductions over the 4 lanes {l, l^16, l^32, l^48} with the gfx950 permlane swaps (VALU
-// only, no LDS round trip). permlane16_swap(x, x) returns rows (0,0,2,2) and (1,1,3,3) of
-// x, permlane32_swap(x, x) its lower and upper halves twice.
-__device__ __forceinline__ float max4rows(float v) {
-  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
 __device__ __forceinline__ float sum4rows(float v) {
   auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
@@ -961,13 +952,6 @@ __device__ __forceinline__ void attend_ring16(const AttnArgs& a, WaveState& st, 
 }
 
 // ---------------------------------------------------------------- ring append
-
-__device__ __forceinline__ float min4rows(float v) {
-  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = fminf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fminf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
 
 __device__ __forceinline__ const uint16_t* ring_of(const AttnArgs& a, int h, int which) {
   return (which == 0 ? a.tail_k : a.tail_v) + (int64_t)h * a.tail_slots * D;

@@ -66,38 +66,62 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
 __device__ __forceinline__ float shfl_xor(float v, int m) { return __shfl_xor(v, m, 64); }
 __device__ __forceinline__ float shfl(float v, int src) { return __shfl(v, src, 64); }
 
+// Reductions over the 4 lanes {l, l^16, l^32, l^48} with the gfx950 permlane swaps (VALU
+// only, no LDS round trip). permlane16_swap(x, x) returns rows (0,0,2,2) and (1,1,3,3) of
+// x, permlane32_swap(x, x) its lower and upper halves twice.
+__device__ __forceinline__ float max4rows(float v) {
+  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float min4rows(float v) {
+  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fminf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fminf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
 // The int8t64 ruler arithmetic shared by every quantizer in this library, written with
 // explicit round-to-nearest intrinsics so that no contraction changes a bit:
 //   step = max((mx - mn) / 255, 1e-8), code = clamp(rint((x - mn) / step), 0, 255).
 __device__ __forceinline__ float ruler_step(float mn, float mx) {
   return fmaxf(__fdiv_rn(__fsub_rn(mx, mn), 255.0f), 1e-8f);
 }
-__device__ __forceinline__ uint32_t ruler_code(float x, float mn, float step) {
-  float r = __builtin_rintf(__fdiv_rn(__fsub_rn(x, mn), step));
-  r = fminf(fmaxf(r, 0.0f), 255.0f);
-  return (uint32_t)r;
+// The quotient taken as (x - mn) * inv, inv = rcp(step) (<= 1 ulp). For quotients in [0, 256] that
+// product is within 2^-14 of the exact quotient, and the correctly rounded quotient within 2^-16 of it,
+// so both round to the same integer unless the product lies within 2^-12 of a half-integer; there the
+// IEEE division decides. The result is that of the division for every input. (The code as a float.)
+__device__ __forceinline__ float ruler_code_f(float x, float mn, float step, float inv) {
+  const float d = __fsub_rn(x, mn), q = __fmul_rn(d, inv);
+  float r = __builtin_rintf(q);
+  if (__builtin_fabsf(q - r) > 0.5f - 0x1p-12f) r = __builtin_rintf(__fdiv_rn(d, step));
+  return fminf(fmaxf(r, 0.0f), 255.0f);
 }
-
-// The same code with the quotient taken as (x - mn) * inv, inv = rcp(step) (<= 1 ulp).
-// For quotients in [0, 256] that product is within 2^-14 of the exact quotient, and the
-// correctly rounded quotient within 2^-16 of it, so both round to the same integer unless
-// the product lies within 2^-12 of a half-integer; there the IEEE division decides. The
-// result is identical to ruler_code for every input.
 __device__ __forceinline__ uint32_t ruler_code_rcp(float x, float mn, float step, float inv) {
-  const float d = __fsub_rn(x, mn);
-  float q = __fmul_rn(d, inv);
-  if (__builtin_fabsf((q - __builtin_floorf(q)) - 0.5f) < 0x1p-12f) q = __fdiv_rn(d, step);
-  const float r = fminf(fmaxf(__builtin_rintf(q), 0.0f), 255.0f);
-  return (uint32_t)r;
+  return (uint32_t)ruler_code_f(x, mn, step, inv);
+}
+// Eight such codes packed, one byte each (they are integers in 0 .. 255: the conversion is exact).
+__device__ __forceinline__ uint2 pack_u8x8(const float (&c)[8]) {
+  uint2 r = {0u, 0u};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    r.x = __builtin_amdgcn_cvt_pk_u8_f32(c[i], i, r.x);
+    r.y = __builtin_amdgcn_cvt_pk_u8_f32(c[i + 4], i, r.y);
+  }
+  return r;
 }
 __device__ __forceinline__ float ruler_inv(float step) { return __builtin_amdgcn_rcpf(step); }
 
 // The per-token symmetric ("tok") arithmetic: scale = max(absmax / 127, 1e-8) in fp32 (stored
 // as fp16), code = clamp(rint(x / scale), -127, 127) with the fp32 scale.
 __device__ __forceinline__ float sym_scale(float amax) { return fmaxf(__fdiv_rn(amax, 127.0f), 1e-8f); }
-__device__ __forceinline__ uint32_t sym_code(float x, float scale) {
-  const float r = fminf(fmaxf(__builtin_rintf(__fdiv_rn(x, scale)), -127.0f), 127.0f);
-  return (uint32_t)(int32_t)r & 0xffu;
+// (the quotient as x * rcp(scale) unless it is near a half-integer, as ruler_code_f: |x / scale| <= 127.1)
+__device__ __forceinline__ uint32_t sym_code(float x, float scale, float inv) {
+  const float q = __fmul_rn(x, inv);
+  float r = __builtin_rintf(q);
+  if (__builtin_fabsf(q - r) > 0.5f - 0x1p-12f) r = __builtin_rintf(__fdiv_rn(x, scale));
+  return (uint32_t)(int32_t)fminf(fmaxf(r, -127.0f), 127.0f) & 0xffu;
 }
 
 // Max over the 16 lanes of each 16-lane row (DPP only).
@@ -116,9 +140,10 @@ __device__ __forceinline__ uint2 sym_quant8(const float (&v)[8], float& scale) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) amax = fmaxf(amax, __builtin_fabsf(v[j]));
   scale = sym_scale(row16_max(amax));
+  const float inv = ruler_inv(scale);
   uint32_t c[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) c[j] = sym_code(v[j], scale);
+  for (int j = 0; j < 8; ++j) c[j] = sym_code(v[j], scale, inv);
   return uint2{c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24), c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24)};
 }
 

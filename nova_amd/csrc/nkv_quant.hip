@@ -1,12 +1,9 @@
 // Asymmetric int8 quantize / dequantize kernels (token axis and channel axis).
 //
-// Token axis, the format the decode path reads (src/nova/kvquant.py:136-149):
-// one wave quantizes one (slab, group of `gs` tokens, 128-channel chunk).
-// Lanes 0..15 own 8 consecutive channels each (16-byte loads, one 128-element
-// row = 256 contiguous bytes per 16 lanes) and lanes (l >> 4) stride over the
-// group's rows, so every load instruction reads four whole rows. Min/max are
-// reduced across the four row-lanes with cross-lane shuffles; groups of at most
-// 64 tokens stay in registers between the two passes.
+// All of them are bound by memory, and small inputs by the latency of one pass: the quantizer of the
+// token axis is therefore spread over a workgroup per group (below), and the others take tiles of 16 or
+// 64 tokens x 128 channels, 8 channels of one to four rows per thread: 16-byte loads, one 128-element
+// row = 256 contiguous bytes per 16 lanes, every load of a thread issued before the first is used.
 #include "nkv_common.h"
 
 #include <mutex>
@@ -84,14 +81,16 @@ struct Elem8<NKV_F32> {
 
 __device__ __forceinline__ uint2 pack_codes8(const float (&x)[8], const float (&mn)[8],
                                              const float (&st)[8], const float (&inv)[8]) {
-  uint32_t c[8];
+  float c[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) c[i] = ruler_code_rcp(x[i], mn[i], st[i], inv[i]);
-  uint2 r;
-  r.x = c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24);
-  r.y = c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24);
-  return r;
+  for (int i = 0; i < 8; ++i) c[i] = ruler_code_f(x[i], mn[i], st[i], inv[i]);
+  return pack_u8x8(c);
 }
+
+// The dequantizers give a thread one row up to 32768 rows (the latency of more would show: 1600 rows of
+// fp16, token axis, 2.8 against 3.5 us), else four (262144 rows: 17.4 against 20.1 us).
+// fp32 outputs are bound by their stores and take one row at every size (262144 rows, tok: 26.1 against 27.3 us).
+static bool few_rows(int64_t rows, int out_dtype) { return rows <= 32768 || out_dtype == NKV_F32; }
 
 __device__ __forceinline__ uint4 pack_h8(const float (&v)[8]) {
   uint4 r;
@@ -103,6 +102,16 @@ __device__ __forceinline__ uint4 pack_h8(const float (&v)[8]) {
 }
 
 // ---------------------------------------------------------------- token-axis quantize
+//
+// The format the decode path reads (src/nova/kvquant.py:136-149). W waves quantize one (slab, group of
+// `gs` tokens, 128-channel chunk): lanes 0..15 of each 16 own 8 consecutive channels, the 4 W rows of
+// 16 lanes stride over the group's tokens. Groups of at most 4 W R tokens stay in registers between the
+// two passes (R rows per lane), longer ones are read twice. The extremes meet across a wave's four rows
+// by lane swaps and across waves in LDS, where one thread per channel makes the ruler.
+// Bound by memory at size and by one pass's latency below: 8 heads x 32768 fp16 tokens (100 MB moved)
+// in 25 us (4.1 TB/s) against 42 us with one wave per group (128 values per lane, one chain of 2000
+// instructions), 2048 tokens in 5.0 us against 12 us. Groups of 2048 and
+// more: 30 us against 429 us (8 heads x 2048).
 
 struct QuantTokArgs {
   const void* x;
@@ -125,94 +134,143 @@ struct QuantTokArgs {
 
 constexpr int64_t PAGE_GROUP_BYTES = 2 * 64 * 128 + 4 * 128 * 2;  // 17408
 
-constexpr int kQuantWaves = 4;
-constexpr int kCacheRows = 16;  // rows per lane kept in registers (groups of <= 64 tokens)
+template <int W>
+struct QuantTokSmem {
+  float ext[2][W][128];  // per wave: channel minima, maxima
+  float rul[3][128];     // min, step, 1 / step
+};
 
-template <int DT, bool CACHE, bool PAGES = false>
-__global__ __launch_bounds__(64 * kQuantWaves) void quant_token_kernel(QuantTokArgs a) {
-  const int lane = threadIdx.x & 63;
-  const int64_t item = (int64_t)blockIdx.x * kQuantWaves + (threadIdx.x >> 6);
-  if (item >= a.items) return;
-  const int64_t chunk = item % a.nchunks;
-  const int64_t gi = (item / a.nchunks) % a.ngroups;
-  const int64_t r = item / (a.nchunks * a.ngroups);
-  const int cl = lane & 15, rl = lane >> 4;
-  const int64_t ch = chunk * 128 + cl * 8;
-  const bool active = ch < a.dim;
-  const int64_t t0 = gi * a.gs;
-  const int64_t nr = min(a.gs, a.n - t0);
+// W == 1: four independent items (one per wave) in a workgroup of 256 threads, no LDS. R == 0: the
+// group's rows are read in a loop, twice.
+template <int DT, int W, int R, bool PAGES = false>
+__global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void quant_token_kernel(QuantTokArgs a) {
+  __shared__ __attribute__((aligned(16))) QuantTokSmem<W> sm;
+  constexpr int RS = 4 * W;            // rows between a lane's rows
+  constexpr int C = R > 0 ? R : 1;
+  const int lane = threadIdx.x & 63, ti = W == 1 ? lane : (int)threadIdx.x;
+  const int cl = ti & 15, rl = ti >> 4, wave = ti >> 6;
+  const uint32_t items = (uint32_t)a.items, nchunks = (uint32_t)a.nchunks, ngroups = (uint32_t)a.ngroups;
+  const uint32_t first = W == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+  for (uint32_t item = first; item < items; item += W == 1 ? gridDim.x * 4 : gridDim.x) {
+    const uint32_t chunk = item % nchunks, rest = item / nchunks, gi = rest % ngroups, r = rest / ngroups;
+    const int64_t ch = (int64_t)chunk * 128 + cl * 8;
+    const bool active = ch < a.dim;
+    const int64_t t0 = (int64_t)gi * a.gs;
+    const int64_t nr = min(a.gs, a.n - t0);
+    const int64_t base = r * a.x_rs + t0 * a.dim + ch;
 
-  float mn[8], mx[8];
+    float mn[8], mx[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) { mn[j] = __builtin_huge_valf(); mx[j] = -__builtin_huge_valf(); }
-  float cache[CACHE ? kCacheRows : 1][8];
-
-  if (active) {
-    const int64_t base = r * a.x_rs + ch;
-    if (CACHE) {
+    for (int j = 0; j < 8; ++j) { mn[j] = __builtin_huge_valf(); mx[j] = -__builtin_huge_valf(); }
+    float cache[C][8];
+    if (active) {
+      if constexpr (R > 0) {
 #pragma unroll
-      for (int i = 0; i < kCacheRows; ++i) {
-        const int64_t t = rl + 4 * i;
-        if (t < nr) {
-          Elem8<DT>::load(a.x, base + (t0 + t) * a.dim, cache[i]);
+        for (int i = 0; i < R; ++i)  // (a row past the group repeats its last one: the extremes stay)
+          Elem8<DT>::load(a.x, base + min<int64_t>(rl + RS * i, nr - 1) * a.dim, cache[i]);
+#pragma unroll
+        for (int i = 0; i < R; ++i)
 #pragma unroll
           for (int j = 0; j < 8; ++j) { mn[j] = fminf(mn[j], cache[i][j]); mx[j] = fmaxf(mx[j], cache[i][j]); }
+      } else {
+#pragma unroll 4
+        for (int64_t t = rl; t < nr; t += RS) {
+          float v[8];
+          Elem8<DT>::load(a.x, base + t * a.dim, v);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) { mn[j] = fminf(mn[j], v[j]); mx[j] = fmaxf(mx[j], v[j]); }
         }
       }
-    } else {
-      for (int64_t t = rl; t < nr; t += 4) {
-        float v[8];
-        Elem8<DT>::load(a.x, base + (t0 + t) * a.dim, v);
+    }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) { mn[j] = fminf(mn[j], v[j]); mx[j] = fmaxf(mx[j], v[j]); }
+    for (int j = 0; j < 8; ++j) {
+      mn[j] = min4rows(mn[j]);
+      mx[j] = max4rows(mx[j]);
+    }
+    uint8_t* codes = a.codes + r * a.c_rs + t0 * a.dim;  // the group's first code row
+    uint16_t* mins = a.mins + r * a.s_rs + (int64_t)gi * a.dim;
+    uint16_t* steps = a.steps + r * a.s_rs + (int64_t)gi * a.dim;
+    if constexpr (PAGES) {
+      // token t of the group is row t of its page's code block; the rulers follow the code blocks
+      const int32_t page = a.table[a.first_group + gi];
+      if (page < 0 || page >= a.num_pages) continue;  // (the whole item agrees)
+      uint8_t* pg = a.pages + ((int64_t)page * a.rows + r) * PAGE_GROUP_BYTES;
+      codes = pg + a.which * 64 * 128;
+      steps = reinterpret_cast<uint16_t*>(pg + 2 * 64 * 128) + a.which * 2 * 128;
+      mins = steps + 128;
+    }
+    float st[8], inv[8];
+    if constexpr (W == 1) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) { st[j] = ruler_step(mn[j], mx[j]); inv[j] = ruler_inv(st[j]); }
+      if (active && rl == 0) {
+        *reinterpret_cast<uint4*>(mins + ch) = pack_h8(mn);
+        *reinterpret_cast<uint4*>(steps + ch) = pack_h8(st);
+      }
+    } else {
+      if (lane < 16) {
+        float4* lo = reinterpret_cast<float4*>(sm.ext[0][wave] + 8 * cl);
+        float4* hi = reinterpret_cast<float4*>(sm.ext[1][wave] + 8 * cl);
+        lo[0] = make_float4(mn[0], mn[1], mn[2], mn[3]); lo[1] = make_float4(mn[4], mn[5], mn[6], mn[7]);
+        hi[0] = make_float4(mx[0], mx[1], mx[2], mx[3]); hi[1] = make_float4(mx[4], mx[5], mx[6], mx[7]);
+      }
+      __syncthreads();
+      if (ti < 128) {
+        float lo = sm.ext[0][0][ti], hi = sm.ext[1][0][ti];
+#pragma unroll
+        for (int w = 1; w < W; ++w) { lo = fminf(lo, sm.ext[0][w][ti]); hi = fmaxf(hi, sm.ext[1][w][ti]); }
+        const float s = ruler_step(lo, hi);
+        sm.rul[0][ti] = lo;
+        sm.rul[1][ti] = s;
+        sm.rul[2][ti] = ruler_inv(s);
+        const int64_t c = (int64_t)chunk * 128 + ti;
+        if (c < a.dim) {
+          mins[c] = f2h(lo);
+          steps[c] = f2h(s);
+        }
+      }
+      __syncthreads();
+      // (the next item writes ext before its first barrier, and rul after it: no third barrier)
+#pragma unroll
+      for (int j = 0; j < 8; j += 4) {
+        const float4 m4 = *reinterpret_cast<const float4*>(sm.rul[0] + 8 * cl + j);
+        const float4 s4 = *reinterpret_cast<const float4*>(sm.rul[1] + 8 * cl + j);
+        const float4 i4 = *reinterpret_cast<const float4*>(sm.rul[2] + 8 * cl + j);
+        mn[j] = m4.x; mn[j + 1] = m4.y; mn[j + 2] = m4.z; mn[j + 3] = m4.w;
+        st[j] = s4.x; st[j + 1] = s4.y; st[j + 2] = s4.z; st[j + 3] = s4.w;
+        inv[j] = i4.x; inv[j + 1] = i4.y; inv[j + 2] = i4.z; inv[j + 3] = i4.w;
+      }
+    }
+    if (!active) continue;
+    if constexpr (R > 0) {
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const int64_t t = rl + RS * i;
+        const uint2 c8 = pack_codes8(cache[i], mn, st, inv);
+        if (t < nr) *reinterpret_cast<uint2*>(codes + t * a.dim + ch) = c8;
+      }
+    } else {
+#pragma unroll 4
+      for (int64_t t = rl; t < nr; t += RS) {
+        float v[8];
+        Elem8<DT>::load(a.x, base + t * a.dim, v);
+        *reinterpret_cast<uint2*>(codes + t * a.dim + ch) = pack_codes8(v, mn, st, inv);
       }
     }
   }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    mn[j] = fminf(mn[j], shfl_xor(mn[j], 16));
-    mn[j] = fminf(mn[j], shfl_xor(mn[j], 32));
-    mx[j] = fmaxf(mx[j], shfl_xor(mx[j], 16));
-    mx[j] = fmaxf(mx[j], shfl_xor(mx[j], 32));
-  }
-  if (!active) return;
-  float st[8], inv[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) { st[j] = ruler_step(mn[j], mx[j]); inv[j] = ruler_inv(st[j]); }
-  uint8_t* codes = a.codes;
-  uint16_t* mins = a.mins;
-  uint16_t* steps = a.steps;
-  int64_t so = r * a.s_rs + gi * a.dim + ch;
-  int64_t cbase = r * a.c_rs + ch;
-  if constexpr (PAGES) {
-    // token t of the group is row t of its page's code block; the rulers follow the code blocks
-    const int32_t page = a.table[a.first_group + gi];
-    if (page < 0 || page >= a.num_pages) return;
-    uint8_t* pg = a.pages + ((int64_t)page * a.rows + r) * PAGE_GROUP_BYTES;
-    codes = pg + a.which * 64 * 128;
-    cbase = ch - t0 * a.dim;  // (t0 + t) * dim below addresses row t
-    steps = reinterpret_cast<uint16_t*>(pg + 2 * 64 * 128) + a.which * 2 * 128;
-    mins = steps + 128;
-    so = ch;
-  }
-  if (rl == 0) {
-    *reinterpret_cast<uint4*>(mins + so) = pack_h8(mn);
-    *reinterpret_cast<uint4*>(steps + so) = pack_h8(st);
-  }
-  if (CACHE) {
-#pragma unroll
-    for (int i = 0; i < kCacheRows; ++i) {
-      const int64_t t = rl + 4 * i;
-      if (t < nr) *reinterpret_cast<uint2*>(codes + cbase + (t0 + t) * a.dim) = pack_codes8(cache[i], mn, st, inv);
-    }
-  } else {
-    const int64_t base = r * a.x_rs + ch;
-    for (int64_t t = rl; t < nr; t += 4) {
-      float v[8];
-      Elem8<DT>::load(a.x, base + (t0 + t) * a.dim, v);
-      *reinterpret_cast<uint2*>(codes + cbase + (t0 + t) * a.dim) = pack_codes8(v, mn, st, inv);
-    }
-  }
+}
+
+// Waves per item: groups of at most 8 tokens take one wave (2 rows a lane), of at most 64 four (4 rows a
+// lane; the paged kernel's groups are always 64), longer ones a workgroup of 16 that reads them twice.
+template <int DT>
+static void launch_quant_token(const QuantTokArgs& a, hipStream_t s) {
+  const int64_t most = 1 << 20;  // workgroups; more items are taken in turns
+  if (a.gs <= 8)
+    hipLaunchKernelGGL((quant_token_kernel<DT, 1, 2>), dim3((unsigned)std::min(cdiv(a.items, 4), most)), dim3(256), 0, s, a);
+  else if (a.gs <= 64)
+    hipLaunchKernelGGL((quant_token_kernel<DT, 4, 4>), dim3((unsigned)std::min(a.items, most)), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((quant_token_kernel<DT, 16, 0>), dim3((unsigned)std::min(a.items, most)), dim3(1024), 0, s, a);
 }
 
 // ---------------------------------------------------------------- channel-axis quantize
@@ -259,6 +317,50 @@ __global__ __launch_bounds__(256) void quant_channel_kernel(QuantChanArgs a) {
   a.steps[so] = f2h(st);
 }
 
+// The same for groups of 8, 16, 32, 64 or 128 channels and 16-byte rows: 16 tokens x 128 channels per
+// workgroup, 8 channels of one token per lane, a group's extremes over its gc / 8 lanes by lane swaps.
+// 8 heads x 3001 bf16 tokens, groups of 32 / 64: 4.8 / 4.8 us against 22 / 33 us with a thread per group
+// (2-byte loads, one byte per store); 32768 fp16 tokens, groups of 64: 24 against 1390 us. Four tokens per
+// thread were slower at every size (2048 tokens: 5.4 against 4.0 us, 32768: 24.2 against 23.7 us).
+template <int DT, int L>  // L: lanes per group
+__global__ __launch_bounds__(256) void quant_channel8_kernel(QuantChanArgs a) {
+  const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4;
+  const uint32_t nchunks = (uint32_t)((a.dim + 127) / 128), nblocks = (uint32_t)((a.n + 15) / 16);
+  const uint32_t chunk = blockIdx.x % nchunks, rest = blockIdx.x / nchunks, tb = rest % nblocks, r = rest / nblocks;
+  const int64_t ch = (int64_t)chunk * 128 + cl * 8, t = (int64_t)tb * 16 + rl;
+  if (ch >= a.dim || t >= a.n) return;  // (whole groups: dim is a multiple of gc)
+  float v[8];
+  Elem8<DT>::load(a.x, r * a.x_rs + t * a.dim + ch, v);
+  float lo = __builtin_huge_valf(), hi = -__builtin_huge_valf();
+#pragma unroll
+  for (int j = 0; j < 8; ++j) { lo = fminf(lo, v[j]); hi = fmaxf(hi, v[j]); }
+#pragma unroll
+  for (int o = 1; o < L; o *= 2) { lo = fminf(lo, shfl_xor(lo, o)); hi = fmaxf(hi, shfl_xor(hi, o)); }
+  const float st = ruler_step(lo, hi), inv = ruler_inv(st);
+  float c[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) c[j] = ruler_code_f(v[j], lo, st, inv);
+  *reinterpret_cast<uint2*>(a.codes + r * a.c_rs + t * a.dim + ch) = pack_u8x8(c);
+  if (cl % L == 0) {
+    const int64_t so = r * a.s_rs + t * a.ngc + ch / a.gc;
+    a.mins[so] = f2h(lo);
+    a.steps[so] = f2h(st);
+  }
+}
+
+template <int DT>
+static void launch_quant_channel(const QuantChanArgs& a, bool wide, hipStream_t s) {
+  const int64_t tiles = a.rows * cdiv(a.n, 16) * cdiv(a.dim, 128);
+  const dim3 grid((unsigned)tiles), block(256);
+  if (tiles >= (1 << 24)) wide = false;  // (a grid of at most 2^32 threads)
+  if (wide && a.gc == 8) hipLaunchKernelGGL((quant_channel8_kernel<DT, 1>), grid, block, 0, s, a);
+  else if (wide && a.gc == 16) hipLaunchKernelGGL((quant_channel8_kernel<DT, 2>), grid, block, 0, s, a);
+  else if (wide && a.gc == 32) hipLaunchKernelGGL((quant_channel8_kernel<DT, 4>), grid, block, 0, s, a);
+  else if (wide && a.gc == 64) hipLaunchKernelGGL((quant_channel8_kernel<DT, 8>), grid, block, 0, s, a);
+  else if (wide && a.gc == 128) hipLaunchKernelGGL((quant_channel8_kernel<DT, 16>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL(quant_channel_kernel<DT>, dim3((unsigned)cdiv(a.items, 256)), block, 0, s, a);
+}
+
 // ---------------------------------------------------------------- dequantize
 
 struct DequantArgs {
@@ -270,7 +372,8 @@ struct DequantArgs {
   int64_t rows, n, dim, group, axis;
   void* out;
   int64_t o_rs;
-  int64_t items;  // rows * n * dim / 8
+  int64_t items;  // tiles: rows * ceil(n / rows of a tile) * ceil(dim / 128)
+  int vec;        // token axis: the rulers of 8 channels are 16-byte aligned
 };
 
 template <int OT>
@@ -291,37 +394,81 @@ __device__ __forceinline__ void store8(void* out, int64_t off, const float (&v)[
   }
 }
 
-template <int OT>
+// 16 R tokens x 128 channels per workgroup, R rows of 8 channels per thread. A lane's rulers are loaded
+// once per group it meets: token axis 8 steps and 8 mins (two 16-byte loads when `vec`), channel axis one
+// pair for its 8 channels when the group is a multiple of 8, else one per channel. 8 heads x 3001 /
+// 32768 fp16 tokens, groups of 64: token axis 4.6 / 17.4 us against 8.7 / 64 us, channel axis 4.6 / 20 us
+// against 7.9 / 49 us with a ruler load per value and 64-bit divisions.
+template <int OT, int R>
 __global__ __launch_bounds__(256) void dequant_kernel(DequantArgs a) {
-  const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (item >= a.items) return;
-  const int64_t per_row = a.dim / 8;
-  const int64_t c8 = (item % per_row) * 8;
-  const int64_t t = (item / per_row) % a.n;
-  const int64_t r = item / (per_row * a.n);
-  const uint2 cw = *reinterpret_cast<const uint2*>(a.codes + r * a.c_rs + t * a.dim + c8);
-  float v[8];
+  const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4;
+  const uint32_t nchunks = (uint32_t)((a.dim + 127) / 128), nblocks = (uint32_t)((a.n + 16 * R - 1) / (16 * R));
+  const bool token = a.axis == NKV_AXIS_TOKEN;
+  for (uint32_t tile = blockIdx.x; tile < (uint32_t)a.items; tile += gridDim.x) {
+    const uint32_t chunk = tile % nchunks, rest = tile / nchunks, tb = rest % nblocks, r = rest / nblocks;
+    const int64_t ch = (int64_t)chunk * 128 + cl * 8;
+    if (ch >= a.dim) continue;
+    const int64_t t0 = (int64_t)tb * (16 * R) + rl;
+    uint2 cw[R];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const uint32_t code = ((j < 4 ? cw.x : cw.y) >> (8 * (j & 3))) & 0xffu;
-    int64_t so;
-    if (a.axis == NKV_AXIS_TOKEN) {
-      so = r * a.s_rs + (t / a.group) * a.dim + c8 + j;
-    } else {
-      const int64_t ngc = a.dim / a.group;
-      so = r * a.s_rs + t * ngc + (c8 + j) / a.group;
+    for (int i = 0; i < R; ++i)
+      cw[i] = *reinterpret_cast<const uint2*>(a.codes + r * a.c_rs + min(t0 + 16 * i, a.n - 1) * a.dim + ch);
+    float st[8], mn[8];
+    int64_t have = -1;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int64_t t = t0 + 16 * i;
+      if (t >= a.n) break;
+      if (token) {
+        // (32-bit: the tile count bounds n)
+        const int64_t gi = (uint32_t)t / (uint32_t)a.group;
+        if (gi != have) {
+          have = gi;
+          const int64_t so = r * a.s_rs + gi * a.dim + ch;
+          if (a.vec) {
+            Elem8<NKV_F16>::load(a.steps, so, st);
+            Elem8<NKV_F16>::load(a.mins, so, mn);
+          } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) { st[j] = h2f(a.steps[so + j]); mn[j] = h2f(a.mins[so + j]); }
+          }
+        }
+      } else {
+        const uint32_t ngc = (uint32_t)(a.dim / a.group);
+        const int64_t so = r * a.s_rs + t * ngc;
+        if (a.group % 8 == 0) {
+          const uint32_t gc = (uint32_t)ch / (uint32_t)a.group;
+          const float s1 = h2f(a.steps[so + gc]), m1 = h2f(a.mins[so + gc]);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) { st[j] = s1; mn[j] = m1; }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const uint32_t gc = (uint32_t)(ch + j) / (uint32_t)a.group;
+            st[j] = h2f(a.steps[so + gc]);
+            mn[j] = h2f(a.mins[so + gc]);
+          }
+        }
+      }
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t code = ((j < 4 ? cw[i].x : cw[i].y) >> (8 * (j & 3))) & 0xffu;
+        // the product of an 8-bit code and an fp16 step is exact in fp32; one rounding in the add
+        v[j] = __fadd_rn(__fmul_rn((float)code, st[j]), mn[j]);
+      }
+      store8<OT>(a.out, r * a.o_rs + t * a.dim + ch, v);
     }
-    // the product of an 8-bit code and an fp16 step is exact in fp32; one rounding in the add
-    v[j] = __fadd_rn(__fmul_rn((float)code, h2f(a.steps[so])), h2f(a.mins[so]));
   }
-  store8<OT>(a.out, r * a.o_rs + t * a.dim + c8, v);
 }
 
 // ---------------------------------------------------------------- per-token symmetric ("tok")
 
 // One (slab, token) row of 128 values per 16-lane row: lane l & 15 quantizes values
-// 8 (l & 15) .. + 7 (16-byte loads, 8-byte code stores); a wave covers 4 tokens, a
-// 256-thread workgroup 16. The absmax is reduced with DPP within the 16-lane row.
+// 8 (l & 15) .. + 7 (16-byte loads, 8-byte code stores); a workgroup takes 16 tokens of one slab. The
+// absmax is reduced with DPP within the 16-lane row. 8 heads x 8191 / 32768 fp16 tokens: 7.3 / 19.8 us against
+// 9.7 / 29 us with an IEEE division per value and 64-bit divisions per thread (four tokens per thread:
+// 8.3 / 20.5 us).
 struct QuantSymArgs {
   const void* x;
   int64_t x_rs;
@@ -330,7 +477,7 @@ struct QuantSymArgs {
   int64_t c_rs;
   uint16_t* scales;
   int64_t s_rs;
-  int64_t items;  // rows * n
+  int64_t items;  // tiles: rows * ceil(n / rows of a tile)
   // page destination (paged cache): token t of slab r is token first_token + t of a sequence,
   // stored in page table[(first_token + t) / 64], KV head r, row (first_token + t) % 64 of
   // tensor `which` (0 K, 1 V) of the page layout [K codes 64 x 128 | V codes | K scales 64 |
@@ -345,27 +492,29 @@ constexpr int64_t PAGE_TOK_BYTES = 2 * 64 * 128 + 2 * 64 * 2;  // 16640
 
 template <int DT, bool PAGES = false>
 __global__ __launch_bounds__(256) void quant_sym_kernel(QuantSymArgs a) {
-  const int64_t item = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-  const bool on = item < a.items;  // whole 16-lane rows agree
-  const int c8 = (threadIdx.x & 15) * 8;
-  const int64_t r = on ? item / a.n : 0, t = on ? item % a.n : 0;
-  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (on) Elem8<DT>::load(a.x, r * a.x_rs + t * 128 + c8, v);
-  float scale;
-  const uint2 cw = sym_quant8(v, scale);
-  if (!on) return;
-  uint8_t* code_row = a.codes + r * a.c_rs + t * 128;
-  uint16_t* scale_at = a.scales + r * a.s_rs + t;
-  if constexpr (PAGES) {
-    const int64_t tok = a.first_token + t;
-    const int32_t page = a.table[tok / 64];
-    if (page < 0 || page >= a.num_pages) return;
-    uint8_t* pg = a.pages + ((int64_t)page * a.rows + r) * PAGE_TOK_BYTES;
-    code_row = pg + a.which * 64 * 128 + (tok % 64) * 128;
-    scale_at = reinterpret_cast<uint16_t*>(pg + 2 * 64 * 128) + a.which * 64 + tok % 64;
+  const int c8 = (threadIdx.x & 15) * 8, rl = threadIdx.x >> 4;
+  const uint32_t nblocks = (uint32_t)((a.n + 15) / 16);
+  for (uint32_t tile = blockIdx.x; tile < (uint32_t)a.items; tile += gridDim.x) {
+    const uint32_t tb = tile % nblocks, r = tile / nblocks;
+    const int64_t t = (int64_t)tb * 16 + rl;
+    if (t >= a.n) continue;  // (whole 16-lane rows agree)
+    float v[8];
+    Elem8<DT>::load(a.x, r * a.x_rs + t * 128 + c8, v);
+    float scale;
+    const uint2 cw = sym_quant8(v, scale);
+    uint8_t* code_row = a.codes + r * a.c_rs + t * 128;
+    uint16_t* scale_at = a.scales + r * a.s_rs + t;
+    if constexpr (PAGES) {
+      const int64_t tok = a.first_token + t;
+      const int32_t page = a.table[tok / 64];
+      if (page < 0 || page >= a.num_pages) continue;
+      uint8_t* pg = a.pages + ((int64_t)page * a.rows + r) * PAGE_TOK_BYTES;
+      code_row = pg + a.which * 64 * 128 + (tok % 64) * 128;
+      scale_at = reinterpret_cast<uint16_t*>(pg + 2 * 64 * 128) + a.which * 64 + tok % 64;
+    }
+    *reinterpret_cast<uint2*>(code_row + c8) = cw;
+    if (c8 == 0) *scale_at = f2h(scale);
   }
-  *reinterpret_cast<uint2*>(code_row + c8) = cw;
-  if (c8 == 0) *scale_at = f2h(scale);
 }
 
 struct DequantSymArgs {
@@ -376,24 +525,37 @@ struct DequantSymArgs {
   int64_t rows, n;
   void* out;
   int64_t o_rs;
-  int64_t items;  // rows * n * 16
+  int64_t items;  // tiles: rows * ceil(n / rows of a tile)
 };
 
-template <int OT>
+template <int OT, int R>
 __global__ __launch_bounds__(256) void dequant_sym_kernel(DequantSymArgs a) {
-  const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (item >= a.items) return;
-  const int c8 = (int)(item % 16) * 8;
-  const int64_t t = (item / 16) % a.n, r = item / (16 * a.n);
-  const uint2 cw = *reinterpret_cast<const uint2*>(a.codes + r * a.c_rs + t * 128 + c8);
-  const float sc = h2f(a.scales[r * a.s_rs + t]);
-  float v[8];
+  const int c8 = (threadIdx.x & 15) * 8, rl = threadIdx.x >> 4;
+  const uint32_t nblocks = (uint32_t)((a.n + 16 * R - 1) / (16 * R));
+  for (uint32_t tile = blockIdx.x; tile < (uint32_t)a.items; tile += gridDim.x) {
+    const uint32_t tb = tile % nblocks, r = tile / nblocks;
+    const int64_t t0 = (int64_t)tb * (16 * R) + rl;
+    uint2 cw[R];
+    float sc[R];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int code = (int)(int8_t)(((j < 4 ? cw.x : cw.y) >> (8 * (j & 3))) & 0xffu);
-    v[j] = __fmul_rn((float)code, sc);  // exact in fp32; rounded once by the store
+    for (int i = 0; i < R; ++i) {
+      const int64_t t = min(t0 + 16 * i, a.n - 1);
+      cw[i] = *reinterpret_cast<const uint2*>(a.codes + r * a.c_rs + t * 128 + c8);
+      sc[i] = h2f(a.scales[r * a.s_rs + t]);
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int64_t t = t0 + 16 * i;
+      if (t >= a.n) break;
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int code = (int)(int8_t)(((j < 4 ? cw[i].x : cw[i].y) >> (8 * (j & 3))) & 0xffu);
+        v[j] = __fmul_rn((float)code, sc[i]);  // exact in fp32; rounded once by the store
+      }
+      store8<OT>(a.out, r * a.o_rs + t * 128 + c8, v);
+    }
   }
-  store8<OT>(a.out, r * a.o_rs + t * 128 + c8, v);
 }
 
 // ---------------------------------------------------------------- copy (traffic calibration)
@@ -425,6 +587,12 @@ __global__ __launch_bounds__(256) void read_bw_kernel(const uint4* __restrict__ 
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = x;
   __syncthreads();
   if (threadIdx.x == 0) sink[blockIdx.x] = part[0] ^ part[1] ^ part[2] ^ part[3];
+}
+
+// One of a kernel's two row counts per thread.
+template <class K, class A>
+static void launch_rows(K one, K four, bool few, dim3 grid, hipStream_t s, const A& a) {
+  hipLaunchKernelGGL(few ? one : four, grid, dim3(256), 0, s, a);
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -459,27 +627,29 @@ extern "C" int nkv_quantize_int8(const void* x, int x_dtype, int64_t x_row_strid
     QuantTokArgs a{x, x_row_stride, rows, n, dim, gs, cdiv(n, gs), cdiv(dim, 128), codes,
                    codes_row_stride, mins, steps, scale_row_stride, 0};
     a.items = rows * a.ngroups * a.nchunks;
-    const dim3 grid((unsigned)cdiv(a.items, kQuantWaves)), block(64 * kQuantWaves);
-    const bool cache = gs <= 4 * kCacheRows;
-#define NKV_QT(DT)                                                                        \
-  if (cache) hipLaunchKernelGGL((quant_token_kernel<DT, true>), grid, block, 0, s, a);    \
-  else hipLaunchKernelGGL((quant_token_kernel<DT, false>), grid, block, 0, s, a);
-    if (x_dtype == NKV_F16) { NKV_QT(NKV_F16) }
-    else if (x_dtype == NKV_BF16) { NKV_QT(NKV_BF16) }
-    else { NKV_QT(NKV_F32) }
-#undef NKV_QT
+    if (a.items >= (int64_t(1) << 32)) return fail(NKV_ERR_UNSUPPORTED, "quantize: %lld groups", (long long)a.items);
+    if (x_dtype == NKV_F16) launch_quant_token<NKV_F16>(a, s);
+    else if (x_dtype == NKV_BF16) launch_quant_token<NKV_BF16>(a, s);
+    else launch_quant_token<NKV_F32>(a, s);
     return check_launch("quantize_int8(token)");
   }
   if (axis == NKV_AXIS_CHANNEL) {
     const int64_t gc = group ? group : dim;
     if (dim % gc) return fail(NKV_ERR_INVALID, "head_dim %lld is not divisible by group_size %lld", (long long)dim, (long long)gc);
+    // slabs that follow one another are one slab
+    if (x_row_stride == n * dim && codes_row_stride == n * dim && scale_row_stride == n * (dim / gc)) {
+      n *= rows;
+      rows = 1;
+    }
     QuantChanArgs a{x, x_row_stride, rows, n, dim, gc, dim / gc, codes, codes_row_stride,
                     mins, steps, scale_row_stride, 0};
     a.items = rows * n * a.ngc;
-    const dim3 grid((unsigned)cdiv(a.items, 256)), block(256);
-    if (x_dtype == NKV_F16) hipLaunchKernelGGL(quant_channel_kernel<NKV_F16>, grid, block, 0, s, a);
-    else if (x_dtype == NKV_BF16) hipLaunchKernelGGL(quant_channel_kernel<NKV_BF16>, grid, block, 0, s, a);
-    else hipLaunchKernelGGL(quant_channel_kernel<NKV_F32>, grid, block, 0, s, a);
+    const int esz = x_dtype == NKV_F32 ? 4 : 2;
+    const bool wide = dim % 8 == 0 && aligned16(x) && (x_row_stride * esz) % 16 == 0 &&
+                      (reinterpret_cast<uintptr_t>(codes) & 7u) == 0 && codes_row_stride % 8 == 0;
+    if (x_dtype == NKV_F16) launch_quant_channel<NKV_F16>(a, wide, s);
+    else if (x_dtype == NKV_BF16) launch_quant_channel<NKV_BF16>(a, wide, s);
+    else launch_quant_channel<NKV_F32>(a, wide, s);
     return check_launch("quantize_int8(channel)");
   }
   return fail(NKV_ERR_INVALID, "axis must be channel (0) or token (1), got %d", axis);
@@ -503,11 +673,11 @@ extern "C" int nkv_paged_quantize_t64(const void* x, int x_dtype, int64_t x_head
   QuantTokArgs a{x, x_head_stride, hkv, n, 128, 64, n / 64, 1, nullptr, 0, nullptr, nullptr, 0, 0,
                  pages, table_row, first_group, num_pages, which};
   a.items = hkv * a.ngroups;
-  const dim3 grid((unsigned)cdiv(a.items, kQuantWaves)), block(64 * kQuantWaves);
+  const dim3 grid((unsigned)std::min<int64_t>(a.items, 1 << 20)), block(256);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (x_dtype == NKV_F16) hipLaunchKernelGGL((quant_token_kernel<NKV_F16, true, true>), grid, block, 0, s, a);
-  else if (x_dtype == NKV_BF16) hipLaunchKernelGGL((quant_token_kernel<NKV_BF16, true, true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((quant_token_kernel<NKV_F32, true, true>), grid, block, 0, s, a);
+  if (x_dtype == NKV_F16) hipLaunchKernelGGL((quant_token_kernel<NKV_F16, 4, 4, true>), grid, block, 0, s, a);
+  else if (x_dtype == NKV_BF16) hipLaunchKernelGGL((quant_token_kernel<NKV_BF16, 4, 4, true>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((quant_token_kernel<NKV_F32, 4, 4, true>), grid, block, 0, s, a);
   return check_launch("paged_quantize_t64");
 }
 
@@ -524,19 +694,30 @@ extern "C" int nkv_dequantize_int8(const uint8_t* codes, int64_t codes_row_strid
   if (rows < 0 || n < 0 || dim <= 0 || group < 0) return fail(NKV_ERR_INVALID, "dequantize: bad sizes");
   if (rows == 0 || n == 0) return NKV_OK;
   if (dim % 8) return fail(NKV_ERR_UNSUPPORTED, "dequantize: head_dim %lld is not a multiple of 8", (long long)dim);
-  const int64_t g = group ? group : (axis == NKV_AXIS_TOKEN ? n : dim);
+  int64_t g = group ? group : (axis == NKV_AXIS_TOKEN ? n : dim);
   if (axis == NKV_AXIS_CHANNEL && dim % g) return fail(NKV_ERR_INVALID, "head_dim is not divisible by group_size");
   const int esz = out_dtype == NKV_F32 ? 4 : 2;
   if ((reinterpret_cast<uintptr_t>(codes) & 7u) || codes_row_stride % 8 || !aligned16(out) ||
       (out_row_stride * esz) % 16)
     return fail(NKV_ERR_UNSUPPORTED, "dequantize: buffers or row strides are not aligned");
+  if (axis == NKV_AXIS_TOKEN) g = std::min(g, n);  // (a longer group is the whole slab)
+  // slabs that follow one another, each of whole groups, are one slab
+  const int64_t rulers = axis == NKV_AXIS_CHANNEL ? n * (dim / g) : n % g ? -1 : n / g * dim;
+  if (codes_row_stride == n * dim && out_row_stride == n * dim && scale_row_stride == rulers) {
+    n *= rows;
+    rows = 1;
+  }
   DequantArgs a{codes, codes_row_stride, mins, steps, scale_row_stride, rows, n, dim, g, axis,
-                out, out_row_stride, rows * n * (dim / 8)};
+                out, out_row_stride, rows * cdiv(n, few_rows(rows * n, out_dtype) ? 16 : 64) * cdiv(dim, 128),
+                aligned16(mins) && aligned16(steps) && scale_row_stride % 8 == 0};
+  if (a.items >= (int64_t(1) << 31) || n >= (int64_t(1) << 32) || dim >= (int64_t(1) << 32))
+    return fail(NKV_ERR_UNSUPPORTED, "dequantize: rows=%lld n=%lld dim=%lld", (long long)rows, (long long)n, (long long)dim);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)cdiv(a.items, 256)), block(256);
-  if (out_dtype == NKV_F16) hipLaunchKernelGGL(dequant_kernel<NKV_F16>, grid, block, 0, s, a);
-  else if (out_dtype == NKV_BF16) hipLaunchKernelGGL(dequant_kernel<NKV_BF16>, grid, block, 0, s, a);
-  else hipLaunchKernelGGL(dequant_kernel<NKV_F32>, grid, block, 0, s, a);
+  const bool few = few_rows(rows * n, out_dtype);
+  const dim3 grid((unsigned)std::min<int64_t>(a.items, 1 << 20));
+  if (out_dtype == NKV_F16) launch_rows(dequant_kernel<NKV_F16, 1>, dequant_kernel<NKV_F16, 4>, few, grid, s, a);
+  else if (out_dtype == NKV_BF16) launch_rows(dequant_kernel<NKV_BF16, 1>, dequant_kernel<NKV_BF16, 4>, few, grid, s, a);
+  else launch_rows(dequant_kernel<NKV_F32, 1>, dequant_kernel<NKV_F32, 4>, few, grid, s, a);
   return check_launch("dequantize_int8");
 }
 
@@ -555,13 +736,17 @@ extern "C" int nkv_quantize_tok(const void* x, int x_dtype, int64_t x_row_stride
   if (!x || !codes || !scales || !aligned16(x) || (reinterpret_cast<uintptr_t>(codes) & 7u) ||
       (reinterpret_cast<uintptr_t>(scales) & 1u) || (x_row_stride * esz) % 16 || codes_row_stride % 8)
     return fail(NKV_ERR_UNSUPPORTED, "quantize_tok: buffers or row strides are not aligned");
+  if (x_row_stride == n * dim && codes_row_stride == n * dim && scale_row_stride == n) {  // one slab
+    n *= rows;
+    rows = 1;
+  }
   QuantSymArgs a{x, x_row_stride, rows, n, reinterpret_cast<uint8_t*>(codes), codes_row_stride, scales,
-                 scale_row_stride, rows * n};
+                 scale_row_stride, rows * cdiv(n, 16)};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)cdiv(a.items, 16)), block(256);
-  if (x_dtype == NKV_F16) hipLaunchKernelGGL(quant_sym_kernel<NKV_F16>, grid, block, 0, s, a);
-  else if (x_dtype == NKV_BF16) hipLaunchKernelGGL(quant_sym_kernel<NKV_BF16>, grid, block, 0, s, a);
-  else hipLaunchKernelGGL(quant_sym_kernel<NKV_F32>, grid, block, 0, s, a);
+  const dim3 grid((unsigned)std::min<int64_t>(a.items, 1 << 22)), block(256);
+  if (x_dtype == NKV_F16) hipLaunchKernelGGL((quant_sym_kernel<NKV_F16>), grid, block, 0, s, a);
+  else if (x_dtype == NKV_BF16) hipLaunchKernelGGL((quant_sym_kernel<NKV_BF16>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((quant_sym_kernel<NKV_F32>), grid, block, 0, s, a);
   return check_launch("quantize_tok");
 }
 
@@ -579,10 +764,10 @@ extern "C" int nkv_paged_quantize_tok(const void* x, int x_dtype, int64_t x_head
   const int esz = x_dtype == NKV_F32 ? 4 : 2;
   if (!aligned16(x) || !aligned16(pages) || (x_head_stride * esz) % 16 || x_head_stride < n * 128)
     return fail(NKV_ERR_UNSUPPORTED, "paged_quantize_tok: x must be 16-byte aligned with a head stride >= n * 128");
-  QuantSymArgs a{x, x_head_stride, hkv, n, nullptr, 0, nullptr, 0, hkv * n, pages, table_row, first_token,
+  QuantSymArgs a{x, x_head_stride, hkv, n, nullptr, 0, nullptr, 0, hkv * cdiv(n, 16), pages, table_row, first_token,
                  num_pages, which};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)cdiv(a.items, 16)), block(256);
+  const dim3 grid((unsigned)std::min<int64_t>(a.items, 1 << 22)), block(256);
   if (x_dtype == NKV_F16) hipLaunchKernelGGL((quant_sym_kernel<NKV_F16, true>), grid, block, 0, s, a);
   else if (x_dtype == NKV_BF16) hipLaunchKernelGGL((quant_sym_kernel<NKV_BF16, true>), grid, block, 0, s, a);
   else hipLaunchKernelGGL((quant_sym_kernel<NKV_F32, true>), grid, block, 0, s, a);
@@ -602,13 +787,18 @@ extern "C" int nkv_dequantize_tok(const int8_t* codes, int64_t codes_row_stride,
   if (!codes || !scales || !out || (reinterpret_cast<uintptr_t>(codes) & 7u) || codes_row_stride % 8 ||
       !aligned16(out) || (out_row_stride * esz) % 16)
     return fail(NKV_ERR_UNSUPPORTED, "dequantize_tok: buffers or row strides are not aligned");
+  if (codes_row_stride == n * dim && out_row_stride == n * dim && scale_row_stride == n) {  // one slab
+    n *= rows;
+    rows = 1;
+  }
+  const bool few = few_rows(rows * n, out_dtype);
   DequantSymArgs a{reinterpret_cast<const uint8_t*>(codes), codes_row_stride, scales, scale_row_stride, rows, n,
-                   out, out_row_stride, rows * n * 16};
+                   out, out_row_stride, rows * cdiv(n, few ? 16 : 64)};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)cdiv(a.items, 256)), block(256);
-  if (out_dtype == NKV_F16) hipLaunchKernelGGL(dequant_sym_kernel<NKV_F16>, grid, block, 0, s, a);
-  else if (out_dtype == NKV_BF16) hipLaunchKernelGGL(dequant_sym_kernel<NKV_BF16>, grid, block, 0, s, a);
-  else hipLaunchKernelGGL(dequant_sym_kernel<NKV_F32>, grid, block, 0, s, a);
+  const dim3 grid((unsigned)std::min<int64_t>(a.items, 1 << 20));
+  if (out_dtype == NKV_F16) launch_rows(dequant_sym_kernel<NKV_F16, 1>, dequant_sym_kernel<NKV_F16, 4>, few, grid, s, a);
+  else if (out_dtype == NKV_BF16) launch_rows(dequant_sym_kernel<NKV_BF16, 1>, dequant_sym_kernel<NKV_BF16, 4>, few, grid, s, a);
+  else launch_rows(dequant_sym_kernel<NKV_F32, 1>, dequant_sym_kernel<NKV_F32, 4>, few, grid, s, a);
   return check_launch("dequantize_tok");
 }
 

@@ -133,3 +133,32 @@ def test_full_size_prefill_quantize_properties():
     assert _eq16(mn, rm) and _eq16(st, rs)
     qg = q.view(1, 8, 512, 64, 128)
     assert int(qg.amin(dim=3).max()) == 0 and int(qg.amax(dim=3).min()) == 255
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("axis,group,n,dim", [
+    ("token", 4, 9, 128), ("token", 8, 17, 64), ("token", 9, 30, 136), ("token", 64, 65, 200),
+    ("token", 0, 65, 128), ("token", 100, 333, 128), ("token", 0, 1500, 8),
+    ("channel", 8, 3, 128), ("channel", 16, 65, 48), ("channel", 32, 129, 160), ("channel", 64, 64, 64),
+    ("channel", 128, 1, 128), ("channel", 0, 70, 128), ("channel", 24, 66, 72), ("channel", 4, 5, 8),
+])
+def test_every_quantizer_route_matches_oracle(axis, group, n, dim, dtype):
+    """Each split of the quantizers and the dequantizer at its edges (groups of one wave, four and
+    sixteen, tails of tokens and channels, channel groups of lanes and the general ones): whole
+    numbers, so the same bits."""
+    from nova_amd.kvquant import dequantize_int8, quantize_int8
+
+    print(f"case {axis} group={group} n={n} dim={dim} {dtype}", flush=True)
+    x = (torch.randn(2, 3, n, dim, generator=torch.Generator().manual_seed(n + dim)) * 2).to(dtype)
+    x[..., 3] *= 8
+    if axis == "token":
+        rq, rm, rs = okq.quantize_int8_token(x.float().numpy(), group)
+        want = okq.dequantize_int8_token(rq, rm, rs, group)
+    else:
+        rq, rm, rs = okq.quantize_int8_channel(x.float().numpy(), group)
+        want = okq.dequantize_int8_channel(rq, rm, rs, group)
+    for src in (x.cuda(), torch.zeros(2, 3, n + 5, dim, dtype=dtype).cuda()[:, :, :n].copy_(x)):
+        q, mn, st = quantize_int8(src, group, axis)
+        assert np.array_equal(npy(q), rq)
+        assert _eq16(mn, rm) and _eq16(st, rs)
+    assert _eq16(dequantize_int8(q, mn, st, group, axis), want)
