@@ -620,6 +620,29 @@ int nkv_prefill_attn_hist_t64(const uint16_t* q, int64_t m, const uint16_t* k16,
                               uint16_t* out, void* workspace, int64_t workspace_bytes, int64_t splits,
                               void* stream);
 
+/* The same with query head i's token j at q + i * q_head_stride + j * q_token_stride (multiples of 8),
+ * so that a projection's token-major output is read where it is; out [hq][m][128]. */
+int nkv_prefill_attn_strided_t64(const uint16_t* q, int64_t q_token_stride, int64_t q_head_stride, int64_t m,
+                                 const uint16_t* k16, const uint16_t* v16, int64_t m_kv, int64_t kv_head_stride,
+                                 const uint8_t* kq, const uint16_t* kmn, const uint16_t* kst, const uint8_t* vq,
+                                 const uint16_t* vmn, const uint16_t* vst, int64_t capacity, int64_t used,
+                                 int64_t hq, int64_t hkv, int64_t head_dim, uint16_t* out, void* workspace,
+                                 int64_t workspace_bytes, int64_t splits, void* stream);
+
+/*
+ * A streamed prefill chunk lands in the cache (KVInt8Cache.update + the bulk quantize of
+ * finish_prefill, src/nova/kvattn.py:668-783, for one chunk): n tokens of hkv heads at positions
+ * start .. start + n - 1 (start a multiple of 64), head h's token j at k + h * k_head_stride +
+ * j * k_token_stride (v likewise; strides multiples of 8). Writes the contiguous fp16 copies k16 /
+ * v16 [hkv][n][128], codes and rulers of the whole groups, and the ring slots (position % 64) of
+ * the newest min(n, 64) tokens. One launch.
+ */
+int nkv_prefill_land_t64(const uint16_t* k, const uint16_t* v, int64_t k_token_stride, int64_t k_head_stride,
+                         int64_t v_token_stride, int64_t v_head_stride, int64_t n, int64_t start, int64_t hkv,
+                         int64_t head_dim, int64_t capacity, uint16_t* k16, uint16_t* v16, uint8_t* kq,
+                         uint16_t* kmn, uint16_t* kst, uint8_t* vq, uint16_t* vmn, uint16_t* vst, uint16_t* tail_k,
+                         uint16_t* tail_v, void* stream);
+
 /*
  * Plain device copy (16-byte vector loads and stores). Used to calibrate the
  * HBM traffic counters (FETCH_SIZE / WRITE_SIZE) against a known byte count;

@@ -91,6 +91,9 @@ SIGNATURES = {
     "nkv_prefill_attn_t64": (c_int, [P, P, P, I64, P, P, P, P, P, P, I64, I64, I64, I64, I64, P, P, I64, I64, P]),
     "nkv_prefill_attn_hist_t64": (c_int, [P, I64, P, P, I64, I64, P, P, P, P, P, P, I64, I64, I64, I64, I64, P, P,
                                           I64, I64, P]),
+    "nkv_prefill_attn_strided_t64": (c_int, [P, I64, I64, I64, P, P, I64, I64, P, P, P, P, P, P, I64, I64, I64, I64, I64,
+                                             P, P, I64, I64, P]),
+    "nkv_prefill_land_t64": (c_int, [P, P, I64, I64, I64, I64, I64, I64, I64, I64, I64, P, P, P, P, P, P, P, P, P, P, P]),
     "nkv_copy_bytes": (c_int, [P, P, I64, P]),
     "nkv_read_bw": (c_int, [P, I64, P, I64, P]),
     "nkv_clock_probe": (c_int, [P, I64, I64, P]),

@@ -3308,7 +3308,8 @@ struct PrefillCut {
 };
 
 struct PrefillArgs {
-  const uint16_t* q;   // [hq][M][D]
+  const uint16_t* q;   // query head i's token j at q + i * q_hs + j * q_ts
+  int64_t q_ts, q_hs;
   const uint16_t* kc;  // fp16 K: head h's token j at kc + h * kc_hs + j * D, j < Mk
   const uint16_t* vc;  // fp16 V, the same layout
   const uint8_t* kq;
@@ -3470,7 +3471,7 @@ __global__ __launch_bounds__(PF_THREADS, PF_WG_PER_CU) void prefill_chunk_kernel
     const int r = row0 + 16 * rb + c;
     const bool ok = r < rows_h;
     const int tk = ok ? r / a.gq : 0, hd = h * a.gq + (ok ? r % a.gq : 0);
-    const uint16_t* qr = a.q + ((int64_t)hd * a.M + tk) * D;
+    const uint16_t* qr = a.q + hd * a.q_hs + tk * a.q_ts;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       uint4 w = {0, 0, 0, 0};
@@ -4710,7 +4711,7 @@ extern "C" int64_t nkv_prefill_preferred_bytes(int64_t hkv, int64_t hq, int64_t 
   return std::max<int64_t>(least, p.slots * prefill_slot_bytes(a));
 }
 
-static int prefill_attn(const char* what, const uint16_t* q, int64_t m, const uint16_t* k16, const uint16_t* v16,
+static int prefill_attn(const char* what, const uint16_t* q, int64_t q_ts, int64_t q_hs, int64_t m, const uint16_t* k16, const uint16_t* v16,
                         int64_t m_kv, int64_t kv_head_stride, const uint8_t* kq, const uint16_t* kmn,
                         const uint16_t* kst, const uint8_t* vq, const uint16_t* vmn, const uint16_t* vst,
                         int64_t capacity, int64_t used, int64_t hq, int64_t hkv, int64_t head_dim, uint16_t* out,
@@ -4718,6 +4719,8 @@ static int prefill_attn(const char* what, const uint16_t* q, int64_t m, const ui
   set_error("");
   if (int rc = check_heads(hq, hkv, head_dim)) return rc;
   if (m <= 0 || m > (1 << 20)) return fail(NKV_ERR_INVALID, "%s: query length %lld", what, (long long)m);
+  if (q_ts % 8 || q_hs % 8)
+    return fail(NKV_ERR_UNSUPPORTED, "%s: q strides %lld, %lld (multiples of 8)", what, (long long)q_ts, (long long)q_hs);
   if (m_kv < m || m_kv > (1 << 24))
     return fail(NKV_ERR_INVALID, "%s: %lld fp16 tokens for %lld queries", what, (long long)m_kv, (long long)m);
   if (kv_head_stride < m_kv * D || kv_head_stride % 8)
@@ -4736,7 +4739,7 @@ static int prefill_attn(const char* what, const uint16_t* q, int64_t m, const ui
     return fail(NKV_ERR_INVALID, "%s: workspace of %lld bytes, need %lld", what, (long long)workspace_bytes,
                 (long long)nkv_prefill_workspace_bytes(hkv, hq, m, parts));
   PrefillArgs a{};
-  a.q = q; a.kc = k16; a.vc = v16;
+  a.q = q; a.q_ts = q_ts; a.q_hs = q_hs; a.kc = k16; a.vc = v16;
   a.kq = kq; a.kmn = kmn; a.kst = kst; a.vq = vq; a.vmn = vmn; a.vst = vst;
   a.capacity = capacity; a.ngroups_cap = cdiv(capacity, GT);
   prefill_shape(a, hkv, hq, m, m_kv, used);
@@ -4762,7 +4765,7 @@ extern "C" int nkv_prefill_attn_t64(const uint16_t* q, const uint16_t* k_chunk, 
                                     const uint16_t* vmn, const uint16_t* vst, int64_t capacity, int64_t used,
                                     int64_t hq, int64_t hkv, int64_t head_dim, uint16_t* out, void* workspace,
                                     int64_t workspace_bytes, int64_t splits, void* stream) {
-  return prefill_attn("prefill_attn_t64", q, m, k_chunk, v_chunk, m, m * D, kq, kmn, kst, vq, vmn, vst, capacity,
+  return prefill_attn("prefill_attn_t64", q, D, m * D, m, k_chunk, v_chunk, m, m * D, kq, kmn, kst, vq, vmn, vst, capacity,
                       used, hq, hkv, head_dim, out, workspace, workspace_bytes, splits, stream);
 }
 
@@ -4772,8 +4775,20 @@ extern "C" int nkv_prefill_attn_hist_t64(const uint16_t* q, int64_t m, const uin
                                          const uint16_t* vst, int64_t capacity, int64_t used, int64_t hq, int64_t hkv,
                                          int64_t head_dim, uint16_t* out, void* workspace, int64_t workspace_bytes,
                                          int64_t splits, void* stream) {
-  return prefill_attn("prefill_attn_hist_t64", q, m, k16, v16, m_kv, kv_head_stride, kq, kmn, kst, vq, vmn, vst,
-                      capacity, used, hq, hkv, head_dim, out, workspace, workspace_bytes, splits, stream);
+  return prefill_attn("prefill_attn_hist_t64", q, D, m * D, m, k16, v16, m_kv, kv_head_stride, kq, kmn, kst, vq, vmn,
+                      vst, capacity, used, hq, hkv, head_dim, out, workspace, workspace_bytes, splits, stream);
+}
+
+extern "C" int nkv_prefill_attn_strided_t64(const uint16_t* q, int64_t q_token_stride, int64_t q_head_stride, int64_t m,
+                                            const uint16_t* k16, const uint16_t* v16, int64_t m_kv,
+                                            int64_t kv_head_stride, const uint8_t* kq, const uint16_t* kmn,
+                                            const uint16_t* kst, const uint8_t* vq, const uint16_t* vmn,
+                                            const uint16_t* vst, int64_t capacity, int64_t used, int64_t hq,
+                                            int64_t hkv, int64_t head_dim, uint16_t* out, void* workspace,
+                                            int64_t workspace_bytes, int64_t splits, void* stream) {
+  return prefill_attn("prefill_attn_strided_t64", q, q_token_stride, q_head_stride, m, k16, v16, m_kv, kv_head_stride,
+                      kq, kmn, kst, vq, vmn, vst, capacity, used, hq, hkv, head_dim, out, workspace, workspace_bytes,
+                      splits, stream);
 }
 
 // ---- the chained decode step: every layer of one token in one launch (kernel C)

@@ -140,6 +140,45 @@ struct QuantTokSmem {
   float rul[3][128];     // min, step, 1 / step
 };
 
+// The workgroup's rulers from its waves' channel extremes (lanes 8 cl .. + 7 of each 16): stores the
+// `nch` channels' mins and steps, returns each lane's in mn, st, inv. Two barriers; calls may follow one
+// another (one writes ext before its first barrier, and rul after it: no third barrier).
+template <int W>
+__device__ __forceinline__ void meet_rulers(QuantTokSmem<W>& sm, float (&mn)[8], const float (&mx)[8], float (&st)[8],
+                                            float (&inv)[8], uint16_t* mins, uint16_t* steps, int nch) {
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, cl = t & 15;
+  if (lane < 16) {
+    float4* lo = reinterpret_cast<float4*>(sm.ext[0][wave] + 8 * cl);
+    float4* hi = reinterpret_cast<float4*>(sm.ext[1][wave] + 8 * cl);
+    lo[0] = make_float4(mn[0], mn[1], mn[2], mn[3]); lo[1] = make_float4(mn[4], mn[5], mn[6], mn[7]);
+    hi[0] = make_float4(mx[0], mx[1], mx[2], mx[3]); hi[1] = make_float4(mx[4], mx[5], mx[6], mx[7]);
+  }
+  __syncthreads();
+  if (t < 128) {
+    float lo = sm.ext[0][0][t], hi = sm.ext[1][0][t];
+#pragma unroll
+    for (int w = 1; w < W; ++w) { lo = fminf(lo, sm.ext[0][w][t]); hi = fmaxf(hi, sm.ext[1][w][t]); }
+    const float s = ruler_step(lo, hi);
+    sm.rul[0][t] = lo;
+    sm.rul[1][t] = s;
+    sm.rul[2][t] = ruler_inv(s);
+    if (t < nch) {
+      mins[t] = f2h(lo);
+      steps[t] = f2h(s);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 8; j += 4) {
+    const float4 m4 = *reinterpret_cast<const float4*>(sm.rul[0] + 8 * cl + j);
+    const float4 s4 = *reinterpret_cast<const float4*>(sm.rul[1] + 8 * cl + j);
+    const float4 i4 = *reinterpret_cast<const float4*>(sm.rul[2] + 8 * cl + j);
+    mn[j] = m4.x; mn[j + 1] = m4.y; mn[j + 2] = m4.z; mn[j + 3] = m4.w;
+    st[j] = s4.x; st[j + 1] = s4.y; st[j + 2] = s4.z; st[j + 3] = s4.w;
+    inv[j] = i4.x; inv[j + 1] = i4.y; inv[j + 2] = i4.z; inv[j + 3] = i4.w;
+  }
+}
+
 // W == 1: four independent items (one per wave) in a workgroup of 256 threads, no LDS. R == 0: the
 // group's rows are read in a loop, twice.
 template <int DT, int W, int R, bool PAGES = false>
@@ -148,7 +187,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void quant_token_kernel(Quan
   constexpr int RS = 4 * W;            // rows between a lane's rows
   constexpr int C = R > 0 ? R : 1;
   const int lane = threadIdx.x & 63, ti = W == 1 ? lane : (int)threadIdx.x;
-  const int cl = ti & 15, rl = ti >> 4, wave = ti >> 6;
+  const int cl = ti & 15, rl = ti >> 4;
   const uint32_t items = (uint32_t)a.items, nchunks = (uint32_t)a.nchunks, ngroups = (uint32_t)a.ngroups;
   const uint32_t first = W == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
   for (uint32_t item = first; item < items; item += W == 1 ? gridDim.x * 4 : gridDim.x) {
@@ -208,38 +247,8 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void quant_token_kernel(Quan
         *reinterpret_cast<uint4*>(steps + ch) = pack_h8(st);
       }
     } else {
-      if (lane < 16) {
-        float4* lo = reinterpret_cast<float4*>(sm.ext[0][wave] + 8 * cl);
-        float4* hi = reinterpret_cast<float4*>(sm.ext[1][wave] + 8 * cl);
-        lo[0] = make_float4(mn[0], mn[1], mn[2], mn[3]); lo[1] = make_float4(mn[4], mn[5], mn[6], mn[7]);
-        hi[0] = make_float4(mx[0], mx[1], mx[2], mx[3]); hi[1] = make_float4(mx[4], mx[5], mx[6], mx[7]);
-      }
-      __syncthreads();
-      if (ti < 128) {
-        float lo = sm.ext[0][0][ti], hi = sm.ext[1][0][ti];
-#pragma unroll
-        for (int w = 1; w < W; ++w) { lo = fminf(lo, sm.ext[0][w][ti]); hi = fmaxf(hi, sm.ext[1][w][ti]); }
-        const float s = ruler_step(lo, hi);
-        sm.rul[0][ti] = lo;
-        sm.rul[1][ti] = s;
-        sm.rul[2][ti] = ruler_inv(s);
-        const int64_t c = (int64_t)chunk * 128 + ti;
-        if (c < a.dim) {
-          mins[c] = f2h(lo);
-          steps[c] = f2h(s);
-        }
-      }
-      __syncthreads();
-      // (the next item writes ext before its first barrier, and rul after it: no third barrier)
-#pragma unroll
-      for (int j = 0; j < 8; j += 4) {
-        const float4 m4 = *reinterpret_cast<const float4*>(sm.rul[0] + 8 * cl + j);
-        const float4 s4 = *reinterpret_cast<const float4*>(sm.rul[1] + 8 * cl + j);
-        const float4 i4 = *reinterpret_cast<const float4*>(sm.rul[2] + 8 * cl + j);
-        mn[j] = m4.x; mn[j + 1] = m4.y; mn[j + 2] = m4.z; mn[j + 3] = m4.w;
-        st[j] = s4.x; st[j + 1] = s4.y; st[j + 2] = s4.z; st[j + 3] = s4.w;
-        inv[j] = i4.x; inv[j + 1] = i4.y; inv[j + 2] = i4.z; inv[j + 3] = i4.w;
-      }
+      meet_rulers<W>(sm, mn, mx, st, inv, mins + (int64_t)chunk * 128, steps + (int64_t)chunk * 128,
+                     (int)min<int64_t>(128, a.dim - (int64_t)chunk * 128));
     }
     if (!active) continue;
     if constexpr (R > 0) {
@@ -271,6 +280,70 @@ static void launch_quant_token(const QuantTokArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((quant_token_kernel<DT, 4, 4>), dim3((unsigned)std::min(a.items, most)), dim3(256), 0, s, a);
   else
     hipLaunchKernelGGL((quant_token_kernel<DT, 16, 0>), dim3((unsigned)std::min(a.items, most)), dim3(1024), 0, s, a);
+}
+
+// ---------------------------------------------------------------- a prefill chunk lands in the cache
+//
+// One workgroup per (KV head, K or V, 64 tokens of the chunk) reads its rows once, from wherever the
+// model left them (any token and head stride), and writes what the streaming cache keeps of them: the
+// fp16 copy that the chunk's own attention reads, the newest 64 tokens' ring slots and, for a whole group,
+// codes and rulers (as quant_token_kernel computes them). 2048 tokens x 8 heads of token-major fp16: one
+// launch of 8 us against two copies, two quantizer launches and five small ones for the ring (about
+// 37 us on the GPU).
+struct LandArgs {
+  const uint16_t* src[2];
+  int64_t ts[2], hs[2];  // token and head strides
+  int64_t n, start, capacity, ngroups_cap;
+  int hkv;
+  uint16_t* copy[2];     // [hkv][n][128]
+  uint8_t* codes[2];     // [hkv][capacity][128]
+  uint16_t* mins[2];     // [hkv][ngroups_cap][128]
+  uint16_t* steps[2];
+  uint16_t* ring[2];     // [hkv][64][128]
+};
+
+__global__ __launch_bounds__(256) void land_chunk_kernel(LandArgs a) {
+  __shared__ __attribute__((aligned(16))) QuantTokSmem<4> sm;
+  const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4;
+  const int h = blockIdx.x % a.hkv, which = blockIdx.x / a.hkv & 1;
+  const int64_t g = blockIdx.x / (2 * a.hkv), t0 = g * 64;
+  const int nr = (int)min<int64_t>(64, a.n - t0);
+  const uint16_t* src = a.src[which] + h * a.hs[which] + t0 * a.ts[which] + 8 * cl;
+  uint4 raw[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) raw[i] = *reinterpret_cast<const uint4*>(src + min(rl + 16 * i, nr - 1) * a.ts[which]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = rl + 16 * i;
+    if (r >= nr) break;
+    *reinterpret_cast<uint4*>(a.copy[which] + (h * a.n + t0 + r) * 128 + 8 * cl) = raw[i];
+    if (t0 + r >= a.n - 64)
+      *reinterpret_cast<uint4*>(a.ring[which] + ((int64_t)h * 64 + (a.start + t0 + r) % 64) * 128 + 8 * cl) = raw[i];
+  }
+  if (nr < 64) return;  // (a partial group stays in the ring)
+  float v[4][8], mn[8], mx[8], st[8], inv[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) { mn[j] = __builtin_huge_valf(); mx[j] = -__builtin_huge_valf(); }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t w[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      v[i][j] = h2f((uint16_t)(w[j >> 1] >> (16 * (j & 1))));
+      mn[j] = fminf(mn[j], v[i][j]);
+      mx[j] = fmaxf(mx[j], v[i][j]);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    mn[j] = min4rows(mn[j]);
+    mx[j] = max4rows(mx[j]);
+  }
+  const int64_t so = ((int64_t)h * a.ngroups_cap + a.start / 64 + g) * 128;
+  meet_rulers<4>(sm, mn, mx, st, inv, a.mins[which] + so, a.steps[which] + so, 128);
+  uint8_t* codes = a.codes[which] + ((int64_t)h * a.capacity + a.start + t0 + rl) * 128 + 8 * cl;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2*>(codes + 16 * 128 * i) = pack_codes8(v[i], mn, st, inv);
 }
 
 // ---------------------------------------------------------------- channel-axis quantize
@@ -679,6 +752,31 @@ extern "C" int nkv_paged_quantize_t64(const void* x, int x_dtype, int64_t x_head
   else if (x_dtype == NKV_BF16) hipLaunchKernelGGL((quant_token_kernel<NKV_BF16, 4, 4, true>), grid, block, 0, s, a);
   else hipLaunchKernelGGL((quant_token_kernel<NKV_F32, 4, 4, true>), grid, block, 0, s, a);
   return check_launch("paged_quantize_t64");
+}
+
+extern "C" int nkv_prefill_land_t64(const uint16_t* k, const uint16_t* v, int64_t k_token_stride, int64_t k_head_stride,
+                                    int64_t v_token_stride, int64_t v_head_stride, int64_t n, int64_t start,
+                                    int64_t hkv, int64_t head_dim, int64_t capacity, uint16_t* k16, uint16_t* v16,
+                                    uint8_t* kq, uint16_t* kmn, uint16_t* kst, uint8_t* vq, uint16_t* vmn,
+                                    uint16_t* vst, uint16_t* tail_k, uint16_t* tail_v, void* stream) {
+  g_err.clear();
+  if (head_dim != 128) return fail(NKV_ERR_UNSUPPORTED, "prefill_land: head_dim %lld (only 128 is built)", (long long)head_dim);
+  if (hkv <= 0 || hkv > (1 << 16) || n <= 0 || n > (1 << 24) || start < 0 || start % 64 || start + n > capacity)
+    return fail(NKV_ERR_INVALID, "prefill_land: %lld tokens from %lld (a multiple of 64), hkv=%lld, capacity %lld",
+                (long long)n, (long long)start, (long long)hkv, (long long)capacity);
+  if (!k || !v || !k16 || !v16 || !kq || !kmn || !kst || !vq || !vmn || !vst || !tail_k || !tail_v)
+    return fail(NKV_ERR_INVALID, "prefill_land: null pointer argument");
+  const void* al[] = {k, v, k16, v16, kq, kmn, kst, vq, vmn, vst, tail_k, tail_v};
+  for (const void* p : al)
+    if (!aligned16(p)) return fail(NKV_ERR_UNSUPPORTED, "prefill_land: buffers must be 16-byte aligned");
+  if (k_token_stride % 8 || k_head_stride % 8 || v_token_stride % 8 || v_head_stride % 8)
+    return fail(NKV_ERR_UNSUPPORTED, "prefill_land: strides must be multiples of 8");
+  const int64_t blocks = cdiv(n, 64) * hkv * 2;
+  if (blocks >= (1 << 24)) return fail(NKV_ERR_UNSUPPORTED, "prefill_land: %lld tokens of %lld heads", (long long)n, (long long)hkv);
+  LandArgs a{{k, v}, {k_token_stride, v_token_stride}, {k_head_stride, v_head_stride}, n, start, capacity,
+             cdiv(capacity, 64), (int)hkv, {k16, v16}, {kq, vq}, {kmn, vmn}, {kst, vst}, {tail_k, tail_v}};
+  hipLaunchKernelGGL(land_chunk_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream), a);
+  return check_launch("prefill_land_t64");
 }
 
 extern "C" int nkv_dequantize_int8(const uint8_t* codes, int64_t codes_row_stride,

@@ -278,6 +278,20 @@ def int8_prefill_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Ten
         _require_gpu_tensor(t, nm, torch.uint8)
     for t, nm in ((kmn, "kmn"), (kst, "kst"), (vmn, "vmn"), (vst, "vst")):
         _require_gpu_tensor(t, nm, torch.float16)
+    return _prefill_attend(query, key, value, kq, kmn, kst, vq, vmn, vst, used, out, scratch, splits)
+
+
+def _rows_aligned(x: torch.Tensor) -> bool:
+    """Rows of 128 halves that the kernels can read in place, whatever the head and token strides."""
+    return x.stride(3) == 1 and x.stride(1) % 8 == 0 and x.stride(2) % 8 == 0 and x.data_ptr() % 16 == 0
+
+
+def _prefill_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, kq: torch.Tensor, kmn: torch.Tensor,
+                    kst: torch.Tensor, vq: torch.Tensor, vmn: torch.Tensor, vst: torch.Tensor, used: int,
+                    out: torch.Tensor | None = None, scratch: torch.Tensor | None = None,
+                    splits: int = 0) -> torch.Tensor:
+    """:func:`int8_prefill_attend` of a query that is read where it is (``_rows_aligned``); the output
+    is contiguous."""
     _, hq, n, d = query.shape
     _, hkv, cap, _ = kq.shape
     m = key.shape[2]
@@ -293,7 +307,7 @@ def int8_prefill_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Ten
     if used % GROUP_T or not 0 <= used <= cap:
         raise ValueError(f"used={used} must be a multiple of {GROUP_T} in [0, {cap}]")
     if out is None:
-        out = torch.empty_like(query)
+        out = torch.empty(query.shape, dtype=query.dtype, device=query.device)
     lib = _lib.load()
     least = splits if splits > 0 else int(lib.nkv_prefill_default_splits(hkv, hq, n, used + (m - n) // GROUP_T * GROUP_T))
     need = int(lib.nkv_prefill_workspace_bytes(hkv, hq, n, least))
@@ -301,7 +315,7 @@ def int8_prefill_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Ten
         if _capturing():
             raise ValueError("under graph capture int8_prefill_attend needs a large enough scratch")
         scratch = _lib.workspace(query.device, max(need, int(lib.nkv_prefill_preferred_bytes(hkv, hq, n, m, used, splits))))
-    _lib.call("nkv_prefill_attn_hist_t64", query.data_ptr(), n, key.data_ptr(), value.data_ptr(), m,
+    _lib.call("nkv_prefill_attn_strided_t64", query.data_ptr(), query.stride(2), query.stride(1), n, key.data_ptr(), value.data_ptr(), m,
               key.stride(1), kq.data_ptr(), kmn.data_ptr(), kst.data_ptr(), vq.data_ptr(), vmn.data_ptr(),
               vst.data_ptr(), cap, used, hq, hkv, d, out.data_ptr(), scratch.data_ptr(),
               scratch.numel() * scratch.element_size(), max(0, splits), _lib.stream_ptr(query.device))
@@ -560,11 +574,19 @@ class KVInt8Cache:
         if start + n > self.max_len:
             raise ValueError(f"the prefill would write up to {start + n}, beyond max_len {self.max_len}")
         k16, v16 = self._chunk_tokens(layer, n)
-        k16.copy_(key)
-        v16.copy_(value)
+        if n and key.device == value.device == self.pos.device and _rows_aligned(key) and _rows_aligned(value):
+            i = layer
+            _lib.call("nkv_prefill_land_t64", key.data_ptr(), value.data_ptr(), key.stride(2), key.stride(1),
+                      value.stride(2), value.stride(1), n, start, self.num_kv_heads, self.head_dim, self.max_len,
+                      k16.data_ptr(), v16.data_ptr(), self.kq[i].data_ptr(), self.kmn[i].data_ptr(),
+                      self.kst[i].data_ptr(), self.vq[i].data_ptr(), self.vmn[i].data_ptr(), self.vst[i].data_ptr(),
+                      self.tail_k[i].data_ptr(), self.tail_v[i].data_ptr(), _lib.stream_ptr(self.pos.device))
+        else:  # rows that do not start on 16 bytes
+            k16.copy_(key)
+            v16.copy_(value)
+            self._quantize_groups(layer, k16, v16, start)
+            self._fill_ring(layer, key, value, start + n)
         plan.lengths[layer] = n
-        self._quantize_groups(layer, k16, v16, start)
-        self._fill_ring(layer, key, value, start + n)
         plan.next_start = start + n
 
     def _set_scalars(self, written: int) -> None:
@@ -613,8 +635,10 @@ class KVInt8Cache:
             k16 = self.staging.key_cache[i][:, :, :end]
             v16 = self.staging.value_cache[i][:, :, :end]
             used = 0
-        return int8_prefill_attend(query.contiguous(), k16, v16, self.kq[i], self.kmn[i], self.kst[i], self.vq[i],
-                                   self.vmn[i], self.vst[i], used)
+        cache = (self.kq[i], self.kmn[i], self.kst[i], self.vq[i], self.vmn[i], self.vst[i])
+        if query.is_cuda and query.dtype == torch.float16 and _rows_aligned(query):
+            return _prefill_attend(query, k16, v16, *cache, used)
+        return int8_prefill_attend(query.contiguous(), k16, v16, *cache, used)
 
     # ---- decoding
 

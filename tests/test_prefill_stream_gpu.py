@@ -154,3 +154,38 @@ def test_graph_decoder_streamed_prefill():
         b.input_ids.copy_(a.input_ids)
     print(f"relative logit differences streamed vs staged: {[f'{r:.2e}' for r in rels]}", flush=True)
     assert max(rels) < 1e-2, rels
+
+
+@pytest.mark.parametrize("chunks", [(64, 1), (128, 63), (65,), (192, 64, 130)])
+def test_streamed_chunk_read_in_place(chunks):
+    """A chunk read where the model left it (token-major rows, or rows inside a wider projection) leaves
+    the same state and outputs, bit for bit, as contiguous tensors and as rows off 16 bytes (copied first)."""
+    total = sum(chunks)
+    print(f"case chunks={chunks}", flush=True)
+    k, v = (randn((1, total, H_KV, D), 500 + i, 1.0).cuda() for i in range(2))
+    q = randn((1, total, HQ, D), 502, 1.0).cuda()
+    wide = torch.zeros(1, total, H_KV * D + 8, dtype=torch.float16, device="cuda")
+    odd = torch.zeros(1, total, H_KV * D + 3, dtype=torch.float16, device="cuda")
+    views = {
+        "contiguous": (k.transpose(1, 2).contiguous(), v.transpose(1, 2).contiguous(), q.transpose(1, 2).contiguous()),
+        "token-major": (k.transpose(1, 2), v.transpose(1, 2), q.transpose(1, 2)),
+        "wider rows": (wide[..., 8:].view(1, total, H_KV, D).copy_(k).transpose(1, 2), v.transpose(1, 2), q.transpose(1, 2)),
+        "odd rows": (k.transpose(1, 2), odd[..., 3:].view(1, total, H_KV, D).copy_(v).transpose(1, 2), q.transpose(1, 2)),
+    }
+    want = None
+    for name, (kk, vv, qq) in views.items():
+        c, _ = _caches(total)
+        c.begin_prefill(total, stream_chunk=192)
+        got, off = [], 0
+        for n in chunks:
+            c.set_prefill_pos(off)
+            for layer in range(LAYERS):
+                c.update(kk[:, :, off:off + n], vv[:, :, off:off + n], layer)
+                got.append(c.attend_prefill(qq[:, :, off:off + n], layer))
+                assert got[-1].is_contiguous()
+            off += n
+        c.finish_prefill(total)
+        got += _state(c)
+        want = want or got
+        for i, (x, y) in enumerate(zip(got, want)):
+            assert torch.equal(x, y), f"{name}: tensor {i}"
