@@ -35,6 +35,7 @@
 // blocks, so no data moves between the two products.
 #include "nkv_common.h"
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -271,6 +272,14 @@ __device__ __forceinline__ void load_q(const uint16_t* qh, int gq, half8_t (&qb)
   asm volatile("" ::"v"(qb[0]), "v"(qb[1]), "v"(qb[2]), "v"(qb[3]));
 }
 
+// The lane, or (OPAQUE) the same read through tail_tid's opaque move, so that the offsets made of it are
+// computed at each use and take no registers in between (the paged step's small workgroups have 128 per
+// lane, and a register spilled to memory would make the loop wait for its own streams).
+template <bool OPAQUE>
+__device__ __forceinline__ int lane_of() {
+  return (OPAQUE ? tail_tid() : (int)threadIdx.x) & 63;
+}
+
 // ---------------------------------------------------------------- HBM -> LDS streaming
 
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
@@ -460,9 +469,10 @@ __device__ __forceinline__ void issue_half_paged(const AttnArgs& a, int b, int h
 // The paged per-token symmetric layout's half group: 4 + 4 loads of code rows from the page,
 // then the half's 32 K and 32 V scales (one load each, 4 lanes), into the same slot layout as
 // issue_half_tok.
+template <bool OPAQUE>
 __device__ __forceinline__ void issue_half_paged_tok(const AttnArgs& a, int b, int h, int64_t grp, int hf,
                                                      uint32_t slot) {
-  const int lane = threadIdx.x & 63;
+  const int lane = lane_of<OPAQUE>();
   const int64_t page = max<int64_t>(page_of(a, b, grp), 0);  // as in issue_half_paged
   const void* pb = uniform_ptr(a.pages + (page * a.hkv + h) * PAGE_TOK_BYTES);
   slot = __builtin_amdgcn_readfirstlane(slot);
@@ -482,9 +492,9 @@ __device__ __forceinline__ void issue_half_paged_tok(const AttnArgs& a, int b, i
 }
 
 // Half `hf` of group `grp` in the per-token symmetric format, from either layout.
-template <bool PAGED>
+template <bool PAGED, bool OPAQUE = false>
 __device__ __forceinline__ void issue_tok(const AttnArgs& a, int b, int h, int64_t grp, int hf, uint32_t slot) {
-  if constexpr (PAGED) issue_half_paged_tok(a, b, h, grp, hf, slot);
+  if constexpr (PAGED) issue_half_paged_tok<OPAQUE>(a, b, h, grp, hf, slot);
   else issue_half_tok(a, h, grp, hf, slot);
 }
 
@@ -813,10 +823,11 @@ __device__ __forceinline__ half8_t dq8_sym_v(uint32_t w0, uint32_t w1, uint4 s) 
 
 // attend_block for 32 tokens of the per-token symmetric format: codes as in attend_block
 // (signed), the tokens' K scales at `ksc` and V scales at `vsc` (32 fp16 each).
+template <bool OPAQUE = false>
 __device__ __forceinline__ void attend_block_tok(const AttnArgs& a, WaveState& st, const half8_t (&qb)[4],
                                                  const uint8_t* kc, const uint8_t* vc, const uint16_t* ksc,
                                                  const uint16_t* vsc, int nvalid) {
-  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int lane = lane_of<OPAQUE>(), c = lane & 15, g = lane >> 4;
   // ---- S^T = K Q^T; lane (c, g) holds token 16b + c, whose scale it splats
   float4_t S[2];
 #pragma unroll
@@ -1281,24 +1292,34 @@ constexpr int MERGE_PRE = 32;  // partials per column pair loaded up front
 constexpr int WTS = 256;       // weights one merging wave holds: up to 256 prefix partials
 static_assert(TB_WAVES == WAVES, "the prefix kernel's last workgroup runs the tail with its own waves");
 
-struct TailSmem {
-  uint8_t ring_lds[2 * RING_BYTES];          // K | V values
-  float ring_part[RING_PARTS][16 * D + 32];  // the ring's partials
-  float wts[TB_WAVES * WTS];                 // prefix merge weights, per merging wave
-  float pre_acc[16 * D];                     // prefix: sum_s w_s acc_s per column
-  float pre_m[16], pre_l[16];                // per head: m_p, l_p
-  float rq_ext[2][2 * D];                    // local requantization: per channel min / max of two half rings
-  int lost[TB_WAVES];                        // a merging wave gave up waiting for a partial word
-  uint32_t fwd[(16 + 2) * D / 2];            // the chained step: forwarded q, k_new, v_new of the head (fp16 pairs)
-  uint8_t xpose[RING_PARTS * GT * 64];       // the chained step's append: each ring wave's 64 x 64 codes
-  int ring_staged;                           // ring waves that have staged their slots (the chained step's append)
-  int ring_done;                             // ring waves whose partial is in ring_part (TB_DIRECT)
+// GQ: query heads per KV head that fit; FULL: for every form of the tail, else for the paged per-token
+// step's (no forwarded inputs, no ring to append from, fewer partials of a sequence).
+template <int GQ, bool FULL>
+struct TailSmemOf {
+  static constexpr int PRE = FULL ? MERGE_PRE : 8;  // partials per column pair loaded up front
+  uint8_t ring_lds[2 * RING_BYTES];              // K | V values
+  float ring_part[RING_PARTS][GQ * D + 2 * GQ];  // the ring's partials
+  float wts[TB_WAVES * WTS];                     // prefix merge weights, per merging wave
+  float pre_acc[GQ * D];                         // prefix: sum_s w_s acc_s per column
+  float pre_m[16], pre_l[16];                    // per head: m_p, l_p
+  float rq_ext[2][2 * D];                        // local requantization: per channel min / max of two half rings
+  int lost[TB_WAVES];                            // a merging wave gave up waiting for a partial word
+  uint32_t fwd[FULL ? (16 + 2) * D / 2 : 1];     // the chained step: forwarded q, k_new, v_new of the head (fp16 pairs)
+  // the append: each ring wave's 64 x 64 codes
+  __attribute__((aligned(16))) uint8_t xpose[FULL ? RING_PARTS * GT * 64 : 16];
+  int ring_staged;                               // ring waves that have staged their slots (the chained step's append)
+  int ring_done;                                 // ring waves whose partial is in ring_part (TB_DIRECT)
 };
+using TailSmem = TailSmemOf<16, true>;
+// The paged per-token step's small workgroups (two per CU): at most 4 query heads per KV head
+constexpr int SMALL_GQ = 4;
+using TailSmemSmall = TailSmemOf<SMALL_GQ, false>;
 constexpr int MERGER_MAX_PARTS = 64;         // prefix parts per head of a fused launch
 constexpr int MERGER_MAX_HEADS = 64;         // KV heads of a fused launch: its part-0 workgroups wait for the others
 constexpr int MERGER_SPIN_LIMIT = 1 << 22;   // polls (each followed by a short sleep) before giving up
 static_assert(sizeof(TailSmem) <= LDS_BYTES && sizeof(TailSmem) <= LDS_BYTES_TOK,
               "the tail's LDS fits in the prefix kernel's stages");
+static_assert(sizeof(TailSmemSmall) <= WAVES * HALF_SLOT_TOK, "and in the small workgroups' stages");
 
 // Loads of data other workgroups of the same launch wrote with agent-scope stores: coherent
 // at agent scope (they bypass the XCD-local L2) when `co`, plain loads otherwise.
@@ -1620,11 +1641,12 @@ __device__ __forceinline__ float* paged_ring_slot(const AttnArgs& a, int h, int 
   return paged_block(a, h, b) + (int64_t)a.seq_parts[2 * b + 1] * part_stride(a.gq);
 }
 
-template <bool PAGED>
-__device__ __forceinline__ void tail_body(const AttnArgs& a, int h, int b, TailSmem& sm, int run, int64_t pos,
+template <bool PAGED, class SM>
+__device__ __forceinline__ void tail_body(const AttnArgs& a, int h, int b, SM& sm, int run, int64_t pos,
                                           bool pos_ok, int64_t U, const TailLoads* pre = nullptr,
                                           const half8_t (*pre_q)[4] = nullptr, int flags = 0, int64_t page = -1,
                                           int64_t tag_in = -1) {
+  constexpr int MERGE_PRE = SM::PRE;
   const int tid = tail_tid(), wave = tid >> 6, lane = tid & 63;
   // the tag of the tagged output words and flags: the caller's, else a.ftag
   const uint32_t ftag = tag_in >= 0 ? (uint32_t)tag_in : a.ftag;
@@ -2045,7 +2067,8 @@ __device__ __forceinline__ void tail_body(const AttnArgs& a, int h, int b, TailS
 // staged ring). A token that completes its group is appended by requantizing the whole ring, by
 // every thread before the attention, the ring then attended as int8 as in tail_body. The last of
 // the sequence's workgroups merges the ring slot with the prefix partials (TB_RING_SLOT).
-__device__ __forceinline__ void paged_ring_tail(const AttnArgs& a, int h, int b, TailSmem& sm, int64_t pos, int64_t U,
+template <class SM>
+__device__ __forceinline__ void paged_ring_tail(const AttnArgs& a, int h, int b, SM& sm, int64_t pos, int64_t U,
                                                 const TailLoads& tl, const half8_t (&qb)[4]) {
   const int tid = tail_tid(), wave = tid >> 6, lane = tid & 63;
   const int gq = a.gq;
@@ -2356,11 +2379,18 @@ __device__ __forceinline__ void oproj_rows(const AttnArgs& a, int h, int part, u
   }
 }
 
-template <int LAYOUT, bool QKV = false>
-__global__ __launch_bounds__(THREADS, 1) void attn_prefix_kernel(AttnArgs a) {
+// SMALL (paged, per-token symmetric): each wave streams half groups through one slot instead of two, in
+// half the LDS, so that two workgroups share a CU, with as many loads in flight as one of the others has.
+// One workgroup then streams while the other starts, merges or runs a tail. Used when a launch has more
+// workgroups than CUs (small_paged).
+template <int LAYOUT, bool QKV = false, bool SMALL = false>
+__global__ __launch_bounds__(THREADS, SMALL ? 4 : 1) void attn_prefix_kernel(AttnArgs a) {
   constexpr bool TOK = LAYOUT == CONTIG_TOK || LAYOUT == PAGED_TOK;
   constexpr bool PAGED = LAYOUT == PAGED_T64 || LAYOUT == PAGED_TOK;
-  __shared__ __attribute__((aligned(16))) uint8_t lds_raw[TOK ? LDS_BYTES_TOK : LDS_BYTES];
+  static_assert(!SMALL || LAYOUT == PAGED_TOK, "small workgroups are the paged per-token step's");
+  constexpr int slot_bytes = TOK ? HALF_SLOT_TOK : HALF_SLOT;
+  constexpr int wave_lds = SMALL ? slot_bytes : TOK ? WAVE_LDS_TOK : WAVE_LDS;
+  __shared__ __attribute__((aligned(16))) uint8_t lds_raw[WAVES * wave_lds];
   __shared__ __attribute__((aligned(16))) uint16_t unit_src[TOK || PAGED ? 8 : UNIT_SRC_BYTES / 2];
   __shared__ __attribute__((aligned(16))) uint16_t q_lds[16 * D];
   __shared__ __attribute__((aligned(16))) float xch[UNIT_CH * 2 * WAVES];
@@ -2377,8 +2407,6 @@ __global__ __launch_bounds__(THREADS, 1) void attn_prefix_kernel(AttnArgs a) {
     part = m & 0xffff;
     nparts = a.seq_parts[2 * b + 1];
   }
-  constexpr int wave_lds = TOK ? WAVE_LDS_TOK : WAVE_LDS;
-  constexpr int slot_bytes = TOK ? HALF_SLOT_TOK : HALF_SLOT;
   uint8_t* my_stages = lds_raw + wave * wave_lds;
   const uint32_t my_lds = __builtin_amdgcn_readfirstlane(lds_addr(my_stages));
   const uint32_t src_lds = __builtin_amdgcn_readfirstlane(lds_addr(unit_src));
@@ -2448,7 +2476,10 @@ __global__ __launch_bounds__(THREADS, 1) void attn_prefix_kernel(AttnArgs a) {
   if (!TOK && wave == 0 && append) issue_unit_rows(uio, part, src_lds);
 
   if (wave < ng) {
-    if constexpr (TOK) {
+    if constexpr (SMALL) {
+      issue_tok<PAGED>(a, b, h, gs + wave, 0, my_lds);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DMA_HALF_TOK) : "memory");
+    } else if constexpr (TOK) {
       issue_tok<PAGED>(a, b, h, gs + wave, 0, my_lds);
       issue_tok<PAGED>(a, b, h, gs + wave, 1, my_lds + HALF_SLOT_TOK);
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * DMA_HALF_TOK) : "memory");
@@ -2486,7 +2517,24 @@ __global__ __launch_bounds__(THREADS, 1) void attn_prefix_kernel(AttnArgs a) {
     load_q_lds(q_lds, a.gq, qb);
 
     int gi = wave;
-    for (int rs = 0; gi < ng; rs ^= 1) {
+    if constexpr (SMALL) {
+      const int left = __builtin_amdgcn_readfirstlane((int)(U - gs * GT));
+      for (; gi < ng; gi += WAVES) {
+        const int64_t grp = gs + gi;
+#pragma unroll 1
+        for (int hf = 0; hf < 2; ++hf) {
+          const int nv = min(32, left - GT * gi - 32 * hf);
+          wait_groups_all();
+          if (nv > 0)
+            attend_block_tok<true>(a, st, qb, my_stages, my_stages + HALF_CODE,
+                                   reinterpret_cast<const uint16_t*>(my_stages + 2 * HALF_CODE),
+                                   reinterpret_cast<const uint16_t*>(my_stages + 2 * HALF_CODE + TOK_SCALE_BYTES), nv);
+          if (hf == 0) issue_tok<PAGED, true>(a, b, h, grp, 1, my_lds);
+          else if (gi + WAVES < ng) issue_tok<PAGED, true>(a, b, h, grp + WAVES, 0, my_lds);
+        }
+      }
+    }
+    for (int rs = 0; !SMALL && gi < ng; rs ^= 1) {
       const int64_t grp = gs + gi;
       const uint8_t* rul = my_stages + 2 * HALF_SLOT + rs * RULER_BYTES;
       const uint8_t* slot1 = my_stages + slot_bytes;
@@ -2596,7 +2644,8 @@ __global__ __launch_bounds__(THREADS, 1) void attn_prefix_kernel(AttnArgs a) {
     if (!merger) return;
   }
   __syncthreads();  // the stages and the merge's LDS are dead: the tail reuses them
-  TailSmem& sm = *reinterpret_cast<TailSmem*>(lds_raw);
+  using SM = std::conditional_t<SMALL, TailSmemSmall, TailSmem>;
+  SM& sm = *reinterpret_cast<SM*>(lds_raw);
   if constexpr (PAGED) {
     const int last = nparts - 1;
     int* ctr = a.tail_ctr_end - 1 - (b * a.hkv + h);
@@ -4493,6 +4542,14 @@ extern "C" int nkv_paged_append_t64(const uint16_t* k_new, const uint16_t* v_new
 // The paged prefix launch with its fused tails. int8t64 (`tok` false): the step's token is
 // already in its sequence's ring (nkv_paged_append_t64 ran before), k_new / v_new are unused.
 // Per-token symmetric (`tok`): the launch appends k_new / v_new itself and attends them as the tail.
+// The paged per-token step's small workgroups (two per CU) when one per CU would not hold the launch at
+// once: 448 workgroups of 48 sequences (64 .. 2048 tokens) 38.1 -> 31.6 us a layer, 520 of 64 (to 3000)
+// 54 -> 44 us, 264 of 16 (to 4096) 26.8 -> 21.6 us, 328 of 40 (to 200) 24.1 -> 16.1 us. With 256 or fewer
+// the large ones, whose waves have a second half group in flight, win (8 sequences of 4000 .. 13000: 32.9
+// against 37.1 us). The int8t64 step gains nothing (43.8 against 43.9 us for the 448): its rulers and
+// append do not fit 128 registers.
+static bool small_paged(int64_t workgroups, int gq) { return workgroups > 256 && gq <= SMALL_GQ; }
+
 static int paged_attn(const char* what, const uint16_t* q, const uint16_t* k_new, const uint16_t* v_new,
                       int64_t kv_seq_stride, int64_t kv_head_stride, const uint8_t* pages, const int32_t* page_table,
                       int64_t table_stride, int64_t num_pages, const uint16_t* rings, const int64_t* pos_dev,
@@ -4528,8 +4585,11 @@ static int paged_attn(const char* what, const uint16_t* q, const uint16_t* k_new
   a.tail_ctr_end = reinterpret_cast<int*>(static_cast<char*>(workspace) + (workspace_bytes & ~int64_t(3)));
   l2_args(a);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (tok) hipLaunchKernelGGL(attn_prefix_kernel<PAGED_TOK>, dim3((unsigned)(hkv * total_parts)), dim3(THREADS), 0, s, a);
-  else hipLaunchKernelGGL(attn_prefix_kernel<PAGED_T64>, dim3((unsigned)(hkv * total_parts)), dim3(THREADS), 0, s, a);
+  const dim3 grid((unsigned)(hkv * total_parts));
+  if (tok && small_paged(hkv * total_parts, a.gq))
+    hipLaunchKernelGGL((attn_prefix_kernel<PAGED_TOK, false, true>), grid, dim3(THREADS), 0, s, a);
+  else if (tok) hipLaunchKernelGGL(attn_prefix_kernel<PAGED_TOK>, grid, dim3(THREADS), 0, s, a);
+  else hipLaunchKernelGGL(attn_prefix_kernel<PAGED_T64>, grid, dim3(THREADS), 0, s, a);
   return check_launch(what);
 }
 

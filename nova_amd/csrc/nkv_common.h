@@ -98,8 +98,15 @@ __device__ __forceinline__ float ruler_code_f(float x, float mn, float step, flo
   if (__builtin_fabsf(q - r) > 0.5f - 0x1p-12f) r = __builtin_rintf(__fdiv_rn(d, step));
   return fminf(fmaxf(r, 0.0f), 255.0f);
 }
+// The same as an integer, for the appends inside the attention kernels: the division's operands take the
+// product's place, and the tails that hold 64 values per lane are a little faster so (the paged int8t64
+// step of 8 sequences, 4000 .. 13000 tokens: 35.05 against 35.3 us a layer).
 __device__ __forceinline__ uint32_t ruler_code_rcp(float x, float mn, float step, float inv) {
-  return (uint32_t)ruler_code_f(x, mn, step, inv);
+  const float d = __fsub_rn(x, mn);
+  float q = __fmul_rn(d, inv);
+  if (__builtin_fabsf((q - __builtin_floorf(q)) - 0.5f) < 0x1p-12f) q = __fdiv_rn(d, step);
+  const float r = fminf(fmaxf(__builtin_rintf(q), 0.0f), 255.0f);
+  return (uint32_t)r;
 }
 // Eight such codes packed, one byte each (they are integers in 0 .. 255: the conversion is exact).
 __device__ __forceinline__ uint2 pack_u8x8(const float (&c)[8]) {

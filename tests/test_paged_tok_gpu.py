@@ -251,3 +251,31 @@ def test_tok_released_sequence_appends_and_attends_nothing():
     assert torch.isfinite(out[0]).all() and float(out[0].abs().sum()) > 0
     changed = (cache.pages[0] != before[0]).any(dim=2).any(dim=1).nonzero().flatten().tolist()
     assert set(changed) <= set(cache._owned[0]), "only sequence 0's pages may change"
+
+
+@pytest.mark.parametrize("lens,target", [
+    ([1, 31, 32, 33, 63, 64, 65, 127, 128, 129] * 3 + [500, 513, 575, 1100], 1),  # whole and half groups of every length
+    ([600, 700, 1025, 2000], 36),  # several units per sequence, fewer groups than waves in each
+])
+def test_tok_small_workgroups_match_contiguous_caches(lens, target):
+    """More workgroups than CUs: the kernel with one half group per wave."""
+    steps = 2
+    print(f"case tok small lens={lens} target={target}", flush=True)
+    ks, vs, qs = _data(lens, steps, seed=150)
+    paged = _paged(lens, steps, ks, vs, seed=151)
+    paged.target_parts = target
+    _fill(paged, lens, ks, vs)
+    assert paged.total_parts * H_KV > 256
+    conts = [_contiguous(n, steps, ks[b], vs[b]) for b, n in enumerate(lens)]
+    for i in range(steps):
+        kn, vn = _step_inputs(ks, vs, lens, i)
+        for layer in range(LAYERS):
+            out = paged.decode_step(kn, vn, qs[i], layer).clone()
+            for b, (n, c) in enumerate(zip(lens, conts)):
+                c.pos.fill_(n + i)
+                want = c.update_attend(ks[b][:, :, n + i:n + i + 1], vs[b][:, :, n + i:n + i + 1],
+                                       qs[i][b:b + 1], layer)
+                assert_ulp_or_abs(npy(out[b, :, 0]), npy(want[0, :, 0]).astype(np.float64), 2.0, 1e-5,
+                                  f"b={b} step={i} layer={layer}")
+        paged.advance()
+    _check_state(paged, conts, lens, steps)
