@@ -124,6 +124,9 @@ int64_t nkv_attn_workspace_bytes(int64_t hkv, int64_t hq, int64_t n_parts);
 
 /* The n_parts value that `n_parts = 0` resolves to for `groups` rulers per head. */
 int64_t nkv_attn_default_parts(int64_t hkv, int64_t groups);
+/* More parts for short prefixes (up to one per group): the n_parts at which a decode step over `groups`
+ * groups takes the least time, for a workspace of nkv_attn_workspace_bytes of as many. */
+int64_t nkv_attn_step_parts(int64_t hkv, int64_t groups);
 
 /*
  * Streaming append of one decode token into the int8 cache of one layer.

@@ -52,6 +52,7 @@ SIGNATURES = {
                                     P, P, P, I64, I64, P]),
     "nkv_attn_workspace_bytes": (I64, [I64, I64, I64]),
     "nkv_attn_default_parts": (I64, [I64, I64]),
+    "nkv_attn_step_parts": (I64, [I64, I64]),
     "nkv_append_t64": (c_int, [P, P, I64, P, P, P, P, P, P, P, P, P, P, P, P, I64, I64, I64, P]),
     "nkv_decode_step_t64": (c_int, _STEP),
     "nkv_decode_step_partials_t64": (c_int, _STEP),
@@ -202,8 +203,8 @@ _WORKSPACES: dict[str, torch.Tensor] = {}
 _RETIRED: list[torch.Tensor] = []
 
 
-def workspace(device: torch.device, nbytes: int, kind: str = "scratch") -> torch.Tensor:
-    """A cached per-device, zero-filled byte workspace of at least ``nbytes``. It grows only
+def workspace(device: torch.device, nbytes: int, kind: str = "scratch", zero: bool = True) -> torch.Tensor:
+    """A cached per-device byte workspace of at least ``nbytes``, zero-filled unless told not to. It grows only
     outside graph capture (a capture that needs more raises); the buffer it replaces is kept,
     never freed, because a captured graph may point into it. Callers pass the whole buffer
     (``numel()`` bytes)."""
@@ -215,6 +216,6 @@ def workspace(device: torch.device, nbytes: int, kind: str = "scratch") -> torch
                                "pass a preallocated scratch buffer")
         if w is not None:
             _RETIRED.append(w)
-        w = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+        w = (torch.zeros if zero else torch.empty)(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _WORKSPACES[key] = w
     return w

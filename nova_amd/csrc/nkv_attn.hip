@@ -3935,6 +3935,18 @@ static int64_t default_parts(int64_t hkv, int64_t groups) {
   return std::min<int64_t>(max_parts, std::max<int64_t>(1, cdiv(groups, 8)));
 }
 
+// The same for latency: one unit per group up to 32 (what the merging waves load at once). A short prefix
+// is bound by the latency of one workgroup's share, not by the merge: a step of 8 KV heads with 8 groups
+// each / this many units: 1000 tokens 13.7 / 10.2 us (per-token format 12.7 / 10.7), 4095 tokens 16.6 /
+// 14.5 (12.9 / 11.6), 8191 tokens 18.0 / 15.8 (13.7 / 12.9). Where a head's workgroups do not share an XCD
+// (the hand-over goes through memory), half as many and at most 16: 2 KV heads, 1000 tokens 13.5 / 10.8 us
+// (15.5 / 15.0), 4095 tokens 17.0 / 15.5 (17.3 / 16.4); up to 8 groups they keep the one unit.
+static int64_t step_parts(int64_t hkv, int64_t groups) {
+  const int64_t max_parts = std::max<int64_t>(1, 256 / std::max<int64_t>(1, hkv)), least = default_parts(hkv, groups);
+  if (hkv % 8) return groups <= 8 ? least : std::max(least, std::min({max_parts, groups / 2, (int64_t)16}));
+  return std::max(least, std::min({max_parts, groups, (int64_t)32}));
+}
+
 static int64_t part_floats(int64_t hq, int64_t hkv) { return part_stride((int)(hq / hkv)); }
 // Bytes of the fused tail's publication area: `n` ints (per head a counter and a flag per
 // partial; paged, a counter per sequence and head), rounded up to 256 bytes.
@@ -4035,6 +4047,7 @@ extern "C" int64_t nkv_attn_workspace_bytes(int64_t hkv, int64_t hq, int64_t n_p
 }
 
 extern "C" int64_t nkv_attn_default_parts(int64_t hkv, int64_t groups) { return default_parts(hkv, groups); }
+extern "C" int64_t nkv_attn_step_parts(int64_t hkv, int64_t groups) { return step_parts(hkv, groups); }
 
 extern "C" int nkv_attn_decode_t64(const uint16_t* q, const uint8_t* kq, const uint16_t* kmn,
                                    const uint16_t* kst, const uint8_t* vq, const uint16_t* vmn,

@@ -116,7 +116,7 @@ def _parts_fitting(hkv: int, hq: int, groups: int, capacity_bytes: int | None) -
     """The library's default prefix parts for ``groups`` rulers per head, reduced until their
     partials fit ``capacity_bytes`` (when given)."""
     lib = _lib.load()
-    parts = int(lib.nkv_attn_default_parts(hkv, groups))
+    parts = int(lib.nkv_attn_step_parts(hkv, groups))
     if capacity_bytes is None:
         return parts
     while parts > 1 and int(lib.nkv_attn_workspace_bytes(hkv, hq, parts)) > capacity_bytes:
@@ -314,7 +314,8 @@ def _prefill_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
     if scratch is None or scratch.numel() * scratch.element_size() < need:
         if _capturing():
             raise ValueError("under graph capture int8_prefill_attend needs a large enough scratch")
-        scratch = _lib.workspace(query.device, max(need, int(lib.nkv_prefill_preferred_bytes(hkv, hq, n, m, used, splits))))
+        need = max(need, int(lib.nkv_prefill_preferred_bytes(hkv, hq, n, m, used, splits)))
+        scratch = _lib.workspace(query.device, need, "prefill", zero=False)  # (written before it is read)
     _lib.call("nkv_prefill_attn_strided_t64", query.data_ptr(), query.stride(2), query.stride(1), n, key.data_ptr(), value.data_ptr(), m,
               key.stride(1), kq.data_ptr(), kmn.data_ptr(), kst.data_ptr(), vq.data_ptr(), vmn.data_ptr(),
               vst.data_ptr(), cap, used, hq, hkv, d, out.data_ptr(), scratch.data_ptr(),
@@ -424,7 +425,7 @@ class KVInt8Cache:
         self.pm = torch.zeros(sshape, dtype=torch.float32, device=device)
         self.pl = torch.zeros_like(self.pm)
         pa_numel = hkv * self.n_splits * PAD_M * d
-        parts = int(lib.nkv_attn_default_parts(hkv, n_groups))
+        parts = int(lib.nkv_attn_step_parts(hkv, n_groups))
         need = int(lib.nkv_attn_workspace_bytes(hkv, self.num_q_heads, parts))
         self._ws = torch.zeros(max(pa_numel, _cdiv(need, 4)), dtype=torch.float32, device=device)
         self._ws_bytes = self._ws.numel() * 4

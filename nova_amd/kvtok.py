@@ -76,7 +76,7 @@ def _check(x: torch.Tensor, name: str, dtype: torch.dtype) -> None:
 
 def _parts(hkv: int, hq: int, groups: int, ws_bytes: int) -> int:
     lib = _lib.load()
-    parts = int(lib.nkv_attn_default_parts(hkv, groups))
+    parts = int(lib.nkv_attn_step_parts(hkv, groups))
     per_part = int(lib.nkv_attn_workspace_bytes(hkv, hq, 1))
     return max(1, min(parts, ws_bytes // per_part))
 
@@ -109,7 +109,7 @@ def int8_tok_attn_decode(q: torch.Tensor, kq: torch.Tensor, ksc: torch.Tensor, v
         out = torch.empty_like(q)
     groups = cap // GROUP
     if scratch is None:
-        parts = int(n_splits) if n_splits else int(_lib.load().nkv_attn_default_parts(hkv, groups))
+        parts = int(n_splits) if n_splits else int(_lib.load().nkv_attn_step_parts(hkv, groups))
         scratch = _lib.workspace(q.device, int(_lib.load().nkv_attn_workspace_bytes(hkv, hq, parts)), "decode")
     else:
         parts = int(n_splits) if n_splits else _parts(hkv, hq, groups, scratch.numel() * scratch.element_size())
@@ -151,7 +151,7 @@ class KVInt8TokCache:
         self.pos = torch.zeros(1, dtype=torch.long, device=device)
         self._written = torch.zeros(1, dtype=torch.long, device=device)
         self._prefill_off = 0
-        self._n_parts = int(_lib.load().nkv_attn_default_parts(self.num_kv_heads, self.max_len // GROUP))
+        self._n_parts = int(_lib.load().nkv_attn_step_parts(self.num_kv_heads, self.max_len // GROUP))
         self._ws_bytes = int(_lib.load().nkv_attn_workspace_bytes(self.num_kv_heads, self.num_q_heads, self._n_parts))
         self.pa = torch.zeros(self._ws_bytes // 4, dtype=torch.float32, device=device)
         self.lse = torch.zeros((1, self.num_q_heads), dtype=torch.float32, device=device)

@@ -246,3 +246,14 @@ def test_chained_step_input_rules(lib):
     assert lib.nkv_decode_layers_check_t64(t.ctypes.data, L, 512, 32, 8, HEAD) == OK
     assert lib.nkv_decode_layers_check_t64(None, L, 512, 32, 8, HEAD) == BAD
     assert lib.nkv_decode_layers_check_t64(t.ctypes.data, L, 512, 32, 8, 2) == BAD
+
+
+def test_step_parts_stay_within_the_workspace_rules(lib):
+    """At least the default parts, at most one workgroup per CU and (beyond the default) one per group
+    and the 32 partials that the merge loads at once."""
+    for hkv in (1, 2, 3, 8, 16, 64, 256, 300):
+        for groups in (1, 2, 8, 9, 31, 32, 33, 256, 257, 1024):
+            least, n = lib.nkv_attn_default_parts(hkv, groups), lib.nkv_attn_step_parts(hkv, groups)
+            assert least <= n <= max(1, 256 // hkv), (hkv, groups, n)
+            assert n == least or n <= min(groups, 32), (hkv, groups, n)
+    assert lib.nkv_attn_step_parts(8, 4) == 4 and lib.nkv_attn_step_parts(2, 8) == 1
