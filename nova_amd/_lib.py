@@ -118,6 +118,8 @@ ABI_VERSION = 11
 _lib = None
 _lock = threading.Lock()
 _l2_probed = False
+_gpu_seen = False  # torch has shown a GPU (it does not go away)
+
 
 class NovaKVError(RuntimeError):
     """A failing ``nkv_*`` call; ``code`` is the NKV_ERR_* status."""
@@ -129,9 +131,13 @@ class NovaKVError(RuntimeError):
 
 def load(require_gpu: bool = True):
     """Load (once) and return the ctypes handle of ``libnova_kv.so``."""
-    global _lib
-    if require_gpu and not torch.cuda.is_available():
-        raise RuntimeError("nova_amd needs a ROCm GPU (gfx950); none is visible to torch")
+    global _lib, _gpu_seen
+    if _lib is not None and _l2_probed and _gpu_seen:  # (every later call)
+        return _lib
+    if require_gpu and not _gpu_seen:
+        if not torch.cuda.is_available():
+            raise RuntimeError("nova_amd needs a ROCm GPU (gfx950); none is visible to torch")
+        _gpu_seen = True
     if _lib is not None:
         if not _l2_probed and require_gpu:
             _probe_l2()
@@ -190,8 +196,10 @@ def call(name: str, *args) -> None:
 
 
 def stream_ptr(device: torch.device | None = None) -> int:
-    """The current torch stream of ``device`` as a raw ``hipStream_t``."""
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current torch stream of ``device`` as a raw ``hipStream_t`` (without the stream object that
+    ``torch.cuda.current_stream`` builds, 2 us of a call)."""
+    index = None if device is None else torch.device(device).index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
