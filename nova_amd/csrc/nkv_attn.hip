@@ -2400,12 +2400,14 @@ __global__ __launch_bounds__(THREADS, SMALL ? 4 : 1) void attn_prefix_kernel(Att
   const int h = blockIdx.x % a.hkv;
   // work unit -> (sequence, part of its prefix, parts of that sequence, partial slot)
   int b = 0, part = blockIdx.x / a.hkv, nparts = a.n_parts;
-  const int pslot = part;
+  int pslot = part;
   if constexpr (PAGED) {
-    const int m = a.wg_map[pslot];
+    const int m = a.wg_map[part];
     b = m >> 16;
     part = m & 0xffff;
-    nparts = a.seq_parts[2 * b + 1];
+    const int2 sp = *reinterpret_cast<const int2*>(a.seq_parts + 2 * b);
+    pslot = sp.x + part;
+    nparts = sp.y;
   }
   uint8_t* my_stages = lds_raw + wave * wave_lds;
   const uint32_t my_lds = __builtin_amdgcn_readfirstlane(lds_addr(my_stages));
@@ -2592,8 +2594,8 @@ __global__ __launch_bounds__(THREADS, SMALL ? 4 : 1) void attn_prefix_kernel(Att
     const int gq = a.gq, pw = part_stride(gq);
     store_wave_partial(st, gq, reinterpret_cast<float*>(my_stages));
     __syncthreads();
-    // (paged: unit pslot is part `part` of sequence b, whose units begin at seq_parts[2b] = pslot - part,
-    // so its slot is that of paged_block without reading seq_parts)
+    // (paged: pslot counts the parts from sequence 0 on, whatever order the units are in, so this is
+    // paged_block's slot `part`)
     float* dst = a.ws + ((int64_t)h * (PAGED ? a.total_parts + a.nseq : a.n_parts) + pslot + (PAGED ? b : 0)) * pw;
     auto wpart = [&](int w) { return reinterpret_cast<const float*>(lds_raw + w * wave_lds); };
     // (a paged sequence's partials beyond the WTS its tail merges are not published)
@@ -4627,6 +4629,7 @@ static int paged_attn(const char* what, const uint16_t* q, const uint16_t* k_new
     a.k_new = k_new; a.v_new = v_new; a.kv_hs = kv_head_stride; a.kv_ss = kv_seq_stride;
   }
   if (!q || !wg_map || !seq_parts || !out || !workspace) return fail(NKV_ERR_INVALID, "%s: null pointer argument", what);
+  if (reinterpret_cast<uintptr_t>(seq_parts) & 7u) return fail(NKV_ERR_UNSUPPORTED, "%s: seq_parts must be 8-byte aligned", what);
   if (!al16(q) || !al16(workspace)) return fail(NKV_ERR_UNSUPPORTED, "%s: buffers must be 16-byte aligned", what);
   if (total_parts < nseq || total_parts > 65535)
     return fail(NKV_ERR_INVALID, "%s: total_parts %lld outside [nseq, 65535]", what, (long long)total_parts);

@@ -228,6 +228,12 @@ class PagedKVInt8Cache:
         grow (each unit covers a fixed fraction of its sequence's groups)."""
         lengths = list(self._len if lengths is None else lengths)
         wg_map, seq_parts = plan_parts(lengths, self.target_parts)
+        if len(wg_map) * self.num_kv_heads > 256:
+            # more workgroups than CUs: the longest units (in groups per wave) start first, so that the ones
+            # that start last, or share a CU, are short. 48 sequences of 64 .. 2048 tokens: 43.0 -> 37.5 us
+            # a layer (per-token format 31.6 -> 26.9), 64 of 100 .. 3000: 66 -> 54 us (45 -> 43)
+            groups = [max(1, int(n) // GT) for n in lengths]
+            wg_map.sort(key=lambda u: -(-(-groups[u >> 16] // (8 * seq_parts[2 * (u >> 16) + 1]))))
         dev = self.page_table.device
         self.wg_map = torch.tensor(wg_map, dtype=torch.int32, device=dev)
         self.seq_parts = torch.tensor(seq_parts, dtype=torch.int32, device=dev)

@@ -241,3 +241,32 @@ def test_released_sequence_appends_and_attends_nothing():
     assert torch.isfinite(out[0]).all() and float(out[0].abs().sum()) > 0
     changed = (cache.pages[0] != before[0]).any(dim=2).any(dim=1).nonzero().flatten().tolist()
     assert set(changed) <= set(cache._owned[0]), "only sequence 0's pages may change"
+
+
+@pytest.mark.parametrize("tok", [False, True])
+def test_unit_order_does_not_change_a_bit(tok):
+    """The plan's order (longest units first where they outnumber the CUs) against units in sequence
+    order and in reverse: the same outputs and pages."""
+    from nova_amd.paged import PagedKVInt8Cache, PagedKVInt8TokCache, plan_parts
+
+    lens = [70, 2000, 64, 1100, 300, 1, 900, 129] * 5
+    cls = PagedKVInt8TokCache if tok else PagedKVInt8Cache
+    g = torch.Generator(device="cuda").manual_seed(7)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").half()  # noqa: E731
+    k, v = rnd(1, H_KV, 2000, D), rnd(1, H_KV, 2000, D)
+    kn, vn, q = rnd(len(lens), H_KV, 1, D), rnd(len(lens), H_KV, 1, D), rnd(len(lens), HQ, 1, D)
+    got = []
+    for order in ("plan", "sequence", "reverse"):
+        cache = cls(1, H_KV, D, HQ, max_seqs=len(lens), num_pages=sum(n // 64 + 1 for n in lens),
+                    max_pages_per_seq=32)
+        for b, n in enumerate(lens):
+            cache.prefill(b, 0, k[:, :, :n], v[:, :, :n])
+        cache.plan()
+        plain, _ = plan_parts(lens, cache.target_parts)
+        assert len(plain) * H_KV > 256 and sorted(cache.wg_map.tolist()) == sorted(plain)
+        if order != "plan":
+            cache.wg_map = torch.tensor(plain if order == "sequence" else plain[::-1], dtype=torch.int32, device="cuda")
+        out = [cache.decode_step(kn, vn, q, 0).clone() for _ in range(2)]
+        got.append((*out, cache.lse.clone(), cache.pages[0]))
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], other))
