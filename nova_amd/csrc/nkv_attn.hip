@@ -4710,14 +4710,15 @@ extern "C" int64_t nkv_prefill_workspace_bytes(int64_t hkv, int64_t hq, int64_t 
 // 2 us. Three cuttings; the one whose longest share is the shortest, its other costs counted in steps:
 //  - at tile boundaries (nothing to merge): many tiles per share;
 //  - every tile into the same number of parts: few tiles of about equal length (512 tokens over 16384:
-//    8 tiles x 4 parts). The partials' writes and the combine kernel cost about 6 steps;
+//    8 tiles x 4 parts; 143 tokens over 337 of fp16 history, 2 KV heads: 5 tiles x 6 parts, 18.3 us, 23.0
+//    at tile boundaries);
 //  - even shares of the head's steps, wherever they end (a cut within 4 steps of a tile boundary moves
 //    there): tiles of unequal length, or a number of them that does not fit the CUs.
 // The first and the last take the tiles in zigzag order, so that each two neighbours have the same
 // sum: with a tile per share, only every second one is cut (2048 tokens: 32 tiles, the last with 31
-// more steps than the first). The last two take what slots the workspace has;
-// nkv_prefill_workspace_bytes always holds the second's.
-constexpr double PF_TILE_COST = 1.0, PF_PARTS_COST = 6.0, PF_EVEN_COST = 8.0;
+// more steps than the first). The combine launch costs about 2.5 steps, and the partials' writes and
+// reads 4.5 for 256 of them (35 MB). The last two take what slots the workspace has.
+constexpr double PF_TILE_COST = 1.0, PF_MERGE_COST = 2.5, PF_PARTIALS_COST = 4.5;
 constexpr int64_t PF_MIN_SHARE = 4;  // steps of an even share, at least
 constexpr int64_t PF_SNAP = 4;
 
@@ -4763,9 +4764,8 @@ static double prefill_cut(const PrefillArgs& a, int64_t T, int64_t W, int64_t sn
   return longest;
 }
 
-// `splits` > 0 bounds the shares to splits per tile; `parts` is the parts per tile of the second
-// cutting. Leaves the chosen order in `a` and in p.
-static void prefill_plan(PrefillArgs& a, int64_t splits, int64_t parts, int64_t avail_slots, PrefillPlan& p) {
+// `splits` > 0 bounds the shares to splits per tile. Leaves the chosen order in `a` and in p.
+static void prefill_plan(PrefillArgs& a, int64_t splits, int64_t avail_slots, PrefillPlan& p) {
   const int64_t G = a.U / GT;
   const int64_t cap = std::max<int64_t>(1, PF_MAX_SHARES / a.hkv);  // one workgroup per CU
   const int64_t W = std::min<int64_t>(cap, a.tiles);
@@ -4775,17 +4775,34 @@ static void prefill_plan(PrefillArgs& a, int64_t splits, int64_t parts, int64_t 
     T += n;
     longest = std::max(longest, n);
   }
-  // parts per tile (no part without a step: tile 0 is the shortest), and the even shares
-  const int64_t per_tile = std::max<int64_t>(1, std::min({parts, (int64_t)(PF_MAX_SHARES / a.tiles), G + pf_fp16_groups(a, 0)}));
+  // parts per tile (one round of workgroups; no part without a step: tile 0 is the shortest), and the even
+  // shares
+  const int64_t parts = splits > 0 ? splits : cap / a.tiles;
+  const int64_t per_tile = std::max<int64_t>(1, std::min({parts, (int64_t)(PF_MAX_SHARES / a.tiles),
+                                                          G + pf_fp16_groups(a, 0), avail_slots / a.tiles}));
   int64_t We = std::max<int64_t>(a.tiles, T / PF_MIN_SHARE);
   if (splits > 0) We = std::min<int64_t>(We, a.tiles * splits);
   We = std::min(We, std::min(cap, T));
   const double none = __builtin_huge_val();
+  auto merge_cost = [&](int64_t partials) {  // of a head
+    return PF_MERGE_COST + PF_PARTIALS_COST * (double)(partials * a.hkv * a.slot_rows) / (256.0 * PF_ROWS);
+  };
   a.zigzag = 1;
-  const double c_even = 2 * We <= avail_slots ? prefill_cut(a, T, We, PF_SNAP, p) + PF_EVEN_COST : none;
+  double c_even = none;
+  if (2 * We <= avail_slots) {
+    c_even = prefill_cut(a, T, We, PF_SNAP, p);
+    int64_t partials = 0;  // a cut inside a tile ends one part of it; the tile's last part ends with it
+    for (int w = 1, tile = -1; w < p.shares; ++w) {
+      if (p.cut[w].step == 0) continue;
+      partials += p.cut[w].tile == tile ? 1 : 2;
+      tile = p.cut[w].tile;
+    }
+    if (partials) c_even += merge_cost(partials);
+  }
   const double c_tiles = prefill_cut(a, T, W, INT64_MAX, p);
-  const double c_parts = per_tile > 1 && a.tiles * per_tile <= avail_slots
-                             ? (double)(cdiv(longest, per_tile) * cdiv(a.tiles * per_tile, cap)) + PF_PARTS_COST : none;
+  const double c_parts = per_tile > 1 ? (double)(cdiv(longest, per_tile) * cdiv(a.tiles * per_tile, cap)) + PF_TILE_COST +
+                                            merge_cost(a.tiles * per_tile)
+                                      : none;
   const double best = std::min({c_tiles, c_parts, c_even});
   p.zigzag = a.zigzag = best != c_parts;
   if (best == c_tiles) return;  // (cut already)
@@ -4826,9 +4843,9 @@ extern "C" int64_t nkv_prefill_preferred_bytes(int64_t hkv, int64_t hq, int64_t 
   PrefillArgs a{};
   prefill_shape(a, hkv, hq, m, m_kv, used);
   PrefillPlan p;
-  const int64_t parts = splits > 0 ? splits : nkv_prefill_default_splits(hkv, hq, m, used);
-  prefill_plan(a, splits, parts, INT64_MAX, p);
-  const int64_t least = nkv_prefill_workspace_bytes(hkv, hq, m, parts);
+  prefill_plan(a, splits, INT64_MAX, p);
+  const int64_t least = nkv_prefill_workspace_bytes(
+      hkv, hq, m, splits > 0 ? splits : nkv_prefill_default_splits(hkv, hq, m, used));
   return std::max<int64_t>(least, p.slots * prefill_slot_bytes(a));
 }
 
@@ -4868,7 +4885,7 @@ static int prefill_attn(const char* what, const uint16_t* q, int64_t q_ts, int64
   a.sl2 = LOG2E / sqrtf((float)head_dim);
   a.ws = static_cast<float*>(workspace); a.out = out;
   PrefillPlan p;
-  prefill_plan(a, splits, parts, workspace_bytes / prefill_slot_bytes(a), p);
+  prefill_plan(a, splits, workspace_bytes / prefill_slot_bytes(a), p);
   a.shares = p.shares; a.slots = p.slots; a.two_slots = p.two_slots;
   for (int w = 0; w <= p.shares; ++w) a.cut[w] = p.cut[w];
   hipStream_t s = static_cast<hipStream_t>(stream);
