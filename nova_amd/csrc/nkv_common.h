@@ -123,11 +123,19 @@ __device__ __forceinline__ float ruler_inv(float step) { return __builtin_amdgcn
 // The per-token symmetric ("tok") arithmetic: scale = max(absmax / 127, 1e-8) in fp32 (stored
 // as fp16), code = clamp(rint(x / scale), -127, 127) with the fp32 scale.
 __device__ __forceinline__ float sym_scale(float amax) { return fmaxf(__fdiv_rn(amax, 127.0f), 1e-8f); }
-// (the quotient as x * rcp(scale) unless it is near a half-integer, as ruler_code_f: |x / scale| <= 127.1)
+// RCP: the quotient as x * rcp(scale) unless it is near a half-integer, as ruler_code_f (|x / scale| <=
+// 127.1): fewer instructions for a kernel that does nothing else; the attention kernels, which quantize one
+// row per head on a cold instruction cache, take the division alone.
+template <bool RCP>
 __device__ __forceinline__ uint32_t sym_code(float x, float scale, float inv) {
-  const float q = __fmul_rn(x, inv);
-  float r = __builtin_rintf(q);
-  if (__builtin_fabsf(q - r) > 0.5f - 0x1p-12f) r = __builtin_rintf(__fdiv_rn(x, scale));
+  float r;
+  if constexpr (RCP) {
+    const float q = __fmul_rn(x, inv);
+    r = __builtin_rintf(q);
+    if (__builtin_fabsf(q - r) > 0.5f - 0x1p-12f) r = __builtin_rintf(__fdiv_rn(x, scale));
+  } else {
+    r = __builtin_rintf(__fdiv_rn(x, scale));
+  }
   return (uint32_t)(int32_t)fminf(fmaxf(r, -127.0f), 127.0f) & 0xffu;
 }
 
@@ -142,15 +150,16 @@ __device__ __forceinline__ float row16_max(float v) {
 
 // One 128-value row quantized by the 16 lanes of a 16-lane row, 8 values per lane: returns
 // the lane's 8 packed codes and (in every lane) the fp32 scale.
+template <bool RCP = false>
 __device__ __forceinline__ uint2 sym_quant8(const float (&v)[8], float& scale) {
   float amax = 0.0f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) amax = fmaxf(amax, __builtin_fabsf(v[j]));
   scale = sym_scale(row16_max(amax));
-  const float inv = ruler_inv(scale);
+  const float inv = RCP ? ruler_inv(scale) : 0.0f;
   uint32_t c[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) c[j] = sym_code(v[j], scale, inv);
+  for (int j = 0; j < 8; ++j) c[j] = sym_code<RCP>(v[j], scale, inv);
   return uint2{c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24), c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24)};
 }
 

@@ -574,7 +574,7 @@ __global__ __launch_bounds__(256) void quant_sym_kernel(QuantSymArgs a) {
     float v[8];
     Elem8<DT>::load(a.x, r * a.x_rs + t * 128 + c8, v);
     float scale;
-    const uint2 cw = sym_quant8(v, scale);
+    const uint2 cw = sym_quant8<true>(v, scale);
     uint8_t* code_row = a.codes + r * a.c_rs + t * 128;
     uint16_t* scale_at = a.scales + r * a.s_rs + t;
     if constexpr (PAGES) {
