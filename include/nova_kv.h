@@ -508,8 +508,8 @@ int nkv_decode_layers_check_tok(const nkv_layer_tok* layers_host, int64_t n_laye
  * k_new / v_new: [nseq][hkv][128] fp16 with strides kv_seq_stride / kv_head_stride.
  * Prefix work unit w (w < total_parts) serves sequence wg_map[w] >> 16, part
  * wg_map[w] & 0xffff of its seq_parts[2b + 1] parts; seq_parts[2b] counts the parts of the sequences
- * before it. The units may be in any order (each of them once); the first ones start first. seq_parts is
- * 8-byte aligned. A sequence has at most 256 parts
+ * before it. The units may be in any order (each of them once); the first ones start first. A sequence has at
+ * most 256 parts
  * (the tail's merge holds 256 partials; it ignores partials beyond them).
  * q / out: [nseq][hq][128] fp16; lse_out [nseq][hq] fp32 (may be NULL).
  * The workspace holds per KV head one partial slot per unit and one per sequence (the int8t64

@@ -2405,9 +2405,8 @@ __global__ __launch_bounds__(THREADS, SMALL ? 4 : 1) void attn_prefix_kernel(Att
     const int m = a.wg_map[part];
     b = m >> 16;
     part = m & 0xffff;
-    const int2 sp = *reinterpret_cast<const int2*>(a.seq_parts + 2 * b);
-    pslot = sp.x + part;
-    nparts = sp.y;
+    pslot = a.seq_parts[2 * b] + part;
+    nparts = a.seq_parts[2 * b + 1];
   }
   uint8_t* my_stages = lds_raw + wave * wave_lds;
   const uint32_t my_lds = __builtin_amdgcn_readfirstlane(lds_addr(my_stages));
@@ -4629,7 +4628,6 @@ static int paged_attn(const char* what, const uint16_t* q, const uint16_t* k_new
     a.k_new = k_new; a.v_new = v_new; a.kv_hs = kv_head_stride; a.kv_ss = kv_seq_stride;
   }
   if (!q || !wg_map || !seq_parts || !out || !workspace) return fail(NKV_ERR_INVALID, "%s: null pointer argument", what);
-  if (reinterpret_cast<uintptr_t>(seq_parts) & 7u) return fail(NKV_ERR_UNSUPPORTED, "%s: seq_parts must be 8-byte aligned", what);
   if (!al16(q) || !al16(workspace)) return fail(NKV_ERR_UNSUPPORTED, "%s: buffers must be 16-byte aligned", what);
   if (total_parts < nseq || total_parts > 65535)
     return fail(NKV_ERR_INVALID, "%s: total_parts %lld outside [nseq, 65535]", what, (long long)total_parts);
