@@ -4963,11 +4963,16 @@ int64_t layers_fwd_bytes(int64_t hq, int64_t n_layers) {
   return n_layers * hq * D / 2 * (int64_t)sizeof(uint64_t) + n_layers * FLAG_COPIES * hq * (int64_t)sizeof(uint32_t);
 }
 
-// Streaming parts per KV head: one workgroup per 8 groups at most, and hkv (parts + 1) workgroups
-// resident at once.
+// Streaming parts per KV head, with hkv (parts + 1) workgroups resident at once.
 int64_t layers_parts(int64_t hkv, int64_t groups, int resident) {
   const int64_t fit = resident / std::max<int64_t>(1, hkv) - 1;
-  return std::min<int64_t>(std::min<int64_t>(fit, WTS), std::max<int64_t>(1, cdiv(groups, 8)));
+  // Four groups per workgroup up to 16 of them, beyond that eight (one per wave). A workgroup's share of a
+  // short prefix is a chain of latencies, and half as many groups in it gain more than the merge of
+  // twice the partials costs: 8 KV heads, per layer with eight / four groups: per-token format, 488
+  // tokens 9.19 / 7.49 us, 2000 9.22 / 7.76, 4000 9.34 / 8.01; int8t64 10.50 / 10.04, 10.73 / 10.34, 10.83 /
+  // 10.84. At 8000 tokens 16 workgroups and 31 take the same (9.81 and 9.92, 11.1 and 11.7).
+  const int64_t parts = std::max(cdiv(groups, 8), std::min<int64_t>(cdiv(groups, 4), 16));
+  return std::min<int64_t>(std::min<int64_t>(fit, WTS), std::max<int64_t>(1, parts));
 }
 
 bool al8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
