@@ -119,17 +119,6 @@ int nkv_attn_decode_t64(const uint16_t* q, const uint8_t* kq, const uint16_t* km
                         float* lse_out, void* workspace, int64_t workspace_bytes,
                         int64_t n_parts, void* stream);
 
-/* The same without a ring, for a workspace that is zero-filled before its first use and used by one
- * stream's decode calls alone (every call leaves the partials it used at zero): one launch, in which one
- * workgroup per KV head merges the parts as they arrive (up to 64 parts and 64 KV heads; two launches
- * beyond). The same bits for the same n_parts. */
-int nkv_attn_decode_zeroed_t64(const uint16_t* q, const uint8_t* kq, const uint16_t* kmn, const uint16_t* kst,
-                               const uint8_t* vq, const uint16_t* vmn, const uint16_t* vst, int64_t hq,
-                               int64_t hkv, int64_t head_dim, int64_t capacity, int64_t used,
-                               int64_t prefix_groups, const int64_t* used_dev, const int64_t* prefix_groups_dev,
-                               uint16_t* out, float* lse_out, void* workspace, int64_t workspace_bytes,
-                               int64_t n_parts, void* stream);
-
 /* Bytes of `workspace` that nkv_attn_decode_t64 / nkv_decode_step_t64 need. */
 int64_t nkv_attn_workspace_bytes(int64_t hkv, int64_t hq, int64_t n_parts);
 
@@ -330,12 +319,6 @@ int nkv_dequantize_tok(const int8_t* codes, int64_t codes_row_stride, const uint
  * when non-NULL). Same launches, q / out / lse / workspace / n_parts contract as
  * nkv_attn_decode_t64 (the counterpart of src/nova/kvattn.py:281-427 for this format). */
 int nkv_attn_decode_tok(const uint16_t* q, const int8_t* kq, const uint16_t* ksc, const int8_t* vq,
-                        const uint16_t* vsc, int64_t hq, int64_t hkv, int64_t head_dim,
-                        int64_t capacity, int64_t used, const int64_t* used_dev, uint16_t* out,
-                        float* lse_out, void* workspace, int64_t workspace_bytes, int64_t n_parts,
-                        void* stream);
-/* nkv_attn_decode_tok as nkv_attn_decode_zeroed_t64: one launch, for a zero-filled workspace of one stream. */
-int nkv_attn_decode_zeroed_tok(const uint16_t* q, const int8_t* kq, const uint16_t* ksc, const int8_t* vq,
                         const uint16_t* vsc, int64_t hq, int64_t hkv, int64_t head_dim,
                         int64_t capacity, int64_t used, const int64_t* used_dev, uint16_t* out,
                         float* lse_out, void* workspace, int64_t workspace_bytes, int64_t n_parts,

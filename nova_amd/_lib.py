@@ -63,8 +63,6 @@ SIGNATURES = {
     "nkv_quantize_tok": (c_int, [P, c_int, I64, I64, I64, I64, P, I64, P, I64, P]),
     "nkv_dequantize_tok": (c_int, [P, I64, P, I64, I64, I64, I64, P, c_int, I64, P]),
     "nkv_attn_decode_tok": (c_int, [P, P, P, P, P, I64, I64, I64, I64, I64, P, P, P, P, I64, I64, P]),
-    "nkv_attn_decode_zeroed_tok": (c_int, [P, P, P, P, P, I64, I64, I64, I64, I64, P, P, P, P, I64, I64, P]),
-    "nkv_attn_decode_zeroed_t64": (c_int, [P, P, P, P, P, P, P, I64, I64, I64, I64, I64, I64, P, P, P, P, P, I64, I64, P]),
     "nkv_append_tok": (c_int, [P, P, I64, P, P, P, P, P, P, I64, I64, I64, P]),
     "nkv_decode_step_tok": (c_int, _STEP_TOK),
     "nkv_decode_step_partials_tok": (c_int, _STEP_TOK),
@@ -230,20 +228,7 @@ def workspace(device: torch.device, nbytes: int, kind: str = "scratch", zero: bo
     return w
 
 
-_STREAM_WORKSPACES = 64  # streams that get a workspace of their own
-
-
-def stream_workspace(device: torch.device, nbytes: int, kind: str, stream: int) -> torch.Tensor | None:
-    """A zero-filled workspace that only calls on ``stream`` use, or None (use :func:`workspace`):
-    under graph capture, whose replays may run on any stream, and for a 65th stream. Where it grows,
-    the shared workspace of ``kind`` grows with it, so that a capture finds one."""
-    if torch.cuda.is_current_stream_capturing():
-        return None
-    key = f"{kind}/{stream}"
-    w = _WORKSPACES.get(f"{device}/{key}")
-    if w is None or w.numel() < nbytes:
-        if w is None and sum(k.startswith(f"{device}/{kind}/") for k in list(_WORKSPACES)) >= _STREAM_WORKSPACES:
-            return None
-        workspace(device, nbytes, kind)
-        w = workspace(device, nbytes, key)
-    return w
+def scratch(device: torch.device, nbytes: int) -> torch.Tensor:
+    """Uninitialized memory for the launches of one call on the current stream: torch's allocator gives it
+    to that stream's later work only, so calls on several streams or threads do not share it."""
+    return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)

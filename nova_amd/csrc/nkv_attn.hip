@@ -4050,15 +4050,15 @@ extern "C" int64_t nkv_attn_workspace_bytes(int64_t hkv, int64_t hq, int64_t n_p
 extern "C" int64_t nkv_attn_default_parts(int64_t hkv, int64_t groups) { return default_parts(hkv, groups); }
 extern "C" int64_t nkv_attn_step_parts(int64_t hkv, int64_t groups) { return step_parts(hkv, groups); }
 
-// `zeroed`: the workspace is zero-filled and this launch's alone, so part 0 of each head merges as the
-// parts arrive (as the fused step does) and no tail launch follows.
-static int attn_decode_t64(const uint16_t* q, const uint8_t* kq, const uint16_t* kmn, const uint16_t* kst,
-                           const uint8_t* vq, const uint16_t* vmn, const uint16_t* vst, int64_t hq, int64_t hkv,
-                           int64_t head_dim, int64_t capacity, int64_t used, int64_t prefix_groups,
-                           const int64_t* used_dev, const int64_t* prefix_groups_dev, const uint16_t* tail_k,
-                           const uint16_t* tail_v, const int64_t* written_dev, const int64_t* first_dev,
-                           uint16_t* out, float* lse_out, void* workspace, int64_t workspace_bytes,
-                           int64_t n_parts, void* stream, bool zeroed) {
+extern "C" int nkv_attn_decode_t64(const uint16_t* q, const uint8_t* kq, const uint16_t* kmn,
+                                   const uint16_t* kst, const uint8_t* vq, const uint16_t* vmn,
+                                   const uint16_t* vst, int64_t hq, int64_t hkv, int64_t head_dim,
+                                   int64_t capacity, int64_t used, int64_t prefix_groups,
+                                   const int64_t* used_dev, const int64_t* prefix_groups_dev,
+                                   const uint16_t* tail_k, const uint16_t* tail_v,
+                                   const int64_t* written_dev, const int64_t* first_dev,
+                                   uint16_t* out, float* lse_out, void* workspace,
+                                   int64_t workspace_bytes, int64_t n_parts, void* stream) {
   set_error("");
   if (int rc = check_heads(hq, hkv, head_dim)) return rc;
   if (capacity <= 0) return fail(NKV_ERR_INVALID, "capacity must be positive");
@@ -4089,34 +4089,7 @@ static int attn_decode_t64(const uint16_t* q, const uint8_t* kq, const uint16_t*
   a.tail_mode = tail_k ? TAIL_SCALARS : TAIL_NONE;
   a.sl2 = LOG2E / sqrtf((float)head_dim);
   a.out = out; a.lse = lse_out; a.ws = static_cast<float*>(workspace);
-  return launch_attn(a, n_parts, workspace_bytes, static_cast<hipStream_t>(stream), "attn_decode_t64",
-                     LAUNCH_PREFIX | LAUNCH_TAIL, zeroed);
-}
-
-extern "C" int nkv_attn_decode_t64(const uint16_t* q, const uint8_t* kq, const uint16_t* kmn,
-                                   const uint16_t* kst, const uint8_t* vq, const uint16_t* vmn,
-                                   const uint16_t* vst, int64_t hq, int64_t hkv, int64_t head_dim,
-                                   int64_t capacity, int64_t used, int64_t prefix_groups,
-                                   const int64_t* used_dev, const int64_t* prefix_groups_dev,
-                                   const uint16_t* tail_k, const uint16_t* tail_v,
-                                   const int64_t* written_dev, const int64_t* first_dev,
-                                   uint16_t* out, float* lse_out, void* workspace,
-                                   int64_t workspace_bytes, int64_t n_parts, void* stream) {
-  return attn_decode_t64(q, kq, kmn, kst, vq, vmn, vst, hq, hkv, head_dim, capacity, used, prefix_groups, used_dev,
-                         prefix_groups_dev, tail_k, tail_v, written_dev, first_dev, out, lse_out, workspace,
-                         workspace_bytes, n_parts, stream, false);
-}
-
-extern "C" int nkv_attn_decode_zeroed_t64(const uint16_t* q, const uint8_t* kq, const uint16_t* kmn,
-                                          const uint16_t* kst, const uint8_t* vq, const uint16_t* vmn,
-                                          const uint16_t* vst, int64_t hq, int64_t hkv, int64_t head_dim,
-                                          int64_t capacity, int64_t used, int64_t prefix_groups,
-                                          const int64_t* used_dev, const int64_t* prefix_groups_dev,
-                                          uint16_t* out, float* lse_out, void* workspace,
-                                          int64_t workspace_bytes, int64_t n_parts, void* stream) {
-  return attn_decode_t64(q, kq, kmn, kst, vq, vmn, vst, hq, hkv, head_dim, capacity, used, prefix_groups, used_dev,
-                         prefix_groups_dev, nullptr, nullptr, nullptr, nullptr, out, lse_out, workspace,
-                         workspace_bytes, n_parts, stream, true);
+  return launch_attn(a, n_parts, workspace_bytes, static_cast<hipStream_t>(stream), "attn_decode_t64");
 }
 
 extern "C" int nkv_append_t64(const uint16_t* k_new, const uint16_t* v_new, int64_t kv_head_stride,
@@ -4443,10 +4416,10 @@ static int check_tok_cache(const char* what, int64_t capacity, const void* kq, c
   return NKV_OK;
 }
 
-static int attn_decode_tok(const uint16_t* q, const int8_t* kq, const uint16_t* ksc, const int8_t* vq,
-                           const uint16_t* vsc, int64_t hq, int64_t hkv, int64_t head_dim, int64_t capacity,
-                           int64_t used, const int64_t* used_dev, uint16_t* out, float* lse_out, void* workspace,
-                           int64_t workspace_bytes, int64_t n_parts, void* stream, bool zeroed) {
+extern "C" int nkv_attn_decode_tok(const uint16_t* q, const int8_t* kq, const uint16_t* ksc, const int8_t* vq,
+                                   const uint16_t* vsc, int64_t hq, int64_t hkv, int64_t head_dim, int64_t capacity,
+                                   int64_t used, const int64_t* used_dev, uint16_t* out, float* lse_out,
+                                   void* workspace, int64_t workspace_bytes, int64_t n_parts, void* stream) {
   set_error("");
   if (int rc = check_heads(hq, hkv, head_dim)) return rc;
   if (int rc = check_tok_cache("attn_decode_tok", capacity, kq, ksc, vq, vsc)) return rc;
@@ -4463,25 +4436,7 @@ static int attn_decode_tok(const uint16_t* q, const int8_t* kq, const uint16_t* 
   a.tail_mode = TAIL_NONE;
   a.sl2 = LOG2E / sqrtf((float)head_dim);
   a.out = out; a.lse = lse_out; a.ws = static_cast<float*>(workspace);
-  return launch_attn(a, n_parts, workspace_bytes, static_cast<hipStream_t>(stream), "attn_decode_tok",
-                     LAUNCH_PREFIX | LAUNCH_TAIL, zeroed);
-}
-
-extern "C" int nkv_attn_decode_tok(const uint16_t* q, const int8_t* kq, const uint16_t* ksc, const int8_t* vq,
-                                   const uint16_t* vsc, int64_t hq, int64_t hkv, int64_t head_dim, int64_t capacity,
-                                   int64_t used, const int64_t* used_dev, uint16_t* out, float* lse_out,
-                                   void* workspace, int64_t workspace_bytes, int64_t n_parts, void* stream) {
-  return attn_decode_tok(q, kq, ksc, vq, vsc, hq, hkv, head_dim, capacity, used, used_dev, out, lse_out, workspace,
-                         workspace_bytes, n_parts, stream, false);
-}
-
-extern "C" int nkv_attn_decode_zeroed_tok(const uint16_t* q, const int8_t* kq, const uint16_t* ksc, const int8_t* vq,
-                                          const uint16_t* vsc, int64_t hq, int64_t hkv, int64_t head_dim,
-                                          int64_t capacity, int64_t used, const int64_t* used_dev, uint16_t* out,
-                                          float* lse_out, void* workspace, int64_t workspace_bytes, int64_t n_parts,
-                                          void* stream) {
-  return attn_decode_tok(q, kq, ksc, vq, vsc, hq, hkv, head_dim, capacity, used, used_dev, out, lse_out, workspace,
-                         workspace_bytes, n_parts, stream, true);
+  return launch_attn(a, n_parts, workspace_bytes, static_cast<hipStream_t>(stream), "attn_decode_tok");
 }
 
 extern "C" int nkv_append_tok(const uint16_t* k_new, const uint16_t* v_new, int64_t kv_head_stride, int8_t* kq,

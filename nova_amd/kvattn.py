@@ -214,30 +214,15 @@ def int8_attn_decode(
             raise ValueError("under graph capture int8_attn_decode needs scratch=(pm, pl, pa): "
                              "no workspace may be allocated inside a graph")
         parts = _parts_fitting(geo.hkv, geo.hq, groups, None)
-        ws = None
+        ws = _lib.scratch(q.device, int(_lib.load().nkv_attn_workspace_bytes(geo.hkv, geo.hq, parts)))
+        ws_bytes = ws.numel()
     if group != GROUP_T or d != HEAD_DIM:
         raise NotImplementedError(f"the HIP kernels read {GROUP_T}-token rulers at head_dim {HEAD_DIM} "
                                   f"(group={group}, head_dim={d})")
-    stream = _lib.stream_ptr(q.device)
-    if ws is None:
-        need = int(_lib.load().nkv_attn_workspace_bytes(geo.hkv, geo.hq, parts))
-        ws = _lib.stream_workspace(q.device, need, "decode", stream)
-        if ws is None:
-            ws = _lib.workspace(q.device, need)
-            ws_bytes = ws.numel()
-        else:
-            ws_bytes = 0
-    if not ws_bytes:
-        # zero-filled and this stream's own: the launch that writes the partials merges them
-        _lib.call("nkv_attn_decode_zeroed_t64", q.data_ptr(), kq.data_ptr(), kmn.data_ptr(), kst.data_ptr(),
-                  vq.data_ptr(), vmn.data_ptr(), vst.data_ptr(), geo.hq, geo.hkv, d, geo.length, used_host, pg_host,
-                  _lib.ptr(used_t), _lib.ptr(prefix_groups_t), out.data_ptr(), _lib.ptr(lse_out), ws.data_ptr(),
-                  ws.numel(), parts, stream)
-        return out
     _lib.call("nkv_attn_decode_t64", q.data_ptr(), kq.data_ptr(), kmn.data_ptr(), kst.data_ptr(), vq.data_ptr(),
               vmn.data_ptr(), vst.data_ptr(), geo.hq, geo.hkv, d, geo.length, used_host, pg_host,
               _lib.ptr(used_t), _lib.ptr(prefix_groups_t), None, None, None, None, out.data_ptr(),
-              _lib.ptr(lse_out), ws.data_ptr(), ws_bytes, parts, stream)
+              _lib.ptr(lse_out), ws.data_ptr(), ws_bytes, parts, _lib.stream_ptr(q.device))
     return out
 
 

@@ -108,20 +108,18 @@ def int8_tok_attn_decode(q: torch.Tensor, kq: torch.Tensor, ksc: torch.Tensor, v
     if out is None:
         out = torch.empty_like(q)
     groups = cap // GROUP
-    entry, stream = "nkv_attn_decode_tok", _lib.stream_ptr(q.device)
     if scratch is None:
         parts = int(n_splits) if n_splits else int(_lib.load().nkv_attn_step_parts(hkv, groups))
         need = int(_lib.load().nkv_attn_workspace_bytes(hkv, hq, parts))
-        scratch = _lib.stream_workspace(q.device, need, "decode", stream)
-        if scratch is None:
-            scratch = _lib.workspace(q.device, need, "decode")
-        else:  # zero-filled and this stream's own: the launch that writes the partials merges them
-            entry = "nkv_attn_decode_zeroed_tok"
+        scratch = _lib.workspace(q.device, need, "decode")  # (a capture takes the one that a call before it left)
+        if not torch.cuda.is_current_stream_capturing():
+            scratch = _lib.scratch(q.device, need)
     else:
         parts = int(n_splits) if n_splits else _parts(hkv, hq, groups, scratch.numel() * scratch.element_size())
-    _lib.call(entry, q.data_ptr(), kq.data_ptr(), ksc.data_ptr(), vq.data_ptr(), vsc.data_ptr(),
+    _lib.call("nkv_attn_decode_tok", q.data_ptr(), kq.data_ptr(), ksc.data_ptr(), vq.data_ptr(), vsc.data_ptr(),
               hq, hkv, d, cap, 0 if used_t is not None else used, _lib.ptr(used_t), out.data_ptr(),
-              _lib.ptr(lse_out), scratch.data_ptr(), scratch.numel() * scratch.element_size(), parts, stream)
+              _lib.ptr(lse_out), scratch.data_ptr(), scratch.numel() * scratch.element_size(), parts,
+              _lib.stream_ptr(q.device))
     return out
 
 

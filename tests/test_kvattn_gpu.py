@@ -287,37 +287,28 @@ def test_scores_that_move_the_softmax_reference(profile):
     assert_ulp_or_abs(npy(got)[0, :, 0], want, 2.0, 1e-5, profile)
 
 
-@pytest.mark.parametrize("hq,hkv,used", [(32, 8, 1), (32, 8, 63), (32, 8, 2048), (16, 2, 640), (16, 16, 129), (8, 1, 5000), (32, 2, 65)])
-def test_one_launch_decode_matches_the_two_launches(hq, hkv, used):
-    """Without a scratch of the caller's the decode merges its parts in the launch that writes them:
-    the same bits as the two launches on a caller's scratch with as many parts, call after call and
-    after a call with other parts on the same workspace, on two streams."""
-    from nova_amd import _lib
+@pytest.mark.parametrize("tok", [False, True])
+def test_decode_calls_overlap_on_many_streams(tok):
+    """Eight streams of 64 KV heads at once: calls without a caller's scratch share nothing, and no
+    workgroup waits for one of another launch, so every call's bits are those of a call alone."""
     from nova_amd.kvattn import int8_attn_decode, pack_int8_kv
     from nova_amd.kvtok import int8_tok_attn_decode, quantize_tok
 
-    print(f"case hq={hq} hkv={hkv} used={used}", flush=True)
-    cap = -(-used // 64) * 64
-    k, v = randn((1, hkv, cap, 128), used).cuda(), randn((1, hkv, cap, 128), used + 1).cuda()
-    q = randn((1, hq, 1, 128), used + 2).cuda()
-    packed, tok = pack_int8_kv(k, v), (*quantize_tok(k), *quantize_tok(v))
-    parts = int(_lib.load().nkv_attn_step_parts(hkv, cap // 64))
-    want = torch.empty_like(q)
-    lse, wlse = (torch.zeros(1, hq, device="cuda") for _ in range(2))
-    ws = torch.zeros(int(_lib.load().nkv_attn_workspace_bytes(hkv, hq, parts)), dtype=torch.uint8, device="cuda")
-    _lib.call("nkv_attn_decode_t64", q.data_ptr(), *(t.data_ptr() for t in packed), hq, hkv, 128, cap, used, -1, None,
-              None, None, None, None, None, want.data_ptr(), wlse.data_ptr(), ws.data_ptr(), ws.numel(), parts,
-              _lib.stream_ptr(q.device))
-    side = torch.cuda.Stream()
-    for i in range(3):
-        assert torch.equal(int8_attn_decode(q, *packed, used=used, lse_out=lse), want) and torch.equal(lse, wlse)
-        int8_attn_decode(q, *packed, used=max(1, used // 3))
-        side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):
-            other = int8_attn_decode(q, *packed, used=used)
-        torch.cuda.current_stream().wait_stream(side)
-        assert torch.equal(other, want)
-    want = int8_tok_attn_decode(q, *tok, used=used, scratch=torch.zeros_like(ws), n_splits=parts).clone()
-    for i in range(2):
-        assert torch.equal(int8_tok_attn_decode(q, *tok, used=used), want)
-        int8_tok_attn_decode(q, *tok, used=max(1, used // 3))
+    heads, cap = 64, 512
+    print(f"case tok={tok}", flush=True)
+    k, v = randn((1, heads, cap, 128), 7).cuda(), randn((1, heads, cap, 128), 8).cuda()
+    q = randn((1, heads, 1, 128), 9).cuda()
+    cache = (*quantize_tok(k), *quantize_tok(v)) if tok else pack_int8_kv(k, v)
+    decode = int8_tok_attn_decode if tok else int8_attn_decode
+    lengths = [512, 65, 300, 1, 448, 129, 64, 511]
+    want = [decode(q, *cache, used=n) for n in lengths]
+    streams = [torch.cuda.Stream() for _ in lengths]
+    torch.cuda.synchronize()
+    got = []
+    for _ in range(4):
+        for s, n in zip(streams, lengths):
+            with torch.cuda.stream(s):
+                got.append(decode(q, *cache, used=n))
+    torch.cuda.synchronize()
+    for i, o in enumerate(got):
+        assert torch.equal(o, want[i % len(want)]), (i, lengths[i % len(lengths)])
