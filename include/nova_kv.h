@@ -596,13 +596,18 @@ int nkv_paged_decode_step_tok(const uint16_t* q, const uint16_t* k_new, const ui
  * `workspace` and a combine kernel merges them (else that launch is left out). splits > 0 bounds
  * the shares to that many per tile; splits <= 0 leaves it to the library.
  * workspace: at least nkv_prefill_workspace_bytes; nkv_prefill_preferred_bytes gives the size at
- * which the work is cut evenly (m_kv: the fp16 tokens, m for nkv_prefill_attn_t64), a smaller one
- * gets the best cut that fits it.
+ * which the work is cut evenly (m_kv: the fp16 tokens, m for nkv_prefill_attn_t64): every workspace of
+ * that size or more gives the same cut and the same bits, a smaller one gets the best cut that fits it.
  */
 int64_t nkv_prefill_workspace_bytes(int64_t hkv, int64_t hq, int64_t m, int64_t splits);
 int64_t nkv_prefill_preferred_bytes(int64_t hkv, int64_t hq, int64_t m, int64_t m_kv, int64_t used, int64_t splits);
 /* The splits value whose nkv_prefill_workspace_bytes a call with `splits` <= 0 needs at least. */
 int64_t nkv_prefill_default_splits(int64_t hkv, int64_t hq, int64_t m, int64_t used);
+/* How a call's work is cut over the workgroups (host only): out[0] 0 at tile boundaries, 1 every tile into
+ * the same number of parts, 2 even shares; then the workgroups and partial slots per KV head, the tiles
+ * that the second launch merges, whether tiles are taken from both ends in turn, and the tiles. */
+int nkv_prefill_cutting(int64_t hkv, int64_t hq, int64_t m, int64_t m_kv, int64_t used, int64_t splits,
+                        int64_t workspace_bytes, int64_t* out);
 int nkv_prefill_attn_t64(const uint16_t* q, const uint16_t* k_chunk, const uint16_t* v_chunk, int64_t m,
                          const uint8_t* kq, const uint16_t* kmn, const uint16_t* kst, const uint8_t* vq,
                          const uint16_t* vmn, const uint16_t* vst, int64_t capacity, int64_t used,

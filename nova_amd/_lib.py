@@ -88,6 +88,7 @@ SIGNATURES = {
                                           P, P, I64, P]),
     "nkv_prefill_workspace_bytes": (I64, [I64, I64, I64, I64]),
     "nkv_prefill_default_splits": (I64, [I64, I64, I64, I64]),
+    "nkv_prefill_cutting": (c_int, [I64, I64, I64, I64, I64, I64, I64, P]),
     "nkv_prefill_preferred_bytes": (I64, [I64, I64, I64, I64, I64, I64]),
     "nkv_prefill_attn_t64": (c_int, [P, P, P, I64, P, P, P, P, P, P, I64, I64, I64, I64, I64, P, P, I64, I64, P]),
     "nkv_prefill_attn_hist_t64": (c_int, [P, I64, P, P, I64, I64, P, P, P, P, P, P, I64, I64, I64, I64, I64, P, P,

@@ -36,6 +36,7 @@
 #include "nkv_common.h"
 
 #include <algorithm>
+#include <iterator>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -4780,6 +4781,16 @@ static void prefill_plan(PrefillArgs& a, int64_t splits, int64_t avail_slots, Pr
   }
 }
 
+// The plan of a call: the shape's own where its slots fit the workspace, so that the same call gives the
+// same bits in every workspace from nkv_prefill_preferred_bytes on; in a smaller one the best that fits.
+static void prefill_plan_in(PrefillArgs& a, int64_t splits, int64_t workspace_bytes, PrefillPlan& p) {
+  prefill_plan(a, splits, INT64_MAX, p);
+  const int64_t avail = workspace_bytes / prefill_slot_bytes(a);
+  if (p.slots <= avail) return;
+  p = PrefillPlan{};
+  prefill_plan(a, splits, avail, p);
+}
+
 static void prefill_shape(PrefillArgs& a, int64_t hkv, int64_t hq, int64_t m, int64_t m_kv, int64_t used) {
   a.M = (int)m; a.hq = (int)hq; a.hkv = (int)hkv; a.gq = (int)(hq / hkv);
   a.tiles = (int)cdiv(m * a.gq, PF_ROWS);
@@ -4800,6 +4811,22 @@ extern "C" int64_t nkv_prefill_preferred_bytes(int64_t hkv, int64_t hq, int64_t 
   const int64_t least = nkv_prefill_workspace_bytes(
       hkv, hq, m, splits > 0 ? splits : nkv_prefill_default_splits(hkv, hq, m, used));
   return std::max<int64_t>(least, p.slots * prefill_slot_bytes(a));
+}
+
+extern "C" int nkv_prefill_cutting(int64_t hkv, int64_t hq, int64_t m, int64_t m_kv, int64_t used, int64_t splits,
+                                   int64_t workspace_bytes, int64_t* out) {
+  set_error("");
+  if (int rc = check_heads(hq, hkv, D)) return rc;
+  if (m <= 0 || m > (1 << 20) || m_kv < m || m_kv > (1 << 24) || used < 0 || used % GT || workspace_bytes < 0 || !out)
+    return fail(NKV_ERR_INVALID, "prefill_cutting: m=%lld m_kv=%lld used=%lld workspace of %lld bytes", (long long)m,
+                (long long)m_kv, (long long)used, (long long)workspace_bytes);
+  PrefillArgs a{};
+  prefill_shape(a, hkv, hq, m, m_kv, used);
+  PrefillPlan p;
+  prefill_plan_in(a, splits, workspace_bytes, p);
+  const int64_t v[] = {p.two_slots ? 2 : p.slots ? 1 : 0, p.shares, p.slots, p.merges, p.zigzag, a.tiles};
+  std::copy(std::begin(v), std::end(v), out);
+  return NKV_OK;
 }
 
 static int prefill_attn(const char* what, const uint16_t* q, int64_t q_ts, int64_t q_hs, int64_t m, const uint16_t* k16, const uint16_t* v16,
@@ -4838,7 +4865,7 @@ static int prefill_attn(const char* what, const uint16_t* q, int64_t q_ts, int64
   a.sl2 = LOG2E / sqrtf((float)head_dim);
   a.ws = static_cast<float*>(workspace); a.out = out;
   PrefillPlan p;
-  prefill_plan(a, splits, workspace_bytes / prefill_slot_bytes(a), p);
+  prefill_plan_in(a, splits, workspace_bytes, p);
   a.shares = p.shares; a.slots = p.slots; a.two_slots = p.two_slots;
   for (int w = 0; w <= p.shares; ++w) a.cut[w] = p.cut[w];
   hipStream_t s = static_cast<hipStream_t>(stream);

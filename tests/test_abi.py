@@ -257,3 +257,25 @@ def test_step_parts_stay_within_the_workspace_rules(lib):
             assert least <= n <= max(1, 256 // hkv), (hkv, groups, n)
             assert n == least or n <= min(groups, 32), (hkv, groups, n)
     assert lib.nkv_attn_step_parts(8, 4) == 4 and lib.nkv_attn_step_parts(2, 8) == 1
+
+
+def _cutting(lib, hq, hkv, m, used, hist=0, splits=0, nbytes=None):
+    """(kind, shares, slots, merges, zigzag, tiles) of a prefill call."""
+    if nbytes is None:
+        nbytes = lib.nkv_prefill_preferred_bytes(hkv, hq, m, m + hist, used, splits)
+    out = (ctypes.c_int64 * 6)()
+    assert lib.nkv_prefill_cutting(hkv, hq, m, m + hist, used, splits, nbytes, out) == 0, lib.nkv_last_error()
+    return tuple(out)
+
+
+def test_prefill_cut_depends_on_the_shape_alone(lib):
+    """Every workspace from the preferred size on gives the same cut, so a call's bits do not follow the
+    sizes of the calls before it (some of these shapes have a dearer plan that needs more slots)."""
+    shapes = [(64, 8, 116, 448, 0), (40, 8, 314, 256, 0), (32, 8, 512, 16384, 0), (32, 8, 2048, 8192, 0)]
+    shapes += [(hq, hkv, m, 64 * g, hist) for hq, hkv in ((32, 8), (8, 8), (16, 2), (28, 4), (64, 8), (8, 1))
+               for m in (1, 7, 40, 87, 143, 314, 780, 1999) for g in (0, 1, 7, 30, 256) for hist in (0, 200)]
+    for hq, hkv, m, used, hist in shapes:
+        best = lib.nkv_prefill_preferred_bytes(hkv, hq, m, m + hist, used, 0)
+        want = _cutting(lib, hq, hkv, m, used, hist)
+        for nbytes in (best + 1, best + (1 << 20), 2 * best, best + (1 << 30)):
+            assert _cutting(lib, hq, hkv, m, used, hist, nbytes=nbytes) == want, (hq, hkv, m, used, hist, nbytes)
