@@ -598,6 +598,7 @@ int nkv_paged_decode_step_tok(const uint16_t* q, const uint16_t* k_new, const ui
  * workspace: at least nkv_prefill_workspace_bytes; nkv_prefill_preferred_bytes gives the size at
  * which the work is cut evenly (m_kv: the fp16 tokens, m for nkv_prefill_attn_t64): every workspace of
  * that size or more gives the same cut and the same bits, a smaller one gets the best cut that fits it.
+ * It holds one call's partials at a time: calls that may overlap (on several streams) need one each.
  */
 int64_t nkv_prefill_workspace_bytes(int64_t hkv, int64_t hq, int64_t m, int64_t splits);
 int64_t nkv_prefill_preferred_bytes(int64_t hkv, int64_t hq, int64_t m, int64_t m_kv, int64_t used, int64_t splits);

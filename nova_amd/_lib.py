@@ -211,8 +211,8 @@ _WORKSPACES: dict[str, torch.Tensor] = {}
 _RETIRED: list[torch.Tensor] = []
 
 
-def workspace(device: torch.device, nbytes: int, kind: str = "scratch", zero: bool = True) -> torch.Tensor:
-    """A cached per-device byte workspace of at least ``nbytes``, zero-filled unless told not to. It grows only
+def workspace(device: torch.device, nbytes: int, kind: str = "scratch") -> torch.Tensor:
+    """A cached per-device, zero-filled byte workspace of at least ``nbytes``. It grows only
     outside graph capture (a capture that needs more raises); the buffer it replaces is kept,
     never freed, because a captured graph may point into it. Callers pass the whole buffer
     (``numel()`` bytes)."""
@@ -224,7 +224,7 @@ def workspace(device: torch.device, nbytes: int, kind: str = "scratch", zero: bo
                                "pass a preallocated scratch buffer")
         if w is not None:
             _RETIRED.append(w)
-        w = (torch.zeros if zero else torch.empty)(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+        w = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _WORKSPACES[key] = w
     return w
 

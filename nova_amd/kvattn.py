@@ -271,7 +271,9 @@ def int8_prefill_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Ten
     ``[1, Hkv, m, 128]`` fp16 (``m >= n``, any head stride) follow them: the first ``m - n`` are an
     fp16 history, the last ``n`` the chunk. Query token ``i`` attends the int8 tokens, the fp16
     history and chunk tokens ``0..i`` — what ``KVInt8Cache.attend_prefill`` computes with SDPA over
-    its fp16 staging (src/nova/kvattn.py:791-815). Returns ``out`` ``[1, Hq, n, 128]`` fp16.
+    its fp16 staging (src/nova/kvattn.py:791-815). ``scratch`` (optional; required under graph capture)
+    holds the partials of one call at a time: calls that may overlap need one each. Returns ``out``
+    ``[1, Hq, n, 128]`` fp16.
     """
     _require_gpu_tensor(query, "query", torch.float16)
     for t, nm in ((kq, "kq"), (vq, "vq")):
@@ -315,7 +317,7 @@ def _prefill_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
         if _capturing():
             raise ValueError("under graph capture int8_prefill_attend needs a large enough scratch")
         need = max(need, int(lib.nkv_prefill_preferred_bytes(hkv, hq, n, m, used, splits)))
-        scratch = _lib.workspace(query.device, need, "prefill", zero=False)  # (written before it is read)
+        scratch = _lib.scratch(query.device, need)
     _lib.call("nkv_prefill_attn_strided_t64", query.data_ptr(), query.stride(2), query.stride(1), n, key.data_ptr(), value.data_ptr(), m,
               key.stride(1), kq.data_ptr(), kmn.data_ptr(), kst.data_ptr(), vq.data_ptr(), vmn.data_ptr(),
               vst.data_ptr(), cap, used, hq, hkv, d, out.data_ptr(), scratch.data_ptr(),

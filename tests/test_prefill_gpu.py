@@ -192,3 +192,23 @@ def test_prefill_cuttings(hq, hkv, used, m, hist, least):
     err = np.abs(npy(got)[0].astype(np.float64) - want)
     assert err.max() <= 2e-3, f"max abs {err.max():.2e}"
     assert err.mean() <= 1.5e-4, f"mean abs {err.mean():.2e}"
+
+
+def test_prefill_calls_overlap_on_streams():
+    """Calls with cut tiles on four streams at once, of different shapes, each with the bits of a call
+    alone: no two calls share the memory of their partials."""
+    from nova_amd.kvattn import int8_prefill_attend
+
+    cases = [_case(32, 8, used, m, seed=400 + i) for i, (used, m) in enumerate([(4096, 300), (2048, 512), (1024, 70), (0, 900)])]
+    lengths = [4096, 2048, 1024, 0]
+    want = [int8_prefill_attend(q, k, v, *p, used=u) for (q, k, v, p), u in zip(cases, lengths)]
+    streams = [torch.cuda.Stream() for _ in cases]
+    torch.cuda.synchronize()
+    got = []
+    for _ in range(6):
+        for s, (q, k, v, p), u in zip(streams, cases, lengths):
+            with torch.cuda.stream(s):
+                got.append(int8_prefill_attend(q, k, v, *p, used=u))
+    torch.cuda.synchronize()
+    for i, o in enumerate(got):
+        assert torch.equal(o, want[i % 4]), f"case {i % 4}, round {i // 4}"
