@@ -283,9 +283,17 @@ def int8_prefill_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Ten
     return _prefill_attend(query, key, value, kq, kmn, kst, vq, vmn, vst, used, out, scratch, splits)
 
 
+def _row_strides(x: torch.Tensor) -> tuple[int, int]:
+    """Token and head stride of ``x`` ``[1, heads, n, D]``; that of a single token or head, which no row
+    is reached by and torch leaves at any value, as in a contiguous tensor."""
+    _, heads, n, d = x.shape
+    return (x.stride(2) if n > 1 else d), (x.stride(1) if heads > 1 else n * d)
+
+
 def _rows_aligned(x: torch.Tensor) -> bool:
     """Rows of 128 halves that the kernels can read in place, whatever the head and token strides."""
-    return x.stride(3) == 1 and x.stride(1) % 8 == 0 and x.stride(2) % 8 == 0 and x.data_ptr() % 16 == 0
+    token, head = _row_strides(x)
+    return x.stride(3) == 1 and token % 8 == 0 and head % 8 == 0 and x.data_ptr() % 16 == 0
 
 
 def _prefill_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, kq: torch.Tensor, kmn: torch.Tensor,
@@ -318,7 +326,7 @@ def _prefill_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
             raise ValueError("under graph capture int8_prefill_attend needs a large enough scratch")
         need = max(need, int(lib.nkv_prefill_preferred_bytes(hkv, hq, n, m, used, splits)))
         scratch = _lib.scratch(query.device, need)
-    _lib.call("nkv_prefill_attn_strided_t64", query.data_ptr(), query.stride(2), query.stride(1), n, key.data_ptr(), value.data_ptr(), m,
+    _lib.call("nkv_prefill_attn_strided_t64", query.data_ptr(), *_row_strides(query), n, key.data_ptr(), value.data_ptr(), m,
               key.stride(1), kq.data_ptr(), kmn.data_ptr(), kst.data_ptr(), vq.data_ptr(), vmn.data_ptr(),
               vst.data_ptr(), cap, used, hq, hkv, d, out.data_ptr(), scratch.data_ptr(),
               scratch.numel() * scratch.element_size(), max(0, splits), _lib.stream_ptr(query.device))
@@ -579,8 +587,8 @@ class KVInt8Cache:
         k16, v16 = self._chunk_tokens(layer, n)
         if n and key.device == value.device == self.pos.device and _rows_aligned(key) and _rows_aligned(value):
             i = layer
-            _lib.call("nkv_prefill_land_t64", key.data_ptr(), value.data_ptr(), key.stride(2), key.stride(1),
-                      value.stride(2), value.stride(1), n, start, self.num_kv_heads, self.head_dim, self.max_len,
+            _lib.call("nkv_prefill_land_t64", key.data_ptr(), value.data_ptr(), *_row_strides(key),
+                      *_row_strides(value), n, start, self.num_kv_heads, self.head_dim, self.max_len,
                       k16.data_ptr(), v16.data_ptr(), self.kq[i].data_ptr(), self.kmn[i].data_ptr(),
                       self.kst[i].data_ptr(), self.vq[i].data_ptr(), self.vmn[i].data_ptr(), self.vst[i].data_ptr(),
                       self.tail_k[i].data_ptr(), self.tail_v[i].data_ptr(), _lib.stream_ptr(self.pos.device))

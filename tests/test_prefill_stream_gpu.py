@@ -189,3 +189,34 @@ def test_streamed_chunk_read_in_place(chunks):
         want = want or got
         for i, (x, y) in enumerate(zip(got, want)):
             assert torch.equal(x, y), f"{name}: tensor {i}"
+
+
+def test_single_token_and_single_head_strides():
+    """The stride of a dimension of size 1 is never used: torch calls such a tensor contiguous at any value
+    of it, so a one-token last chunk of a projection whose width is not a multiple of 8, and a query of one
+    head, attend as their contiguous copies do."""
+    from nova_amd.kvattn import int8_prefill_attend, pack_int8_kv
+
+    total, width = 65, HQ * D + 4
+    k, v = (randn((1, H_KV, total, D), 510 + i, 1.0).cuda() for i in range(2))
+    rows = torch.zeros(1, total, width, dtype=torch.float16, device="cuda")
+    rows[..., :HQ * D] = randn((1, total, HQ * D), 512, 1.0).cuda()
+    q = rows[..., :HQ * D].unflatten(-1, (HQ, D)).transpose(1, 2)
+    last = q[:, :, 64:]
+    assert last.is_contiguous() and last.stride(2) == width and last.data_ptr() % 16 == 0
+    outs = []
+    for one in (last, torch.empty(1, HQ, 1, D, dtype=q.dtype, device="cuda").copy_(last)):
+        c, _ = _caches(total)
+        c.begin_prefill(total, stream_chunk=64)
+        c.set_prefill_pos(0)
+        c.update(k[:, :, :64], v[:, :, :64], 0)
+        c.attend_prefill(q[:, :, :64].contiguous(), 0)
+        c.set_prefill_pos(64)
+        c.update(k[:, :, 64:], v[:, :, 64:], 0)
+        outs.append(c.attend_prefill(one, 0))
+    packed = pack_int8_kv(k[:, :1, :64].contiguous(), v[:, :1, :64].contiguous())
+    head = torch.as_strided(rows, (1, 1, 9, D), (1, width - 1, D, 1))
+    for one in (head, torch.empty(1, 1, 9, D, dtype=q.dtype, device="cuda").copy_(head)):
+        assert one.is_contiguous()
+        outs.append(int8_prefill_attend(one, k[:, :1, :9].contiguous(), v[:, :1, :9].contiguous(), *packed, 64))
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[2], outs[3])
