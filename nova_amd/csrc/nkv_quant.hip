@@ -668,6 +668,13 @@ static void launch_rows(K one, K four, bool few, dim3 grid, hipStream_t s, const
   hipLaunchKernelGGL(few ? one : four, grid, dim3(256), 0, s, a);
 }
 
+// The kernels that take tiles in turns count them in 32 bits, one stride of the grid (at most 2^22 tiles)
+// past the last: below 2^31 that sum does not wrap, and every workgroup leaves its loop.
+static int check_items(const char* what, int64_t items) {
+  if (items < (int64_t(1) << 31)) return NKV_OK;
+  return fail(NKV_ERR_UNSUPPORTED, "%s: %lld tiles (fewer than 2^31)", what, (long long)items);
+}
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace nkv
@@ -700,7 +707,7 @@ extern "C" int nkv_quantize_int8(const void* x, int x_dtype, int64_t x_row_strid
     QuantTokArgs a{x, x_row_stride, rows, n, dim, gs, cdiv(n, gs), cdiv(dim, 128), codes,
                    codes_row_stride, mins, steps, scale_row_stride, 0};
     a.items = rows * a.ngroups * a.nchunks;
-    if (a.items >= (int64_t(1) << 32)) return fail(NKV_ERR_UNSUPPORTED, "quantize: %lld groups", (long long)a.items);
+    if (int rc = check_items("quantize", a.items)) return rc;
     if (x_dtype == NKV_F16) launch_quant_token<NKV_F16>(a, s);
     else if (x_dtype == NKV_BF16) launch_quant_token<NKV_BF16>(a, s);
     else launch_quant_token<NKV_F32>(a, s);
@@ -746,6 +753,7 @@ extern "C" int nkv_paged_quantize_t64(const void* x, int x_dtype, int64_t x_head
   QuantTokArgs a{x, x_head_stride, hkv, n, 128, 64, n / 64, 1, nullptr, 0, nullptr, nullptr, 0, 0,
                  pages, table_row, first_group, num_pages, which};
   a.items = hkv * a.ngroups;
+  if (int rc = check_items("paged_quantize", a.items)) return rc;
   const dim3 grid((unsigned)std::min<int64_t>(a.items, 1 << 20)), block(256);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (x_dtype == NKV_F16) hipLaunchKernelGGL((quant_token_kernel<NKV_F16, 4, 4, true>), grid, block, 0, s, a);
@@ -808,7 +816,8 @@ extern "C" int nkv_dequantize_int8(const uint8_t* codes, int64_t codes_row_strid
   DequantArgs a{codes, codes_row_stride, mins, steps, scale_row_stride, rows, n, dim, g, axis,
                 out, out_row_stride, rows * cdiv(n, few_rows(rows * n, out_dtype) ? 16 : 64) * cdiv(dim, 128),
                 aligned16(mins) && aligned16(steps) && scale_row_stride % 8 == 0};
-  if (a.items >= (int64_t(1) << 31) || n >= (int64_t(1) << 32) || dim >= (int64_t(1) << 32))
+  if (int rc = check_items("dequantize", a.items)) return rc;
+  if (n >= (int64_t(1) << 32) || dim >= (int64_t(1) << 32))
     return fail(NKV_ERR_UNSUPPORTED, "dequantize: rows=%lld n=%lld dim=%lld", (long long)rows, (long long)n, (long long)dim);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool few = few_rows(rows * n, out_dtype);
@@ -840,6 +849,7 @@ extern "C" int nkv_quantize_tok(const void* x, int x_dtype, int64_t x_row_stride
   }
   QuantSymArgs a{x, x_row_stride, rows, n, reinterpret_cast<uint8_t*>(codes), codes_row_stride, scales,
                  scale_row_stride, rows * cdiv(n, 16)};
+  if (int rc = check_items("quantize_tok", a.items)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)std::min<int64_t>(a.items, 1 << 22)), block(256);
   if (x_dtype == NKV_F16) hipLaunchKernelGGL((quant_sym_kernel<NKV_F16>), grid, block, 0, s, a);
@@ -864,6 +874,7 @@ extern "C" int nkv_paged_quantize_tok(const void* x, int x_dtype, int64_t x_head
     return fail(NKV_ERR_UNSUPPORTED, "paged_quantize_tok: x must be 16-byte aligned with a head stride >= n * 128");
   QuantSymArgs a{x, x_head_stride, hkv, n, nullptr, 0, nullptr, 0, hkv * cdiv(n, 16), pages, table_row, first_token,
                  num_pages, which};
+  if (int rc = check_items("paged_quantize_tok", a.items)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)std::min<int64_t>(a.items, 1 << 22)), block(256);
   if (x_dtype == NKV_F16) hipLaunchKernelGGL((quant_sym_kernel<NKV_F16, true>), grid, block, 0, s, a);
@@ -892,6 +903,7 @@ extern "C" int nkv_dequantize_tok(const int8_t* codes, int64_t codes_row_stride,
   const bool few = few_rows(rows * n, out_dtype);
   DequantSymArgs a{reinterpret_cast<const uint8_t*>(codes), codes_row_stride, scales, scale_row_stride, rows, n,
                    out, out_row_stride, rows * cdiv(n, few ? 16 : 64)};
+  if (int rc = check_items("dequantize_tok", a.items)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)std::min<int64_t>(a.items, 1 << 20));
   if (out_dtype == NKV_F16) launch_rows(dequant_sym_kernel<NKV_F16, 1>, dequant_sym_kernel<NKV_F16, 4>, few, grid, s, a);

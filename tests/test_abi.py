@@ -279,3 +279,23 @@ def test_prefill_cut_depends_on_the_shape_alone(lib):
         want = _cutting(lib, hq, hkv, m, used, hist)
         for nbytes in (best + 1, best + (1 << 20), 2 * best, best + (1 << 30)):
             assert _cutting(lib, hq, hkv, m, used, hist, nbytes=nbytes) == want, (hq, hkv, m, used, hist, nbytes)
+
+
+def test_tile_counts_that_would_wrap_are_refused(lib):
+    """The quantizers' workgroups take tiles in turns with 32-bit counts: a count near 2^32, whose next
+    turn would wrap to a tile below it (and the loop never end), is refused before any launch."""
+    from nova_amd import _lib
+
+    p = 1 << 20  # an aligned address that nothing reads
+    n = (1 << 32) - 5
+    calls = {
+        "quantize": lambda: lib.nkv_quantize_int8(p, 0, 8 * n, 1, n, 8, 1, 1, p, 8 * n, p, p, 8 * n, None),
+        "paged_quantize": lambda: lib.nkv_paged_quantize_t64(p, 0, 1 << 31, n, 1 << 6, 0, p, p, 0, 1, None),
+        "quantize_tok": lambda: lib.nkv_quantize_tok(p, 0, 8, n, 1, 128, p, 8, p, 8, None),
+        "paged_quantize_tok": lambda: lib.nkv_paged_quantize_tok(p, 0, 1 << 31, n, 1, 0, p, p, 0, 1, None),
+        "dequantize_tok": lambda: lib.nkv_dequantize_tok(p, 256, p, 8, n, 1, 128, p, 0, 256, None),
+        "dequantize": lambda: lib.nkv_dequantize_int8(p, 16, p, p, 8, n, 1, 8, 1, 1, p, 0, 16, None),
+    }
+    for name, call in calls.items():
+        assert call() == _lib.NKV_ERR_UNSUPPORTED, name
+        assert b"tiles" in lib.nkv_last_error(), (name, lib.nkv_last_error())
