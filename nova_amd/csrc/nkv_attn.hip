@@ -4758,8 +4758,9 @@ static void prefill_plan(PrefillArgs& a, int64_t splits, int64_t avail_slots, Pr
                                             merge_cost(a.tiles * per_tile)
                                       : none;
   const double best = std::min({c_tiles, c_parts, c_even});
+  p.zigzag = 1;
+  if (best == c_tiles) return;  // (cut already, in this order)
   p.zigzag = a.zigzag = best != c_parts;
-  if (best == c_tiles) return;  // (cut already)
   if (best == c_parts) {
     p.shares = (int)(a.tiles * per_tile);
     p.slots = p.shares;

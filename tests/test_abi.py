@@ -281,6 +281,14 @@ def test_prefill_cut_depends_on_the_shape_alone(lib):
             assert _cutting(lib, hq, hkv, m, used, hist, nbytes=nbytes) == want, (hq, hkv, m, used, hist, nbytes)
 
 
+@pytest.mark.parametrize("hq,hkv,m,used,splits", [(64, 8, 226, 384, 0), (64, 8, 253, 384, 4), (16, 2, 87, 0, 0)])
+def test_prefill_cut_at_tile_boundaries_keeps_its_order(lib, hq, hkv, m, used, splits):
+    """Cuts at tile boundaries are made for the zigzag order of the tiles, also where parts of every tile
+    cost the same (the first two)."""
+    kind, shares, slots, merges, zigzag, tiles = _cutting(lib, hq, hkv, m, used, splits=splits)
+    assert tiles >= 3 and (kind, slots, merges, zigzag) == (0, 0, 0, 1)
+
+
 def test_tile_counts_that_would_wrap_are_refused(lib):
     """The quantizers' workgroups take tiles in turns with 32-bit counts: a count near 2^32, whose next
     turn would wrap to a tile below it (and the loop never end), is refused before any launch."""
