@@ -606,8 +606,8 @@ int64_t nkv_prefill_preferred_bytes(int64_t hkv, int64_t hq, int64_t m, int64_t 
 int64_t nkv_prefill_default_splits(int64_t hkv, int64_t hq, int64_t m, int64_t used);
 /* How a call's work is cut over the workgroups (host only): out[0] 0 at tile boundaries, 1 every tile into
  * the same number of parts, 2 even shares; then the workgroups and partial slots per KV head, the tiles
- * that the second launch merges, whether tiles are taken from both ends in turn, the tiles, and the longest
- * share in steps of 64 tokens. */
+ * that the second launch merges, whether tiles are taken from both ends in turn, the tiles, the longest share
+ * in steps of 64 tokens, and the price by which the cutting was chosen, in thousandths of a step. */
 int nkv_prefill_cutting(int64_t hkv, int64_t hq, int64_t m, int64_t m_kv, int64_t used, int64_t splits,
                         int64_t workspace_bytes, int64_t* out);
 int nkv_prefill_attn_t64(const uint16_t* q, const uint16_t* k_chunk, const uint16_t* v_chunk, int64_t m,

@@ -4672,12 +4672,13 @@ extern "C" int64_t nkv_prefill_workspace_bytes(int64_t hkv, int64_t hq, int64_t 
 // sum: with a tile per share, only every second one is cut (2048 tokens: 32 tiles, the last with 31
 // more steps than the first). The combine launch costs about 2.5 steps, and the partials' writes and
 // reads 4.5 for 256 of them (35 MB). The last two take what slots the workspace has.
-constexpr double PF_TILE_COST = 1.0, PF_MERGE_COST = 2.5, PF_PARTIALS_COST = 4.5;
+constexpr double PF_TILE_COST = 1.0, PF_MERGE_COST = 2.5, PF_PARTIALS_COST = 4.5, PF_FEWER_PARTS = 0.85;
 constexpr int64_t PF_MIN_SHARE = 4;  // steps of an even share, at least
 constexpr int64_t PF_SNAP = 4;
 
 struct PrefillPlan {
   int shares = 0, slots = 0, two_slots = 0, merges = 0, zigzag = 0;
+  double price = 0.0;  // in steps
   PrefillCut cut[PF_MAX_SHARES + 1];
   PrefillMerge merge[PF_MAX_SHARES];
 };
@@ -4720,7 +4721,7 @@ static double prefill_cut(const PrefillArgs& a, int64_t T, int64_t W, int64_t sn
 
 // Cuts at tile boundaries into W shares: a tile each where there are as many (even shares moved to the
 // nearest boundary would give one share two short tiles and the next none: 87 tokens over nothing, 8 q
-// heads per KV head, 19.5 against 14.4 us), else about even ones. Returns the longest as prefill_cut does.
+// heads per KV head, 19.5 against 11.7 us), else about even ones. Returns the longest as prefill_cut does.
 static double prefill_cut_tiles(const PrefillArgs& a, int64_t T, int64_t W, PrefillPlan& p) {
   if (W < a.tiles) return prefill_cut(a, T, W, INT64_MAX, p);
   p.shares = a.tiles;
@@ -4754,11 +4755,11 @@ static void prefill_plan(PrefillArgs& a, int64_t splits, int64_t avail_slots, Pr
     T += n;
     longest = std::max(longest, n);
   }
-  // parts per tile (one round of workgroups; no part without a step: tile 0 is the shortest), and the even
-  // shares
+  // parts per tile, at most (one round of workgroups; no part without a step: tile 0 is the shortest), and
+  // the even shares
   const int64_t parts = splits > 0 ? splits : cap / a.tiles;
-  const int64_t per_tile = std::max<int64_t>(1, std::min({parts, (int64_t)(PF_MAX_SHARES / a.tiles),
-                                                          G + pf_fp16_groups(a, 0), avail_slots / a.tiles}));
+  const int64_t most = std::min({parts, (int64_t)(PF_MAX_SHARES / a.tiles), G + pf_fp16_groups(a, 0),
+                                 avail_slots / a.tiles});
   int64_t We = std::max<int64_t>(a.tiles, T / PF_MIN_SHARE);
   if (splits > 0) We = std::min<int64_t>(We, a.tiles * splits);
   We = std::min(We, std::min(cap, T));
@@ -4779,10 +4780,22 @@ static void prefill_plan(PrefillArgs& a, int64_t splits, int64_t avail_slots, Pr
     if (partials) c_even += merge_cost(partials);
   }
   const double c_tiles = prefill_cut_tiles(a, T, W, p);
-  const double c_parts = per_tile > 1 ? (double)(cdiv(longest, per_tile) * cdiv(a.tiles * per_tile, cap)) + PF_TILE_COST +
-                                            merge_cost(a.tiles * per_tile)
-                                      : none;
+  // as many parts as there are workgroups for, or the cheapest number where the prices put it 15% below:
+  // fewer partials, the longest share hardly longer (314 tokens over 256, 16 heads, 8 -> 3 parts: 23.5 ->
+  // 18.9 us; 116 over 1920, 2 KV heads, 31 -> 16: 27.2 -> 22.0). Closer ones the prices do not tell apart (68
+  // over 256, 32 q heads, 5 -> 3 parts, priced 8% cheaper: 13.9 -> 16.0 us).
+  double c_parts = none, c_most = none;
+  int64_t per_tile = 1;
+  for (int64_t k = most; k >= 2; --k) {
+    const double c = (double)(cdiv(longest, k) * cdiv(a.tiles * k, cap)) + PF_TILE_COST + merge_cost(a.tiles * k);
+    if (k == most) c_most = c;
+    if (k == most || (c < PF_FEWER_PARTS * c_most && c < c_parts)) {
+      c_parts = c;
+      per_tile = k;
+    }
+  }
   const double best = std::min({c_tiles, c_parts, c_even});
+  p.price = best;
   p.zigzag = 1;
   if (best == c_tiles) return;  // (cut already, in this order)
   p.zigzag = a.zigzag = best != c_parts;
@@ -4851,7 +4864,7 @@ extern "C" int nkv_prefill_cutting(int64_t hkv, int64_t hq, int64_t m, int64_t m
   PrefillPlan p;
   prefill_plan_in(a, splits, workspace_bytes, p);
   const int64_t v[] = {p.two_slots ? 2 : p.slots ? 1 : 0, p.shares, p.slots, p.merges, p.zigzag, a.tiles,
-                       prefill_longest(a, p)};
+                       prefill_longest(a, p), (int64_t)(1000.0 * p.price + 0.5)};
   std::copy(std::begin(v), std::end(v), out);
   return NKV_OK;
 }

@@ -260,10 +260,10 @@ def test_step_parts_stay_within_the_workspace_rules(lib):
 
 
 def _cutting(lib, hq, hkv, m, used, hist=0, splits=0, nbytes=None):
-    """(kind, shares, slots, merges, zigzag, tiles, longest share) of a prefill call."""
+    """(kind, shares, slots, merges, zigzag, tiles, longest share, price) of a prefill call."""
     if nbytes is None:
         nbytes = lib.nkv_prefill_preferred_bytes(hkv, hq, m, m + hist, used, splits)
-    out = (ctypes.c_int64 * 7)()
+    out = (ctypes.c_int64 * 8)()
     assert lib.nkv_prefill_cutting(hkv, hq, m, m + hist, used, splits, nbytes, out) == 0, lib.nkv_last_error()
     return tuple(out)
 
@@ -285,7 +285,7 @@ def test_prefill_cut_depends_on_the_shape_alone(lib):
 def test_prefill_cut_at_tile_boundaries_keeps_its_order(lib, hq, hkv, m, used, splits):
     """Cuts at tile boundaries are made for the zigzag order of the tiles, also where parts of every tile
     cost the same (the first two)."""
-    kind, shares, slots, merges, zigzag, tiles, longest = _cutting(lib, hq, hkv, m, used, splits=splits)
+    kind, shares, slots, merges, zigzag, tiles, longest, _ = _cutting(lib, hq, hkv, m, used, splits=splits)
     assert tiles >= 3 and (kind, slots, merges, zigzag) == (0, 0, 0, 1)
 
 
@@ -295,11 +295,22 @@ def test_prefill_share_per_tile_holds_one_tile(lib):
     for hq, hkv in ((16, 2), (8, 1), (64, 8), (32, 8), (12, 4)):
         for m in (40, 68, 87, 100, 130, 200):
             for used, hist in ((0, 0), (64, 0), (0, 70)):
-                kind, shares, _, _, _, tiles, longest = _cutting(lib, hq, hkv, m, used, hist)
+                kind, shares, _, _, _, tiles, longest, _ = _cutting(lib, hq, hkv, m, used, hist)
                 if kind == 0 and shares == tiles:
                     assert longest == used // 64 + -(-(m + hist) // 64), (hq, hkv, m, used, hist)
                     seen += tiles > 2
     assert seen > 5
+
+
+def test_prefill_cut_is_near_the_cheapest_of_all_numbers_of_parts(lib):
+    """No bound on the parts per tile gives a cut that is priced 15% cheaper than the one without: not only
+    the largest number of parts is looked at (314 tokens over 256, one q head per KV head, took two tiles
+    whole, as 8 parts of each cost the same)."""
+    for hq, hkv, m, used in ((16, 16, 314, 256), (32, 8, 87, 896), (28, 4, 68, 1920), (64, 8, 116, 448),
+                             (40, 8, 314, 256), (32, 8, 512, 16384), (8, 1, 33, 4096), (32, 8, 2048, 2048)):
+        price = _cutting(lib, hq, hkv, m, used)[7]
+        for parts in range(1, 33):
+            assert 0.85 * price <= _cutting(lib, hq, hkv, m, used, splits=parts)[7] + 1, (hq, hkv, m, used, parts)
 
 
 def test_tile_counts_that_would_wrap_are_refused(lib):
