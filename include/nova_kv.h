@@ -106,7 +106,8 @@ int nkv_dequantize_int8(const uint8_t* codes, int64_t codes_row_stride, const ui
  * workspace: >= nkv_attn_workspace_bytes(hkv, hq, n_parts) bytes of device memory,
  *   16-byte aligned (any contents).
  * n_parts: prefix work units per KV head (fixed for a captured graph); 0 picks one
- *   from `capacity` (or from `used` when no device scalar is given).
+ *   from `capacity` (or from `used` when no device scalar is given). A prefix too short for
+ *   them uses fewer (on the device, from its length): at most one more than its groups.
  * Calls that overlap on one GPU must not share `workspace`.
  */
 int nkv_attn_decode_t64(const uint16_t* q, const uint8_t* kq, const uint16_t* kmn,

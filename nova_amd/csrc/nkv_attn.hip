@@ -139,6 +139,7 @@ struct AttnArgs {
   int64_t tail_slots;
   int hq, hkv, gq;
   int n_parts;
+  int part_one, part_few, part_add, part_shift;  // how many of them a short prefix uses (parts_used)
   int tail_mode;
   float sl2;  // softmax scale * log2(e)
   uint16_t* out;
@@ -192,6 +193,17 @@ struct AttnArgs {
   uint16_t* h1_out;
   int fwd_agent;
 };
+
+// The prefix parts per KV head that a step over the prefix [0, U) of a contiguous cache uses, up to
+// n_parts. A cache's n_parts follows its capacity; while the context is shorter, parts without a group
+// would only be waited for and merged (32 parts over 4 groups, 8 KV heads: 10.7 us a step, 10.0 with 4;
+// 16 parts over 3 groups, 2 KV heads of 16 q heads: 23.7 us, 18.7 with one). So the parts are those of a
+// cache of about this length, by step_parts' rule (part_rule): part_few up to part_one groups W, else
+// (W + part_add) >> part_shift.
+__device__ __forceinline__ int parts_used(const AttnArgs& a, int64_t U) {
+  const int W = (int)((U + GT - 1) / GT);
+  return min(a.n_parts, W <= a.part_one ? a.part_few : (W + a.part_add) >> a.part_shift);
+}
 
 // XOR key of the 16-byte chunk positions of LDS row `row` (a token within its group).
 // K reads (16 consecutive rows, one chunk) and V transpose reads (rows 4g + {0..3} of
@@ -1653,7 +1665,7 @@ __device__ __forceinline__ void tail_body(const AttnArgs& a, int h, int b, SM& s
   const uint32_t ftag = tag_in >= 0 ? (uint32_t)tag_in : a.ftag;
   const bool poll = run != TAIL_KERNEL;  // partials written in this launch: poll their words
   const int gq = a.gq, pw = part_stride(gq), cols = gq * D;
-  const int P0 = PAGED ? min(a.seq_parts[2 * b + 1], WTS) : a.n_parts;  // prefix partials
+  const int P0 = PAGED ? min(a.seq_parts[2 * b + 1], WTS) : parts_used(a, U);  // prefix partials
   const bool fused = PAGED || a.tail_mode == TAIL_FUSED;
   // TB_RING_SLOT: another workgroup attends over the ring and publishes one ring partial in the
   // sequence's ring slot (the slot after its P0 prefix partials: ring_slot needs P0 equal to the
@@ -1667,7 +1679,7 @@ __device__ __forceinline__ void tail_body(const AttnArgs& a, int h, int b, SM& s
   const bool direct = (flags & TB_DIRECT) && (flags & TB_KEEP_BLOCK) && P0 + 1 <= 64 && nmw >= gq;
   const bool slot_in_combine = ring_slot && direct;
   const int P = P0 + (ring_slot && !direct ? 1 : 0);
-  float* hws = PAGED ? paged_block(a, h, b) : a.ws + (int64_t)h * P0 * pw;
+  float* hws = PAGED ? paged_block(a, h, b) : a.ws + (int64_t)h * a.n_parts * pw;
   auto pp = [&](int64_t u) -> float* { return hws + u * pw; };
 
   // ---- loads: the ring rows (or the new token) and q of the ring waves, the merging waves'
@@ -2400,7 +2412,7 @@ __global__ __launch_bounds__(THREADS, SMALL ? 4 : 1) void attn_prefix_kernel(Att
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = blockIdx.x % a.hkv;
   // work unit -> (sequence, part of its prefix, parts of that sequence, partial slot)
-  int b = 0, part = blockIdx.x / a.hkv, nparts = a.n_parts;
+  int b = 0, part = blockIdx.x / a.hkv, nparts;
   int pslot = part;
   if constexpr (PAGED) {
     const int m = a.wg_map[part];
@@ -2424,6 +2436,7 @@ __global__ __launch_bounds__(THREADS, SMALL ? 4 : 1) void attn_prefix_kernel(Att
     U = pos_ok ? (TOK ? pos : pos / GT * GT) : 0;
   } else {
     U = prefix_limit(a, pos, pos_ok);
+    nparts = parts_used(a, U);
   }
   // the fused step's append: int8t64 units in parts < APPEND_UNITS (the grid has at least
   // that many parts), the per-token symmetric token in part 0 (of each sequence when paged;
@@ -2431,9 +2444,10 @@ __global__ __launch_bounds__(THREADS, SMALL ? 4 : 1) void attn_prefix_kernel(Att
   const bool append = (PAGED ? TOK : a.tail_mode == TAIL_FUSED) && pos_ok && (TOK ? part == 0 : part < APPEND_UNITS);
   const bool prefix = part < nparts;
 
-  const int64_t W = (U + GT - 1) / GT;
-  const int64_t gs = prefix ? (int64_t)part * W / nparts : 0;
-  const int64_t ge = prefix ? (int64_t)(part + 1) * W / nparts : 0;
+  // (32-bit: at most 256 parts of 2^18 groups)
+  const uint32_t W = (uint32_t)((U + GT - 1) / GT);
+  const int64_t gs = prefix ? (uint32_t)part * W / (uint32_t)nparts : 0;
+  const int64_t ge = prefix ? (uint32_t)(part + 1) * W / (uint32_t)nparts : 0;
   // Groups gs + gi, gi < ng: wave w takes gi = w, w + WAVES, ... (a fixed assignment, so a
   // partial's summation order, and the result, are the same on every run). A group's
   // halves (32 tokens) go to slots 0 and 1 (int8t64: its rulers to the wave's ruler set,
@@ -3949,6 +3963,26 @@ static int64_t step_parts(int64_t hkv, int64_t groups) {
   return std::max(least, std::min({max_parts, groups, (int64_t)32}));
 }
 
+// The parts that a step uses of a cache that its context does not fill: one per group and one more (part 0,
+// which merges, then has none to stream); where a head's workgroups do not share an XCD, one per two groups
+// and four up to 8 (4 KV heads, 200 tokens in room for 2048: 14.0 us, 14.6 with one). More than 32 KV heads of the int8t64 format have 32 append workgroups each in the
+// launch, several rounds of the CUs, and gain nothing from a part per group (64 heads over 3 groups: 4
+// parts 21.2 us, one 18.4): one per eight.
+static void part_rule(AttnArgs& a) {
+  a.part_one = 0;
+  a.part_few = a.part_add = 1;
+  a.part_shift = 0;
+  if (a.hkv > 32 && !a.tok) {
+    a.part_one = a.part_add = 7;
+    a.part_shift = 3;
+  } else if (a.hkv % 8) {
+    a.part_one = 8;
+    a.part_few = 4;
+    a.part_add = 0;
+    a.part_shift = 1;
+  }
+}
+
 static int64_t part_floats(int64_t hq, int64_t hkv) { return part_stride((int)(hq / hkv)); }
 // Bytes of the fused tail's publication area: `n` ints (per head a counter and a flag per
 // partial; paged, a counter per sequence and head), rounded up to 256 bytes.
@@ -3971,6 +4005,7 @@ static int launch_attn(AttnArgs& a, int64_t n_parts, int64_t workspace_bytes, hi
                        int launches = LAUNCH_PREFIX | LAUNCH_TAIL, bool fusable = false) {
   if (n_parts < 0) return fail(NKV_ERR_INVALID, "%s: n_parts %lld is negative", what, (long long)n_parts);
   a.n_parts = (int)n_parts;
+  part_rule(a);
   // both launches in one call: the prefix kernel's part-0 workgroup of each head runs the tail
   // (at most MERGER_MAX_PARTS parts and MERGER_MAX_HEADS heads; beyond, the two launches)
   const bool fuse = fusable && n_parts > 0 && n_parts <= MERGER_MAX_PARTS && a.hkv <= MERGER_MAX_HEADS &&
@@ -4365,6 +4400,7 @@ extern "C" int nkv_decode_step_qkv_t64(const uint16_t* x, const uint16_t* x_gamm
   a.sl2 = LOG2E / sqrtf((float)head_dim);
   a.out = out; a.lse = lse_out; a.ws = static_cast<float*>(workspace);
   a.n_parts = (int)n_parts;
+  part_rule(a);
   a.inline_tail = 1;
   a.tail_ctr_end = reinterpret_cast<int*>(ws + (workspace_bytes & ~int64_t(3)));
   a.x = x; a.x_gamma = x_gamma; a.w_qkv = w_qkv; a.q_gamma = q_gamma; a.k_gamma = k_gamma; a.inv_freq = inv_freq;
@@ -5065,7 +5101,8 @@ int launch_layers(AttnArgs& a, bool tok, const void* layers_dev, int64_t n_layer
   if (workspace_bytes < need)
     return fail(NKV_ERR_INVALID, "%s: workspace of %lld bytes, need %lld", what, (long long)workspace_bytes, (long long)need);
   if (a.dep_all && a.hq > 64) return fail(NKV_ERR_UNSUPPORTED, "%s: the all-head dependency polls at most 64 query heads' flags", what);
-  a.n_parts = (int)n_parts;
+  a.n_parts = a.part_add = (int)n_parts;  // every part at any length: its streaming workgroups all publish
+  a.part_one = -1;
   a.n_layers = (int)n_layers;
   a.tail_ctr_end = reinterpret_cast<int*>(reinterpret_cast<char*>(a.ws) + (workspace_bytes & ~int64_t(3)));
   a.fwd_out = reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(a.ws) + part_bytes);

@@ -485,3 +485,40 @@ def test_nbytes_ratio():
     assert 0.4 < ratio < 0.6
     ref = ostream.StreamCache(2, H_KV, D, 2048, HQ)
     assert c.nbytes() == ref.nbytes()
+
+
+@pytest.mark.parametrize("tok", [False, True])
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (16, 2), (12, 4), (8, 1), (48, 48), (40, 40)])
+def test_steps_do_not_depend_on_spare_room(tok, hq, hkv):
+    """A cache with room for sixteen times the context gives the bits of one with a group or two to spare:
+    a step uses the parts that its length calls for, not those of the capacity. Steps across group
+    boundaries on one workspace (a part left unmerged would show), and at 9 and at 20 groups."""
+    from nova_amd.kvattn import KVInt8Cache
+    from nova_amd.kvtok import KVInt8TokCache
+
+    print(f"case tok={tok} hq={hq} hkv={hkv}", flush=True)
+    cls = KVInt8TokCache if tok else KVInt8Cache
+    for ctx, steps in ((62, 4), (190, 3), (600, 2), (1300, 2)):
+        small = (ctx + steps + 63) // 64 * 64 + 64
+        k, v = (randn((1, hkv, ctx + steps, D), 60 + i, 1.0).cuda() for i in range(2))
+        q = randn((1, hq, steps, D), 62, 1.0).cuda()
+        outs = []
+        # (where a head's workgroups do not share an XCD, a cache of up to 8 groups has one part for them all)
+        for room in ((16 * small, 64 * small) if hkv % 8 and small <= 512 else (small, 16 * small)):
+            c = cls(num_slots=1, num_kv_heads=hkv, head_dim=D, max_len=room, num_q_heads=hq)
+            c.begin_prefill(ctx)
+            c.set_prefill_pos(0)
+            c.update(k[:, :, :ctx], v[:, :, :ctx], 0)
+            c.finish_prefill(ctx)
+            got = []
+            for i in range(steps):
+                c.pos.fill_(ctx + i)
+                args = (k[:, :, ctx + i:ctx + i + 1], v[:, :, ctx + i:ctx + i + 1], q[:, :, i:i + 1].contiguous(), 0)
+                got.append(c.update_attend(*args).clone())
+                got.append(c.lse.clone())
+            outs.append(got)
+        for i, (x, y) in enumerate(zip(*outs)):
+            assert torch.equal(x, y), f"ctx {ctx} step {i // 2}"
+        if not tok:
+            want = _reference(k[:, :, :ctx + 1], v[:, :, :ctx + 1], q[:, :, :1], ctx + 1, (ctx + 1) // 64 * 64)
+            assert_ulp_or_abs(npy(outs[0][0])[0, :, 0], want, MAX_ULP, ABS_TOL, f"ctx={ctx}")
