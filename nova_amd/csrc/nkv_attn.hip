@@ -1640,8 +1640,9 @@ __device__ __forceinline__ void tail_load_rows(const AttnArgs& a, int h, int b, 
 // alone), and the tail returns without a final barrier; TB_RING_SLOT (paged, with pos_ok): no
 // ring attention here: the ring partial that paged_ring_tail publishes in the sequence's ring
 // slot takes the ring partials' place in the direct combine (without the direct path it is
-// merged as one more prefix partial).
-constexpr int TB_APPEND = 1, TB_KEEP_BLOCK = 2, TB_POISON = 4, TB_DIRECT = 8, TB_RING_SLOT = 16;
+// merged as one more prefix partial); TB_ALL_PARTS (the chained step's merger), every one of the n_parts
+// publishes, at any length.
+constexpr int TB_APPEND = 1, TB_KEEP_BLOCK = 2, TB_POISON = 4, TB_DIRECT = 8, TB_RING_SLOT = 16, TB_ALL_PARTS = 32;
 
 // The paged workspace: per KV head, per sequence b, its seq_parts[2b + 1] prefix partial slots
 // and one more, the ring slot (the paged int8t64 step's ring partial, published by the first of
@@ -1665,7 +1666,8 @@ __device__ __forceinline__ void tail_body(const AttnArgs& a, int h, int b, SM& s
   const uint32_t ftag = tag_in >= 0 ? (uint32_t)tag_in : a.ftag;
   const bool poll = run != TAIL_KERNEL;  // partials written in this launch: poll their words
   const int gq = a.gq, pw = part_stride(gq), cols = gq * D;
-  const int P0 = PAGED ? min(a.seq_parts[2 * b + 1], WTS) : parts_used(a, U);  // prefix partials
+  const int P0 = PAGED ? min(a.seq_parts[2 * b + 1], WTS)  // prefix partials
+                       : (flags & TB_ALL_PARTS) ? a.n_parts : parts_used(a, U);
   const bool fused = PAGED || a.tail_mode == TAIL_FUSED;
   // TB_RING_SLOT: another workgroup attends over the ring and publishes one ring partial in the
   // sequence's ring slot (the slot after its P0 prefix partials: ring_slot needs P0 equal to the
@@ -2944,7 +2946,7 @@ __device__ __forceinline__ bool merger_layer(const AttnArgs& args, const void* l
     la.kv_hs = 0;
   }
   tail_body<false>(la, h, 0, sm, TAIL_MERGER, pos, pos_ok, U, nullptr, fwd ? &qb : nullptr,
-                   TB_APPEND | TB_KEEP_BLOCK | TB_DIRECT | (lost || gave_up ? TB_POISON : 0));
+                   TB_APPEND | TB_KEEP_BLOCK | TB_DIRECT | TB_ALL_PARTS | (lost || gave_up ? TB_POISON : 0));
   // every wave's stores (out, lse, the ring slot) complete before the workgroup meets; then one
   // release at agent scope publishes them all with the count
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -5022,15 +5024,16 @@ int64_t layers_fwd_bytes(int64_t hq, int64_t n_layers) {
 }
 
 // Streaming parts per KV head, with hkv (parts + 1) workgroups resident at once.
-int64_t layers_parts(int64_t hkv, int64_t groups, int resident) {
+int64_t layers_parts(int64_t hkv, int64_t groups, int resident, bool tok) {
   const int64_t fit = resident / std::max<int64_t>(1, hkv) - 1;
-  // Four groups per workgroup up to 16 of them, beyond that eight (one per wave). A workgroup's share of a
-  // short prefix is a chain of latencies, and half as many groups in it gain more than the merge of
-  // twice the partials costs: 8 KV heads, per layer with eight / four groups: per-token format, 488
-  // tokens 9.19 / 7.49 us, 2000 9.22 / 7.76, 4000 9.34 / 8.01; int8t64 10.50 / 10.04, 10.73 / 10.34, 10.83 /
-  // 10.84. At 8000 tokens 16 workgroups and 31 take the same (9.81 and 9.92, 11.1 and 11.7).
-  const int64_t parts = std::max(cdiv(groups, 8), std::min<int64_t>(cdiv(groups, 4), 16));
-  return std::min<int64_t>(std::min<int64_t>(fit, WTS), std::max<int64_t>(1, parts));
+  // Eight groups per workgroup, one per wave. The per-token format takes four, up to 16 workgroups, where
+  // a head's workgroups share an XCD: two waves then halve a group's chain of latencies, which gains more
+  // than the merge of twice the partials costs (8 KV heads, per layer: 492 tokens in 512 9.4 -> 7.6 us, 2028
+  // in 2048 9.4 -> 7.9, 4076 in 4096 9.6 -> 8.2; 200 in 2048 7.66 -> 7.71, in 4096 7.8 -> 8.0). Not int8t64 (2028
+  // in 2048 10.84 -> 10.72, 200 in 4096 10.6 -> 10.9), nor hand-overs through memory (2 KV heads of 16 q
+  // heads, 1000 in 4096 18.7 -> 22.7).
+  const int64_t few = tok && hkv % 8 == 0 ? std::min<int64_t>(cdiv(groups, 4), 16) : 1;
+  return std::min<int64_t>(std::min<int64_t>(fit, WTS), std::max({(int64_t)1, cdiv(groups, 8), few}));
 }
 
 bool al8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
@@ -5087,7 +5090,7 @@ int launch_layers(AttnArgs& a, bool tok, const void* layers_dev, int64_t n_layer
   if (a.capacity > (int64_t(1) << 24)) return fail(NKV_ERR_UNSUPPORTED, "%s: capacity %lld exceeds 16M tokens", what, (long long)a.capacity);
   int resident = 0;
   if (int rc = layers_resident(tok, &resident)) return rc;
-  if (n_parts <= 0) n_parts = layers_parts(a.hkv, a.ngroups_cap, resident);
+  if (n_parts <= 0) n_parts = layers_parts(a.hkv, a.ngroups_cap, resident, tok);
   if (n_parts < 1 || n_parts > WTS)
     return fail(NKV_ERR_UNSUPPORTED, "%s: %lld streaming parts per KV head (1..%d)", what, (long long)n_parts, WTS);
   const int64_t grid = (int64_t)a.hkv * (n_parts + 1);
@@ -5101,8 +5104,7 @@ int launch_layers(AttnArgs& a, bool tok, const void* layers_dev, int64_t n_layer
   if (workspace_bytes < need)
     return fail(NKV_ERR_INVALID, "%s: workspace of %lld bytes, need %lld", what, (long long)workspace_bytes, (long long)need);
   if (a.dep_all && a.hq > 64) return fail(NKV_ERR_UNSUPPORTED, "%s: the all-head dependency polls at most 64 query heads' flags", what);
-  a.n_parts = a.part_add = (int)n_parts;  // every part at any length: its streaming workgroups all publish
-  a.part_one = -1;
+  a.n_parts = (int)n_parts;
   a.n_layers = (int)n_layers;
   a.tail_ctr_end = reinterpret_cast<int*>(reinterpret_cast<char*>(a.ws) + (workspace_bytes & ~int64_t(3)));
   a.fwd_out = reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(a.ws) + part_bytes);
@@ -5124,7 +5126,7 @@ extern "C" int64_t nkv_layers_default_parts(int64_t hkv, int64_t capacity, int t
   set_error("");
   int resident = 0;
   if (hkv <= 0 || capacity <= 0 || layers_resident(tok != 0, &resident) != NKV_OK) return 0;
-  const int64_t parts = layers_parts(hkv, cdiv(capacity, GT), resident);
+  const int64_t parts = layers_parts(hkv, cdiv(capacity, GT), resident, tok != 0);
   return parts >= 1 && hkv * (parts + 1) <= resident ? parts : 0;
 }
 

@@ -369,3 +369,17 @@ def test_chain_argument_checks():
     with pytest.raises(ValueError, match="all-head"):
         ChainedStep(cache, p_ks, p_vs, p_qs, p_outs, dep="head")
     ChainedStep(cache, p_ks, p_vs, p_qs, p_outs, dep="all")
+
+
+def test_default_parts_of_short_prefixes():
+    """Eight groups per streaming part; four, up to 16 parts, for the per-token format where the workgroups of
+    a KV head share an XCD alone (elsewhere more parts made a step with room to spare slower)."""
+    from nova_amd import _lib
+
+    lib = _lib.load()
+    for groups in (1, 4, 8, 9, 16, 31, 33, 47, 64, 65, 128, 129):
+        eight = -(-groups // 8)
+        for hkv in (1, 2, 4, 8):
+            assert lib.nkv_layers_default_parts(hkv, 64 * groups, 0) == eight, (hkv, groups)
+            want = max(eight, min(16, -(-groups // 4))) if hkv % 8 == 0 else eight
+            assert lib.nkv_layers_default_parts(hkv, 64 * groups, 1) == want, (hkv, groups)
