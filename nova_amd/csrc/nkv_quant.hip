@@ -110,8 +110,7 @@ __device__ __forceinline__ uint4 pack_h8(const float (&v)[8]) {
 // by lane swaps and across waves in LDS, where one thread per channel makes the ruler.
 // Bound by memory at size and by one pass's latency below: 8 heads x 32768 fp16 tokens (100 MB moved)
 // in 25 us (4.1 TB/s) against 42 us with one wave per group (128 values per lane, one chain of 2000
-// instructions), 2048 tokens in 5.0 us against 12 us. Groups of 2048 and
-// more: 30 us against 429 us (8 heads x 2048).
+// instructions), 2048 tokens in 5.5 us against 12.6 us. One group of 2048 tokens per head: 31 us against 360 us.
 
 struct QuantTokArgs {
   const void* x;
@@ -269,17 +268,34 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void quant_token_kernel(Quan
   }
 }
 
-// Waves per item: groups of at most 8 tokens take one wave (2 rows a lane), of at most 64 four (4 rows a
-// lane; the paged kernel's groups are always 64), longer ones a workgroup of 16 that reads them twice.
+template <int DT, int W, int R>
+static void launch_quant_token_as(const QuantTokArgs& a, hipStream_t s) {
+  const int64_t groups = W == 1 ? cdiv(a.items, 4) : a.items, most = 1 << 20;  // more are taken in turns
+  hipLaunchKernelGGL((quant_token_kernel<DT, W, R>), dim3((unsigned)std::min(groups, most)), dim3(W == 1 ? 256 : 64 * W), 0, s, a);
+}
+
+// Waves per item, by the tokens of a group that there are (a slab can be shorter than one), and the rows
+// that a lane keeps. A few waves per group hide the latency of one pass, but each of a group's waves costs
+// the ruler's meeting, so short groups take no more than their rows fill: 16384 fp16 groups of 128 channels
+// with one / two / four waves: 8 rows 19.7 / 32 / 44 us, 16 rows 27 / 35 / 45, 32 rows 42 / 39 / 49; few of
+// them take four (512 of 16 rows 4.7 / 5.1 / 4.4, one of 32 5.5 / 4.4 / 3.7). 33 to 64 rows: four waves of 4 rows a lane (64 rows 82 us; two of 8 rows the
+// same, and 5.7 against 4.5 us alone). Longer groups are read twice, by as many waves as leave each about
+// 16 rows: of many groups (fp16, 4096: 65 rows 28.6 / 34 / 65 us with 4 / 8 / 16 waves, 128 rows 52 / 48 / 77,
+// 512 groups of 512 rows 36 / 28 / 28), of few the more the rows (one group: 65 rows 5.7 / 4.9 / 5.2 us, 512
+// rows 22 / 13 / 10.7). fp32 rows count twice.
 template <int DT>
 static void launch_quant_token(const QuantTokArgs& a, hipStream_t s) {
-  const int64_t most = 1 << 20;  // workgroups; more items are taken in turns
-  if (a.gs <= 8)
-    hipLaunchKernelGGL((quant_token_kernel<DT, 1, 2>), dim3((unsigned)std::min(cdiv(a.items, 4), most)), dim3(256), 0, s, a);
-  else if (a.gs <= 64)
-    hipLaunchKernelGGL((quant_token_kernel<DT, 4, 4>), dim3((unsigned)std::min(a.items, most)), dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL((quant_token_kernel<DT, 16, 0>), dim3((unsigned)std::min(a.items, most)), dim3(1024), 0, s, a);
+  const int64_t gr = std::min(a.gs, a.n), bytes = gr * (DT == NKV_F32 ? 4 : 2);
+  if (gr <= 8) return launch_quant_token_as<DT, 1, 2>(a, s);
+  if (gr <= 32 && a.items <= 1024) return launch_quant_token_as<DT, 4, 2>(a, s);
+  if (gr <= 16) return launch_quant_token_as<DT, 1, 4>(a, s);
+  if (gr <= 32) return launch_quant_token_as<DT, 2, 4>(a, s);
+  if (gr <= 64) return launch_quant_token_as<DT, 4, 4>(a, s);
+  const bool many = a.items >= 512;
+  if constexpr (DT != NKV_F32)
+    if (many && bytes <= 192) return launch_quant_token_as<DT, 4, 0>(a, s);
+  if (many ? bytes <= 768 : gr <= 96) return launch_quant_token_as<DT, 8, 0>(a, s);
+  launch_quant_token_as<DT, 16, 0>(a, s);
 }
 
 // ---------------------------------------------------------------- a prefill chunk lands in the cache

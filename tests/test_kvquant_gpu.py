@@ -162,3 +162,52 @@ def test_every_quantizer_route_matches_oracle(axis, group, n, dim, dtype):
         assert np.array_equal(npy(q), rq)
         assert _eq16(mn, rm) and _eq16(st, rs)
     assert _eq16(dequantize_int8(q, mn, st, group, axis), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,n,group", [
+    (3, 9, 0), (3, 32, 64), (1024, 16, 0), (1025, 16, 0), (1025, 17, 32), (1025, 32, 0), (3, 33, 0), (700, 64, 0),
+    (5, 65, 0), (5, 96, 100), (5, 97, 0), (512, 65, 0), (512, 96, 0), (512, 97, 0), (512, 192, 0), (512, 384, 0),
+    (512, 385, 0),
+])
+def test_token_groups_over_the_splits_match_oracle(rows, n, group, dtype):
+    """The waves that a group gets follow its tokens and the number of groups: at the edges of each, the
+    oracle's codes and rulers."""
+    from nova_amd.kvquant import quantize_int8
+
+    print(f"case rows={rows} n={n} group={group} {dtype}", flush=True)
+    x = (torch.randn(rows, n, 8, generator=torch.Generator().manual_seed(n + rows)) * 2).to(dtype)
+    rq, rm, rs = okq.quantize_int8_token(x.float().numpy(), group)
+    q, mn, st = quantize_int8(x.cuda(), group, "token")
+    assert np.array_equal(npy(q), rq)
+    assert _eq16(mn, rm) and _eq16(st, rs)
+
+
+def _graph_us(fn, inner=10, reps=10):
+    """GPU time of a call: the least of several replays of a captured run of them."""
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(inner):
+            fn()
+    best = float("inf")
+    for _ in range(reps):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        graph.replay()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / inner)
+    return best
+
+
+def test_short_slabs_do_not_pay_for_long_groups():
+    """A group longer than its slab is the slab: the time is that of a group of its length (it took a
+    workgroup of sixteen waves for three tokens, 5.5 times as long)."""
+    from nova_amd.kvquant import quantize_int8
+
+    x = torch.randn(1000, 3, 512, dtype=torch.float16, device="cuda")
+    short, long = (_graph_us(lambda: quantize_int8(x, g, "token")) for g in (3, 128))
+    print(f"group 3 {short:.1f} us, group 128 {long:.1f} us", flush=True)
+    assert long < 2 * short
