@@ -87,7 +87,18 @@ __device__ __forceinline__ uint2 pack_codes8(const float (&x)[8], const float (&
   return pack_u8x8(c);
 }
 
-// The dequantizers give a thread one row up to 32768 rows (the latency of more would show: 1600 rows of
+// How the 256 threads of a workgroup lie over rows of at most 64 channels: as many lanes to a row as it has
+// 8-channel units, so that none idles (8 x 32768 rows of 8 channels, fp16: dequantized in 14.2 us with 15 of 16
+// lanes idle, 4.9 so). Rows of 72 to 120 channels take the 16 lanes of 128: theirs would start off the cache
+// lines (96 channels 15.2 against 18.0 us). mul: tid / lanes == tid * mul >> 16 (lanes <= 16, tid < 256).
+struct TileLanes {
+  uint32_t lanes, mul, rows;
+  explicit TileLanes(int64_t dim)
+      : lanes((uint32_t)std::min<int64_t>(16, dim / 8)), mul(65536u / lanes + 1), rows(256u / lanes) {}
+  TileLanes() = default;
+};
+
+// The dequantizers give a thread one row up to 32768 rows of 128 channels (the latency of more would show: 1600 rows of
 // fp16, token axis, 2.8 against 3.5 us), else four (262144 rows: 17.4 against 20.1 us).
 // fp32 outputs are bound by their stores and take one row at every size (262144 rows, tok: 26.1 against 27.3 us).
 static bool few_rows(int64_t rows, int out_dtype) { return rows <= 32768 || out_dtype == NKV_F32; }
@@ -374,6 +385,7 @@ struct QuantChanArgs {
   uint16_t* steps;
   int64_t s_rs;
   int64_t items;  // rows * n * ngc
+  TileLanes tl{};
 };
 
 template <int DT>
@@ -407,17 +419,31 @@ __global__ __launch_bounds__(256) void quant_channel_kernel(QuantChanArgs a) {
 }
 
 // The same for groups of 8, 16, 32, 64 or 128 channels and 16-byte rows: 16 tokens x 128 channels per
-// workgroup, 8 channels of one token per lane, a group's extremes over its gc / 8 lanes by lane swaps.
+// workgroup (more tokens of narrower rows), 8 channels of one token per lane, a group's extremes over its gc / 8 lanes by lane swaps.
 // 8 heads x 3001 bf16 tokens, groups of 32 / 64: 4.8 / 4.8 us against 22 / 33 us with a thread per group
 // (2-byte loads, one byte per store); 32768 fp16 tokens, groups of 64: 24 against 1390 us. Four tokens per
 // thread were slower at every size (2048 tokens: 5.4 against 4.0 us, 32768: 24.2 against 23.7 us).
-template <int DT, int L>  // L: lanes per group
+template <int DT, int L, bool NARROW>  // L: lanes per group; NARROW: fewer than 128 channels (TileLanes)
 __global__ __launch_bounds__(256) void quant_channel8_kernel(QuantChanArgs a) {
-  const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4;
-  const uint32_t nchunks = (uint32_t)((a.dim + 127) / 128), nblocks = (uint32_t)((a.n + 15) / 16);
-  const uint32_t chunk = blockIdx.x % nchunks, rest = blockIdx.x / nchunks, tb = rest % nblocks, r = rest / nblocks;
-  const int64_t ch = (int64_t)chunk * 128 + cl * 8, t = (int64_t)tb * 16 + rl;
-  if (ch >= a.dim || t >= a.n) return;  // (whole groups: dim is a multiple of gc)
+  const int rl = NARROW ? threadIdx.x * a.tl.mul >> 16 : threadIdx.x >> 4;
+  const int cl = threadIdx.x - rl * (NARROW ? a.tl.lanes : 16);
+  int64_t ch, t;
+  uint32_t r;
+  // (the lanes that leave are whole groups: dim is a multiple of gc, and a row's lanes are one of L)
+  if constexpr (NARROW) {
+    const uint32_t row = blockIdx.x * a.tl.rows + rl;
+    if (rl >= (int)a.tl.rows || row >= (uint32_t)(a.rows * a.n)) return;
+    r = row / (uint32_t)a.n;
+    t = row - r * (uint32_t)a.n;
+    ch = cl * 8;
+  } else {
+    const uint32_t nchunks = (uint32_t)((a.dim + 127) / 128), nblocks = (uint32_t)((a.n + 15) / 16);
+    const uint32_t chunk = blockIdx.x % nchunks, rest = blockIdx.x / nchunks, tb = rest % nblocks;
+    r = rest / nblocks;
+    ch = (int64_t)chunk * 128 + cl * 8;
+    t = (int64_t)tb * 16 + rl;
+    if (ch >= a.dim || t >= a.n) return;
+  }
   float v[8];
   Elem8<DT>::load(a.x, r * a.x_rs + t * a.dim + ch, v);
   float lo = __builtin_huge_valf(), hi = -__builtin_huge_valf();
@@ -437,17 +463,29 @@ __global__ __launch_bounds__(256) void quant_channel8_kernel(QuantChanArgs a) {
   }
 }
 
-template <int DT>
-static void launch_quant_channel(const QuantChanArgs& a, bool wide, hipStream_t s) {
-  const int64_t tiles = a.rows * cdiv(a.n, 16) * cdiv(a.dim, 128);
+template <int DT, bool NARROW>
+static void launch_quant_channel8(const QuantChanArgs& a, int64_t tiles, hipStream_t s) {
   const dim3 grid((unsigned)tiles), block(256);
-  if (tiles >= (1 << 24)) wide = false;  // (a grid of at most 2^32 threads)
-  if (wide && a.gc == 8) hipLaunchKernelGGL((quant_channel8_kernel<DT, 1>), grid, block, 0, s, a);
-  else if (wide && a.gc == 16) hipLaunchKernelGGL((quant_channel8_kernel<DT, 2>), grid, block, 0, s, a);
-  else if (wide && a.gc == 32) hipLaunchKernelGGL((quant_channel8_kernel<DT, 4>), grid, block, 0, s, a);
-  else if (wide && a.gc == 64) hipLaunchKernelGGL((quant_channel8_kernel<DT, 8>), grid, block, 0, s, a);
-  else if (wide && a.gc == 128) hipLaunchKernelGGL((quant_channel8_kernel<DT, 16>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL(quant_channel_kernel<DT>, dim3((unsigned)cdiv(a.items, 256)), block, 0, s, a);
+  if (a.gc == 8) hipLaunchKernelGGL((quant_channel8_kernel<DT, 1, NARROW>), grid, block, 0, s, a);
+  else if (a.gc == 16) hipLaunchKernelGGL((quant_channel8_kernel<DT, 2, NARROW>), grid, block, 0, s, a);
+  else if (a.gc == 32) hipLaunchKernelGGL((quant_channel8_kernel<DT, 4, NARROW>), grid, block, 0, s, a);
+  else if (a.gc == 64) hipLaunchKernelGGL((quant_channel8_kernel<DT, 8, NARROW>), grid, block, 0, s, a);
+  else if constexpr (!NARROW) hipLaunchKernelGGL((quant_channel8_kernel<DT, 16, NARROW>), grid, block, 0, s, a);
+}
+
+template <int DT>
+static void launch_quant_channel(QuantChanArgs a, bool wide, hipStream_t s) {
+  if (wide && (a.gc == 8 || a.gc == 16 || a.gc == 32 || a.gc == 64 || a.gc == 128)) {
+    const bool narrow = a.dim <= 64;
+    if (narrow) a.tl = TileLanes(a.dim);
+    const int64_t tiles = narrow ? cdiv(a.rows * a.n, (int64_t)a.tl.rows) : a.rows * cdiv(a.n, 16) * cdiv(a.dim, 128);
+    if (tiles < (1 << 24)) {  // (a grid of at most 2^32 threads)
+      if (narrow) launch_quant_channel8<DT, true>(a, tiles, s);
+      else launch_quant_channel8<DT, false>(a, tiles, s);
+      return;
+    }
+  }
+  hipLaunchKernelGGL(quant_channel_kernel<DT>, dim3((unsigned)cdiv(a.items, 256)), dim3(256), 0, s, a);
 }
 
 // ---------------------------------------------------------------- dequantize
@@ -463,6 +501,7 @@ struct DequantArgs {
   int64_t o_rs;
   int64_t items;  // tiles: rows * ceil(n / rows of a tile) * ceil(dim / 128)
   int vec;        // token axis: the rulers of 8 channels are 16-byte aligned
+  TileLanes tl;
 };
 
 template <int OT>
@@ -483,37 +522,62 @@ __device__ __forceinline__ void store8(void* out, int64_t off, const float (&v)[
   }
 }
 
-// 16 R tokens x 128 channels per workgroup, R rows of 8 channels per thread. A lane's rulers are loaded
+// 16 R tokens x 128 channels per workgroup (more tokens of narrower rows), R rows of 8 channels per thread. A lane's rulers are loaded
 // once per group it meets: token axis 8 steps and 8 mins (two 16-byte loads when `vec`), channel axis one
 // pair for its 8 channels when the group is a multiple of 8, else one per channel. 8 heads x 3001 /
 // 32768 fp16 tokens, groups of 64: token axis 4.6 / 17.4 us against 8.7 / 64 us, channel axis 4.6 / 20 us
 // against 7.9 / 49 us with a ruler load per value and 64-bit divisions.
-template <int OT, int R>
+template <int OT, int R, bool NARROW>
 __global__ __launch_bounds__(256) void dequant_kernel(DequantArgs a) {
-  const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4;
-  const uint32_t nchunks = (uint32_t)((a.dim + 127) / 128), nblocks = (uint32_t)((a.n + 16 * R - 1) / (16 * R));
+  const int rl = NARROW ? threadIdx.x * a.tl.mul >> 16 : threadIdx.x >> 4;
+  const int cl = threadIdx.x - rl * (NARROW ? a.tl.lanes : 16);
+  const uint32_t RR = NARROW ? a.tl.rows : 16;  // rows of a pass
   const bool token = a.axis == NKV_AXIS_TOKEN;
+  if (NARROW && rl >= (int)RR) return;
+  const uint32_t nchunks = (uint32_t)((a.dim + 127) / 128), nblocks = (uint32_t)((a.n + 16 * R - 1) / (16 * R));
+  const uint32_t all = (uint32_t)(a.rows * a.n);  // (NARROW: the slabs' rows as one sequence)
   for (uint32_t tile = blockIdx.x; tile < (uint32_t)a.items; tile += gridDim.x) {
-    const uint32_t chunk = tile % nchunks, rest = tile / nchunks, tb = rest % nblocks, r = rest / nblocks;
-    const int64_t ch = (int64_t)chunk * 128 + cl * 8;
+    uint32_t chunk = 0, r = 0;
+    int64_t t0;
+    if constexpr (NARROW) {
+      t0 = (int64_t)tile * RR * R + rl;
+    } else {
+      const uint32_t rest = tile / nchunks;
+      chunk = tile % nchunks;
+      r = rest / nblocks;
+      t0 = (int64_t)(rest % nblocks) * (16 * R) + rl;
+    }
+    const int64_t ch = (int64_t)chunk * 128 + cl * 8, last = (NARROW ? (int64_t)all : a.n) - 1;
     if (ch >= a.dim) continue;
-    const int64_t t0 = (int64_t)tb * (16 * R) + rl;
     uint2 cw[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-      cw[i] = *reinterpret_cast<const uint2*>(a.codes + r * a.c_rs + min(t0 + 16 * i, a.n - 1) * a.dim + ch);
-    float st[8], mn[8];
-    int64_t have = -1;
+    [[maybe_unused]] uint32_t slab[R], tok[R];  // NARROW: of each pass's row
 #pragma unroll
     for (int i = 0; i < R; ++i) {
-      const int64_t t = t0 + 16 * i;
-      if (t >= a.n) break;
+      if constexpr (NARROW) {
+        const uint32_t row = (uint32_t)min(t0 + RR * i, last);
+        slab[i] = row / (uint32_t)a.n;
+        tok[i] = row - slab[i] * (uint32_t)a.n;
+        cw[i] = *reinterpret_cast<const uint2*>(a.codes + slab[i] * a.c_rs + (int64_t)tok[i] * a.dim + ch);
+      } else {
+        cw[i] = *reinterpret_cast<const uint2*>(a.codes + r * a.c_rs + min(t0 + 16 * i, last) * a.dim + ch);
+      }
+    }
+    float st[8], mn[8];
+    int64_t have = -1;  // the group of st, mn (NARROW: the offset of its rulers)
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      if (t0 + RR * i > last) break;
+      int64_t t = t0 + RR * i;
+      if constexpr (NARROW) {
+        r = slab[i];
+        t = tok[i];
+      }
       if (token) {
         // (32-bit: the tile count bounds n)
         const int64_t gi = (uint32_t)t / (uint32_t)a.group;
-        if (gi != have) {
-          have = gi;
-          const int64_t so = r * a.s_rs + gi * a.dim + ch;
+        const int64_t so = r * a.s_rs + gi * a.dim + ch, key = NARROW ? so : gi;
+        if (key != have) {
+          have = key;
           if (a.vec) {
             Elem8<NKV_F16>::load(a.steps, so, st);
             Elem8<NKV_F16>::load(a.mins, so, mn);
@@ -684,6 +748,12 @@ static void launch_rows(K one, K four, bool few, dim3 grid, hipStream_t s, const
   hipLaunchKernelGGL(few ? one : four, grid, dim3(256), 0, s, a);
 }
 
+template <int OT>
+static void launch_dequant(const DequantArgs& a, bool narrow, bool few, dim3 grid, hipStream_t s) {
+  if (narrow) launch_rows(dequant_kernel<OT, 1, true>, dequant_kernel<OT, 4, true>, few, grid, s, a);
+  else launch_rows(dequant_kernel<OT, 1, false>, dequant_kernel<OT, 4, false>, few, grid, s, a);
+}
+
 // The kernels that take tiles in turns count them in 32 bits, one stride of the grid (at most 2^22 tiles)
 // past the last: below 2^31 that sum does not wrap, and every workgroup leaves its loop.
 static int check_items(const char* what, int64_t items) {
@@ -829,18 +899,20 @@ extern "C" int nkv_dequantize_int8(const uint8_t* codes, int64_t codes_row_strid
     n *= rows;
     rows = 1;
   }
+  const TileLanes tl(dim);
+  const bool narrow = dim <= 64, few = few_rows(rows * n * tl.lanes / 16, out_dtype);
+  const int64_t pass = (narrow ? tl.rows : 16) * (few ? 1 : 4);
   DequantArgs a{codes, codes_row_stride, mins, steps, scale_row_stride, rows, n, dim, g, axis,
-                out, out_row_stride, rows * cdiv(n, few_rows(rows * n, out_dtype) ? 16 : 64) * cdiv(dim, 128),
-                aligned16(mins) && aligned16(steps) && scale_row_stride % 8 == 0};
+                out, out_row_stride, narrow ? cdiv(rows * n, pass) : rows * cdiv(n, pass) * cdiv(dim, 128),
+                aligned16(mins) && aligned16(steps) && scale_row_stride % 8 == 0, tl};
   if (int rc = check_items("dequantize", a.items)) return rc;
-  if (n >= (int64_t(1) << 32) || dim >= (int64_t(1) << 32))
+  if (n >= (int64_t(1) << 32) || dim >= (int64_t(1) << 32) || (narrow && rows * n >= (int64_t(1) << 32)))
     return fail(NKV_ERR_UNSUPPORTED, "dequantize: rows=%lld n=%lld dim=%lld", (long long)rows, (long long)n, (long long)dim);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool few = few_rows(rows * n, out_dtype);
   const dim3 grid((unsigned)std::min<int64_t>(a.items, 1 << 20));
-  if (out_dtype == NKV_F16) launch_rows(dequant_kernel<NKV_F16, 1>, dequant_kernel<NKV_F16, 4>, few, grid, s, a);
-  else if (out_dtype == NKV_BF16) launch_rows(dequant_kernel<NKV_BF16, 1>, dequant_kernel<NKV_BF16, 4>, few, grid, s, a);
-  else launch_rows(dequant_kernel<NKV_F32, 1>, dequant_kernel<NKV_F32, 4>, few, grid, s, a);
+  if (out_dtype == NKV_F16) launch_dequant<NKV_F16>(a, narrow, few, grid, s);
+  else if (out_dtype == NKV_BF16) launch_dequant<NKV_BF16>(a, narrow, few, grid, s);
+  else launch_dequant<NKV_F32>(a, narrow, few, grid, s);
   return check_launch("dequantize_int8");
 }
 

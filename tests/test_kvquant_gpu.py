@@ -211,3 +211,45 @@ def test_short_slabs_do_not_pay_for_long_groups():
     short, long = (_graph_us(lambda: quantize_int8(x, g, "token")) for g in (3, 128))
     print(f"group 3 {short:.1f} us, group 128 {long:.1f} us", flush=True)
     assert long < 2 * short
+
+
+@pytest.mark.parametrize("axis,group,rows,n,dim", [
+    ("token", 8, 6, 17, 8), ("token", 9, 6, 30, 24), ("token", 64, 5, 70, 40), ("token", 0, 3, 3, 56), ("token", 8, 6, 17, 64),
+    ("token", 8, 6, 17, 72), ("token", 64, 3, 180001, 8), ("channel", 8, 5, 30, 24), ("channel", 8, 6, 17, 40),
+    ("channel", 16, 3, 70, 16), ("channel", 32, 5, 9, 32), ("channel", 64, 5, 33, 64), ("channel", 8, 3, 180001, 8),
+    ("channel", 4, 4, 33, 24), ("channel", 24, 3, 11, 72),
+])
+def test_narrow_rows_match_oracle(axis, group, rows, n, dim):
+    """Rows of at most 64 channels lie over a workgroup as one sequence over the slabs: slabs that do not end
+    on a group, few rows and many, and inputs inside longer slabs."""
+    from nova_amd.kvquant import dequantize_int8, quantize_int8
+
+    print(f"case {axis} group={group} rows={rows} n={n} dim={dim}", flush=True)
+    x = (torch.randn(rows, n, dim, generator=torch.Generator().manual_seed(n + dim)) * 2).half()
+    quantize, dequantize = ((okq.quantize_int8_token, okq.dequantize_int8_token) if axis == "token" else
+                            (okq.quantize_int8_channel, okq.dequantize_int8_channel))
+    rq, rm, rs = quantize(x.float().numpy(), group)
+    for src in (x.cuda(), torch.zeros(rows, n + 5, dim, dtype=x.dtype).cuda()[:, :n].copy_(x)):
+        q, mn, st = quantize_int8(src, group, axis)
+        assert np.array_equal(npy(q), rq)
+        assert _eq16(mn, rm) and _eq16(st, rs)
+    assert _eq16(dequantize_int8(q, mn, st, group, axis), dequantize(rq, rm, rs, group))
+
+
+@pytest.mark.parametrize("axis,group", [("token", 64), ("channel", 8)])
+def test_narrow_rows_keep_their_lanes_busy(axis, group):
+    """As many bytes in rows of 8 channels as in rows of 128 take about as long (three to four times, with
+    15 of 16 lanes idle)."""
+    from nova_amd.kvquant import dequantize_int8, quantize_int8
+
+    times = []
+    for n, dim in ((32768, 8), (2048, 128)):
+        x = torch.randn(8, n, dim, dtype=torch.float16, device="cuda")
+        q, mn, st = quantize_int8(x, group, axis)
+        times.append((_graph_us(lambda: dequantize_int8(q, mn, st, group, axis)),
+                      _graph_us(lambda: quantize_int8(x, group, axis))))
+    (d8, q8), (d128, q128) = times
+    print(f"dequantize {d8:.1f} / {d128:.1f} us, quantize {q8:.1f} / {q128:.1f} us", flush=True)
+    assert d8 < 2 * d128
+    if axis == "channel":
+        assert q8 < 2.5 * q128
