@@ -326,7 +326,7 @@ def test_tile_counts_that_would_wrap_are_refused(lib):
         "quantize_tok": lambda: lib.nkv_quantize_tok(p, 0, 8, n, 1, 128, p, 8, p, 8, None),
         "paged_quantize_tok": lambda: lib.nkv_paged_quantize_tok(p, 0, 1 << 31, n, 1, 0, p, p, 0, 1, None),
         "dequantize_tok": lambda: lib.nkv_dequantize_tok(p, 256, p, 8, n, 1, 128, p, 0, 256, None),
-        "dequantize": lambda: lib.nkv_dequantize_int8(p, 16, p, p, 8, n, 1, 8, 1, 1, p, 0, 16, None),
+        "dequantize": lambda: lib.nkv_dequantize_int8(p, 256, p, p, 128, n, 1, 128, 1, 1, p, 0, 256, None),
     }
     for name, call in calls.items():
         assert call() == _lib.NKV_ERR_UNSUPPORTED, name
