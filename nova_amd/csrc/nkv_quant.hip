@@ -595,11 +595,21 @@ __global__ __launch_bounds__(256) void dequant_kernel(DequantArgs a) {
 #pragma unroll
           for (int j = 0; j < 8; ++j) { st[j] = s1; mn[j] = m1; }
         } else {
+          // one division, then a ruler per group that the channels meet (with a division and two loads per
+          // channel, groups of 4: 8 x 32768 rows of 80 channels 37.9 us, 21.0 so)
+          uint32_t gc = (uint32_t)ch / (uint32_t)a.group, left = (gc + 1) * (uint32_t)a.group - (uint32_t)ch;
+          float s1 = h2f(a.steps[so + gc]), m1 = h2f(a.mins[so + gc]);
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            const uint32_t gc = (uint32_t)(ch + j) / (uint32_t)a.group;
-            st[j] = h2f(a.steps[so + gc]);
-            mn[j] = h2f(a.mins[so + gc]);
+            if (left == 0) {
+              ++gc;
+              left = (uint32_t)a.group;
+              s1 = h2f(a.steps[so + gc]);
+              m1 = h2f(a.mins[so + gc]);
+            }
+            --left;
+            st[j] = s1;
+            mn[j] = m1;
           }
         }
       }
