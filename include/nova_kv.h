@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define NKV_ABI_VERSION 11
+#define NKV_ABI_VERSION 12
 
 #define NKV_OK 0
 #define NKV_ERR_INVALID 1     /* argument outside what the reference accepts */

@@ -112,7 +112,7 @@ SIGNATURES = {
     "nkv_qk_norm_rope": (c_int, [P, I64, I64, I64, P, P, c_float, P, P, P]),
 }
 
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 _lib = None
 _lock = threading.Lock()
@@ -146,12 +146,13 @@ def load(require_gpu: bool = True):
             if not LIB_PATH.exists():
                 raise RuntimeError(f"{LIB_PATH} is missing: build it with `python -m nova_amd.build`")
             lib = ctypes.CDLL(str(LIB_PATH))
+            lib.nkv_abi_version.restype = c_int
+            if lib.nkv_abi_version() != ABI_VERSION:  # (before the names: an older library lacks some)
+                raise RuntimeError(f"libnova_kv ABI {lib.nkv_abi_version()} != {ABI_VERSION}: rebuild it")
             for name, (res, args) in SIGNATURES.items():
                 fn = getattr(lib, name)
                 fn.restype = res
                 fn.argtypes = args
-            if lib.nkv_abi_version() != ABI_VERSION:
-                raise RuntimeError(f"libnova_kv ABI {lib.nkv_abi_version()} != {ABI_VERSION}: rebuild it")
             _lib = lib
     if require_gpu:
         _probe_l2()

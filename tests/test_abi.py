@@ -331,3 +331,32 @@ def test_tile_counts_that_would_wrap_are_refused(lib):
     for name, call in calls.items():
         assert call() == _lib.NKV_ERR_UNSUPPORTED, name
         assert b"tiles" in lib.nkv_last_error(), (name, lib.nkv_last_error())
+
+
+def test_an_older_library_is_named_as_one(tmp_path, monkeypatch):
+    """A library of another ABI version is refused by its version, also when it lacks entry points."""
+    import shutil
+    import subprocess
+
+    from nova_amd import _lib
+
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if cc is None:
+        pytest.skip("no C compiler")
+    src, so = tmp_path / "old.c", tmp_path / "libold.so"
+    src.write_text(f"int nkv_abi_version(void) {{ return {_lib.ABI_VERSION - 1}; }}\n")
+    subprocess.run([cc, "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    monkeypatch.setattr(_lib, "LIB_PATH", so)
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(RuntimeError, match="rebuild"):
+        _lib.load(require_gpu=False)
+    assert _lib._lib is None
+
+
+def test_version_of_this_interface():
+    """The header and the bindings state one version, past 11: the library of that number had neither the
+    strided prefill and landing entry points nor units in any order."""
+    from nova_amd import _lib
+
+    version = int(re.search(r"#define NKV_ABI_VERSION (\d+)", HEADER.read_text()).group(1))
+    assert version == _lib.ABI_VERSION and version > 11
