@@ -163,33 +163,54 @@ def test_staged_prefill_in_three_chunks_against_oracle():
     cache.finish_prefill(total)
 
 
-@pytest.mark.parametrize("hq,hkv,used,m,hist,least", [
-    (4, 1, 192, 1999, 0, False),    # even shares in zigzag order: parts of one step up to whole tiles
-    (4, 1, 192, 1999, 0, True),     # the least workspace: tile boundaries alone
-    (16, 1, 0, 700, 130, False),    # 16 tokens per tile, an fp16 history that ends inside a group
-    (2, 2, 64, 1025, 0, False),     # 256 tokens per tile: waves of a tile end at different groups
-    (6, 2, 1088, 171, 0, False),    # 3 heads per KV head: tiles that start inside a token
-    (8, 8, 320, 64, 0, True),       # parts per tile, in the least workspace
+TILES, PARTS, EVEN = 0, 1, 2  # the cuttings of nkv_prefill_cutting
+
+
+@pytest.mark.parametrize("hq,hkv,used,m,hist,least,kind,whole", [
+    (4, 1, 192, 1999, 0, False, PARTS, 0),    # 32 tiles of 64 tokens in four parts each
+    (4, 1, 192, 1999, 0, True, PARTS, 0),     # the same in two, in the least workspace
+    (16, 1, 0, 700, 130, False, PARTS, 0),    # 16 tokens per tile, an fp16 history that ends inside a group
+    (2, 2, 64, 1025, 0, False, PARTS, 0),     # 256 tokens per tile: waves of a tile end at different groups
+    (6, 2, 1088, 171, 0, False, PARTS, 0),    # 3 heads per KV head: tiles that start inside a token
+    (8, 8, 320, 64, 0, True, PARTS, 0),       # one tile, in the least workspace
+    (16, 1, 0, 700, 0, False, TILES, 1),      # a tile per share
+    (64, 8, 384, 226, 0, False, TILES, 1),    # the same, in zigzag order where parts cost as much
+    (256, 64, 64, 400, 0, False, TILES, 2),   # two tiles per share: the stages are used again after a tile's store
+    (512, 32, 192, 150, 0, False, TILES, 2),
+    (32, 8, 0, 1024, 0, False, EVEN, 0),      # the end of one tile and the start of another in a share
+    (64, 16, 64, 1100, 0, False, EVEN, 2),    # and whole tiles between
+    (12, 4, 64, 1800, 100, False, EVEN, 0),   # over an fp16 history
+    (64, 16, 64, 1100, 30, True, TILES, 2),   # tile boundaries alone, in the least workspace
 ])
-def test_prefill_cuttings(hq, hkv, used, m, hist, least):
-    """Each way the work of a head is cut over the workgroups, against the oracle."""
+def test_prefill_cuttings(hq, hkv, used, m, hist, least, kind, whole):
+    """Each way the work of a head is cut over the workgroups, against the oracle; the case is cut the way
+    that it stands for (``whole``: the most tiles that a share holds, at least)."""
     from nova_amd import _lib
     from nova_amd.kvattn import int8_prefill_attend
 
     print(f"case hq={hq} hkv={hkv} used={used} m={m} hist={hist} least={least}", flush=True)
-    q, k16, v16, packed = _case(hq, hkv, used, m + hist, seed=95 + m)
-    q = q[:, :, hist:].contiguous()
     lib, scratch = _lib.load(), None
+    nbytes = int(lib.nkv_prefill_preferred_bytes(hkv, hq, m, m + hist, used, 0))
     if least:
         splits = int(lib.nkv_prefill_default_splits(hkv, hq, m, used))
-        scratch = torch.empty(int(lib.nkv_prefill_workspace_bytes(hkv, hq, m, splits)), dtype=torch.uint8, device="cuda")
+        nbytes = int(lib.nkv_prefill_workspace_bytes(hkv, hq, m, splits))
+        scratch = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    cut = np.zeros(8, np.int64)
+    assert lib.nkv_prefill_cutting(hkv, hq, m, m + hist, used, 0, nbytes, cut.ctypes.data) == 0
+    assert cut[0] == kind and -(-cut[5] // cut[1]) >= whole  # tiles over shares
+    assert kind == TILES or cut[3] > 0                     # cut tiles, merged by the second launch
+    q, k16, v16, packed = _case(hq, hkv, used, m + hist, seed=95 + m)
+    q = q[:, :, hist:].contiguous()
     got = int8_prefill_attend(q, k16, v16, *packed, used=used, scratch=scratch)
     # the oracle takes a chunk of all fp16 tokens; its last m queries are this call's
-    kq, kmn, kst, vq, vmn, vst = (npy(t)[0] for t in packed)
-    qa = torch.zeros(1, hq, m + hist, D, dtype=q.dtype)
-    qa[:, :, hist:] = q.cpu()
-    want = oattn.chunk_prefill_attend(npy(qa)[0], kq, kmn, kst, vq, vmn, vst, used, npy(k16)[0], npy(v16)[0])[:, hist:]
-    err = np.abs(npy(got)[0].astype(np.float64) - want)
+    heads = list(range(hkv)) if hkv <= 8 else [0, hkv // 2, hkv - 1]
+    rows = [h * (hq // hkv) + j for h in heads for j in range(hq // hkv)]
+    kq, kmn, kst, vq, vmn, vst = (npy(t)[0][heads] for t in packed)
+    qa = torch.zeros(1, len(rows), m + hist, D, dtype=q.dtype)
+    qa[:, :, hist:] = q[:, rows].cpu()
+    want = oattn.chunk_prefill_attend(npy(qa)[0], kq, kmn, kst, vq, vmn, vst, used, npy(k16)[0][heads],
+                                      npy(v16)[0][heads])[:, hist:]
+    err = np.abs(npy(got)[0][rows].astype(np.float64) - want)
     assert err.max() <= 2e-3, f"max abs {err.max():.2e}"
     assert err.mean() <= 1.5e-4, f"mean abs {err.mean():.2e}"
 
