@@ -123,7 +123,8 @@ struct AttnArgs {
   int tok;        // 1: per-token symmetric int8 codes and scales, 0: int8t64
   // paged batch (int8t64): pages [num_pages][hkv][PAGE_BYTES], page table [nseq][table_stride],
   // rings [nseq][hkv][K, V][64][D], pos_dev [nseq]; prefix work unit w serves sequence
-  // wg_map[w] >> 16, part wg_map[w] & 0xffff of seq_parts[2b + 1] starting at unit seq_parts[2b]
+  // wg_map[w] >> 16, part wg_map[w] & 0xffff of seq_parts[2b + 1]; seq_parts[2b] counts the parts
+  // of the sequences before it (the units may be in any order)
   uint8_t* pages;
   const int32_t* table;
   int64_t table_stride;
@@ -3343,7 +3344,8 @@ __global__ void ring_mask_kernel(const int64_t* written, const int64_t* qlen, co
 // step in 2.0 us. Against one workgroup per tile and split, with the fp16 groups loaded and scattered
 // between two barriers (3.9 us each) and a combine launch after every call (8 KV heads, 32 q heads):
 // 2048 tokens over 0 / 8192: 131 -> 60 us, 391 -> 326 us; 4096 over 0: 354 -> 149 us; 12001 over 0:
-// 2270 -> 1250 us; 8 over 16384: 46 -> 25 us; 512 over 16384 (no imbalance): 158 -> 156 us.
+// 2270 -> 1250 us; 8 over 16384: 46 -> 25 us; 512 over 16384, cut evenly before: the
+// same 157 us.
 constexpr int PF_WAVES = 8;
 constexpr int PF_THREADS = 64 * PF_WAVES;
 constexpr int PF_RB = 2;                             // MFMA row blocks per wave
@@ -3353,7 +3355,7 @@ constexpr int PF_KROW = D + 8;                       // fp16 K tile row stride (
 constexpr int PF_VROW = GT + 16;                     // fp16 V^T tile row stride (halves, 16-byte rows)
 constexpr float PF_TAU = 8.0f;                       // lazy softmax rescaling threshold (log2)
 constexpr int PF_PART = D + 4;                       // floats per row partial: acc[128], m, l, pad
-constexpr int PF_MAX_SHARES = 256;                   // shares of a head's steps (one workgroup per CU)
+constexpr int PF_MAX_SHARES = CUS;                   // shares of a head's steps (one workgroup per CU)
 constexpr int PF_STAGE = 2 * GT * D * 2;             // bytes of a stage: an fp16 group, or an int8 one with its rulers
 static_assert(PF_STAGE >= 2 * CODE_BYTES + RULER_BYTES, "an int8 group fits a stage");
 static_assert(2 * PF_STAGE >= PF_ROWS * D * 2, "a tile's fp16 output fits the stages");
@@ -3947,9 +3949,9 @@ static void l2_args(AttnArgs& a) {
 }
 
 // Prefix work units per KV head: at least 8 groups (one per wave) per workgroup, and at
-// most one workgroup per CU (256 CUs).
+// most one workgroup per CU.
 static int64_t default_parts(int64_t hkv, int64_t groups) {
-  const int64_t max_parts = std::max<int64_t>(1, 256 / std::max<int64_t>(1, hkv));
+  const int64_t max_parts = std::max<int64_t>(1, CUS / std::max<int64_t>(1, hkv));
   return std::min<int64_t>(max_parts, std::max<int64_t>(1, cdiv(groups, 8)));
 }
 
@@ -3960,7 +3962,7 @@ static int64_t default_parts(int64_t hkv, int64_t groups) {
 // (the hand-over goes through memory), half as many and at most 16: 2 KV heads, 1000 tokens 13.5 / 10.8 us
 // (15.5 / 15.0), 4095 tokens 17.0 / 15.5 (17.3 / 16.4); up to 8 groups they keep the one unit.
 static int64_t step_parts(int64_t hkv, int64_t groups) {
-  const int64_t max_parts = std::max<int64_t>(1, 256 / std::max<int64_t>(1, hkv)), least = default_parts(hkv, groups);
+  const int64_t max_parts = std::max<int64_t>(1, CUS / std::max<int64_t>(1, hkv)), least = default_parts(hkv, groups);
   if (hkv % 8) return groups <= 8 ? least : std::max(least, std::min({max_parts, groups / 2, (int64_t)16}));
   return std::max(least, std::min({max_parts, groups, (int64_t)32}));
 }
@@ -4592,17 +4594,17 @@ extern "C" int nkv_paged_append_t64(const uint16_t* k_new, const uint16_t* v_new
   return check_launch("paged_append_t64");
 }
 
-// The paged prefix launch with its fused tails. int8t64 (`tok` false): the step's token is
-// already in its sequence's ring (nkv_paged_append_t64 ran before), k_new / v_new are unused.
-// Per-token symmetric (`tok`): the launch appends k_new / v_new itself and attends them as the tail.
 // The paged per-token step's small workgroups (two per CU) when one per CU would not hold the launch at
 // once: 448 workgroups of 48 sequences (64 .. 2048 tokens) 38.1 -> 31.6 us a layer, 520 of 64 (to 3000)
 // 54 -> 44 us, 264 of 16 (to 4096) 26.8 -> 21.6 us, 328 of 40 (to 200) 24.1 -> 16.1 us. With 256 or fewer
 // the large ones, whose waves have a second half group in flight, win (8 sequences of 4000 .. 13000: 32.9
 // against 37.1 us). The int8t64 step gains nothing (43.8 against 43.9 us for the 448): its rulers and
 // append do not fit 128 registers.
-static bool small_paged(int64_t workgroups, int gq) { return workgroups > 256 && gq <= SMALL_GQ; }
+static bool small_paged(int64_t workgroups, int gq) { return workgroups > CUS && gq <= SMALL_GQ; }
 
+// The paged prefix launch with its fused tails. int8t64 (`tok` false): the step's token is
+// already in its sequence's ring (nkv_paged_append_t64 ran before), k_new / v_new are unused.
+// Per-token symmetric (`tok`): the launch appends k_new / v_new itself and attends them as the tail.
 static int paged_attn(const char* what, const uint16_t* q, const uint16_t* k_new, const uint16_t* v_new,
                       int64_t kv_seq_stride, int64_t kv_head_stride, const uint8_t* pages, const int32_t* page_table,
                       int64_t table_stride, int64_t num_pages, const uint16_t* rings, const int64_t* pos_dev,
@@ -4685,12 +4687,12 @@ extern "C" int nkv_paged_decode_step_tok(const uint16_t* q, const uint16_t* k_ne
 
 // ---------------------------------------------------------------- chunked prefill
 
-// Splits of the cache's groups: enough workgroups for every resident slot (256 CUs x
+// Splits of the cache's groups: enough workgroups for every resident slot (CUs x
 // PF_WG_PER_CU), at least one group per split.
 extern "C" int64_t nkv_prefill_default_splits(int64_t hkv, int64_t hq, int64_t m, int64_t used) {
   if (hkv <= 0 || hq <= 0 || m <= 0 || used < 0 || hq % hkv) return 0;
   const int64_t tiles = cdiv(m * (hq / hkv), PF_ROWS);
-  return std::max<int64_t>(1, std::min<int64_t>(cdiv(256 * PF_WG_PER_CU, hkv * tiles), std::max<int64_t>(1, used / GT)));
+  return std::max<int64_t>(1, std::min<int64_t>(cdiv(CUS * PF_WG_PER_CU, hkv * tiles), std::max<int64_t>(1, used / GT)));
 }
 
 extern "C" int64_t nkv_prefill_workspace_bytes(int64_t hkv, int64_t hq, int64_t m, int64_t splits) {

@@ -17,6 +17,10 @@ void set_error(const char* fmt, ...);
 int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);
 
+// Compute units of an MI355X. The plans that cut work to one workgroup per CU are made for these, without
+// asking the device, so that a host without one makes the same.
+constexpr int CUS = 256;
+
 // ---------------------------------------------------------------- vector types
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));

@@ -752,16 +752,29 @@ __global__ __launch_bounds__(256) void read_bw_kernel(const uint4* __restrict__ 
   if (threadIdx.x == 0) sink[blockIdx.x] = part[0] ^ part[1] ^ part[2] ^ part[3];
 }
 
-// One of a kernel's two row counts per thread.
-template <class K, class A>
-static void launch_rows(K one, K four, bool few, dim3 grid, hipStream_t s, const A& a) {
-  hipLaunchKernelGGL(few ? one : four, grid, dim3(256), 0, s, a);
+// One row per thread or four (fp32 outputs always take one: few_rows).
+template <int OT, bool NARROW>
+static void launch_dequant_as(const DequantArgs& a, bool few, dim3 grid, hipStream_t s) {
+  if constexpr (OT != NKV_F32)
+    if (!few) {
+      hipLaunchKernelGGL((dequant_kernel<OT, 4, NARROW>), grid, dim3(256), 0, s, a);
+      return;
+    }
+  hipLaunchKernelGGL((dequant_kernel<OT, 1, NARROW>), grid, dim3(256), 0, s, a);
 }
-
 template <int OT>
 static void launch_dequant(const DequantArgs& a, bool narrow, bool few, dim3 grid, hipStream_t s) {
-  if (narrow) launch_rows(dequant_kernel<OT, 1, true>, dequant_kernel<OT, 4, true>, few, grid, s, a);
-  else launch_rows(dequant_kernel<OT, 1, false>, dequant_kernel<OT, 4, false>, few, grid, s, a);
+  if (narrow) launch_dequant_as<OT, true>(a, few, grid, s);
+  else launch_dequant_as<OT, false>(a, few, grid, s);
+}
+template <int OT>
+static void launch_dequant_sym(const DequantSymArgs& a, bool few, dim3 grid, hipStream_t s) {
+  if constexpr (OT != NKV_F32)
+    if (!few) {
+      hipLaunchKernelGGL((dequant_sym_kernel<OT, 4>), grid, dim3(256), 0, s, a);
+      return;
+    }
+  hipLaunchKernelGGL((dequant_sym_kernel<OT, 1>), grid, dim3(256), 0, s, a);
 }
 
 // The kernels that take tiles in turns count them in 32 bits, one stride of the grid (at most 2^22 tiles)
@@ -1004,9 +1017,9 @@ extern "C" int nkv_dequantize_tok(const int8_t* codes, int64_t codes_row_stride,
   if (int rc = check_items("dequantize_tok", a.items)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)std::min<int64_t>(a.items, 1 << 20));
-  if (out_dtype == NKV_F16) launch_rows(dequant_sym_kernel<NKV_F16, 1>, dequant_sym_kernel<NKV_F16, 4>, few, grid, s, a);
-  else if (out_dtype == NKV_BF16) launch_rows(dequant_sym_kernel<NKV_BF16, 1>, dequant_sym_kernel<NKV_BF16, 4>, few, grid, s, a);
-  else launch_rows(dequant_sym_kernel<NKV_F32, 1>, dequant_sym_kernel<NKV_F32, 4>, few, grid, s, a);
+  if (out_dtype == NKV_F16) launch_dequant_sym<NKV_F16>(a, few, grid, s);
+  else if (out_dtype == NKV_BF16) launch_dequant_sym<NKV_BF16>(a, few, grid, s);
+  else launch_dequant_sym<NKV_F32>(a, few, grid, s);
   return check_launch("dequantize_tok");
 }
 

@@ -42,6 +42,7 @@ PAGE_BYTES = 2 * GT * D + 4 * D * 2
 PAGE_BYTES_TOK = 2 * GT * D + 2 * GT * 2
 CODE_BYTES = GT * D
 MAX_PARTS_PER_SEQ = 256  # partials the tail's merge holds for one sequence
+CUS = 256  # compute units of an MI355X: one workgroup each at a time
 
 
 class PagePool:
@@ -108,8 +109,9 @@ def plan_parts(lengths: list[int], target_parts: int) -> tuple[list[int], list[i
     """The prefix kernel's work plan: about ``target_parts`` units per KV head split over the
     sequences in proportion to their groups, each sequence at least one and at most
     ``MAX_PARTS_PER_SEQ``. Returns ``(wg_map, seq_parts)``: unit w serves sequence
-    ``wg_map[w] >> 16``, part ``wg_map[w] & 0xffff``; ``seq_parts[2b]`` is the first unit of
-    sequence b and ``seq_parts[2b + 1]`` its number of parts."""
+    ``wg_map[w] >> 16``, part ``wg_map[w] & 0xffff``; ``seq_parts[2b]`` counts the parts
+    of the sequences before b and ``seq_parts[2b + 1]`` those of b; the units themselves may be put in any
+    order."""
     if not lengths:
         raise ValueError("no sequences to plan")
     groups = [max(1, int(n) // GT) for n in lengths]
@@ -146,7 +148,7 @@ class PagedKVInt8Cache:
         self.pos = torch.zeros(self.max_seqs, dtype=torch.long, device=device)
         self.merged = torch.zeros((self.max_seqs, self.num_q_heads, 1, D), dtype=torch.float16, device=device)
         self.lse = torch.zeros((self.max_seqs, self.num_q_heads), dtype=torch.float32, device=device)
-        self.target_parts = int(target_parts or max(1, 256 // self.num_kv_heads))
+        self.target_parts = int(target_parts or max(1, CUS // self.num_kv_heads))
         self.wg_map = self.seq_parts = self.ws = None
         self.total_parts = 0
         self.nseq = 0
@@ -228,7 +230,7 @@ class PagedKVInt8Cache:
         grow (each unit covers a fixed fraction of its sequence's groups)."""
         lengths = list(self._len if lengths is None else lengths)
         wg_map, seq_parts = plan_parts(lengths, self.target_parts)
-        if len(wg_map) * self.num_kv_heads > 256:
+        if len(wg_map) * self.num_kv_heads > CUS:
             # more workgroups than CUs: the longest units (in groups per wave) start first, so that the ones
             # that start last, or share a CU, are short. 48 sequences of 64 .. 2048 tokens: 43.0 -> 37.5 us
             # a layer (per-token format 31.6 -> 26.9), 64 of 100 .. 3000: 66 -> 54 us (45 -> 43)
