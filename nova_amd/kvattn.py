@@ -821,9 +821,9 @@ class KVInt8Cache:
         return o
 
     def set_parts(self, n_parts: int) -> None:
-        """Prefix work units per KV head of the decode launches (before any capture); grows the
-        zero-filled workspace when needed, and zero-fills it (the fused projection step's tagged
-        words move with the partials' size)."""
+        """Prefix work units per KV head of the decode launches, at most: a short context uses fewer
+        (before any capture); grows the zero-filled workspace when needed, and zero-fills it (the
+        fused projection step's tagged words move with the partials' size)."""
         n_parts = int(n_parts)
         need = int(_lib.load().nkv_attn_workspace_bytes(self.num_kv_heads, self.num_q_heads, n_parts))
         if need > self._ws_bytes:

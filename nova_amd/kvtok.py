@@ -90,7 +90,9 @@ def int8_tok_attn_decode(q: torch.Tensor, kq: torch.Tensor, ksc: torch.Tensor, v
     ``q`` fp16 ``[1, Hq, 1, 128]``; ``kq``/``vq`` int8 ``[1, Hkv, L, 128]`` with ``L`` a
     multiple of 64; ``ksc``/``vsc`` fp16 ``[1, Hkv, L]``. ``used`` (host int) or
     ``used_t`` (device int64 ``[1]``, graph-safe) gives the length; ``out`` / ``lse_out``
-    / ``scratch`` may be preallocated for capture. Returns ``out`` ``[1, Hq, 1, 128]``.
+    / ``scratch`` may be preallocated for capture: without ``scratch`` captured calls share one
+    workspace per device, so their replays must not overlap (eager calls take one each). Returns
+    ``out`` ``[1, Hq, 1, 128]``.
     """
     _check(q, "q", torch.float16)
     for t, nm in ((kq, "kq"), (vq, "vq")):
